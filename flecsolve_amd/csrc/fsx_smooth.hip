@@ -198,6 +198,196 @@ __global__ __launch_bounds__(kRunThreads) void gs_run_kernel(
 	}
 }
 
+// Matrices whose x fits the shared memory of one CU: the whole relaxation
+// (every level of every sweep) in one workgroup, x resident in LDS.
+//
+// A sweep is a chain of levels; what bounds it is the latency from one
+// level's stores of x to the next one's gathers.  Through global memory that
+// is a trip through L2 (1.7 us per level in gs_run_kernel).  Here the chain
+// runs through LDS alone: the gathers, the row sums, the stores and a count
+// of finished steps.
+//
+// Levels are cut into steps of at most one wave's rows, dealt to the waves
+// in turn; a wave starts a step when every step of the levels before has
+// been counted, so the steps of one level run at once.  Everything else a
+// row reads does not depend on x: each wave loads its next step's rows while
+// the other waves work through theirs (row ids a turn earlier, since b is
+// read through them).  A row's entries sit in one record of `width` columns
+// (16 bits: a row index here is below 2^16) and values, so that a row takes
+// few wide loads from one address.
+//
+// The levels of one colour whose entries' mirrors are all stored order every
+// neighbour strictly before or after a row (checked at setup), so x in LDS
+// holds for each entry exactly the value the sequential sweep reads: no
+// snapshot, and the same sums in the same order, bit for bit.
+//
+// Measured (MI355X) on the seven Gauss-Seidel levels of a 48 x 44 x 40
+// aggregation hierarchy, 15671 rows and fewer, ~900 levels per direction:
+// the AMG-CG solve 371 ms -> 120 ms, of which a level costs ~0.5 us against
+// 1.7 us in gs_run_kernel.  Also measured: a barrier per step for the whole
+// workgroup 290 ms (each step then waits for its group's next loads to be
+// issued); 1024 threads, which leave no registers to gather a row's x at
+// once, 184 ms.
+constexpr int kLdsThreads = 512; // 2 waves per SIMD: a row's entries and x stay in registers
+constexpr int kLdsWaves = kLdsThreads / 64;
+constexpr int kLdsRow = 24;      // entries of a row kept in registers
+constexpr int kLdsMaxWidth = 64; // longest row of a matrix relaxed here
+
+// Rows [start, start + cnt) of the level order; `need`: steps of the sweep
+// that must have finished before; `groups`: eights of entries of its longest
+// row (1 .. kLdsRow / 8).
+struct gs_step {
+	int32_t start, cnt, need, groups;
+};
+
+struct gs_dir_view {
+	const gs_step * steps;
+	const int32_t * row;
+	const int32_t * len;
+	const double * diag;
+	// width per row, in the reference's order; padding: column n (x there
+	// is zero) and value zero, so that it adds +-0 to a sum that is never -0
+	const uint16_t * col;
+	const double * val;
+	int nsteps, width;    // width: a multiple of 8
+};
+
+struct gs_lds_row {
+	uint4 c[kLdsRow / 8];
+	double2 v[kLdsRow / 2];
+	double b, diag;
+	int r, len;
+};
+
+__device__ __forceinline__ int gs_col16(const uint4 & q, int k) {
+	const uint32_t w = k < 2 ? q.x : k < 4 ? q.y : k < 6 ? q.z : q.w;
+	return (int)((k & 1) ? w >> 16 : w & 0xffffu);
+}
+
+// The lane's row of the step: everything but the row id, which is known.
+__device__ __forceinline__ void gs_lds_load(gs_lds_row & m, const gs_dir_view & D, int p, int r,
+                                            int groups, const double * __restrict__ b) {
+	m.r = r;
+	m.len = D.len[p];
+	m.diag = D.diag[p];
+	m.b = b[r];
+	const uint4 * cp = (const uint4 *)(D.col + (int64_t)p * D.width);
+	const double2 * vp = (const double2 *)(D.val + (int64_t)p * D.width);
+#pragma unroll
+	for (int q = 0; q < kLdsRow / 8; ++q)
+		if (q < groups) {
+			m.c[q] = cp[q];
+#pragma unroll
+			for (int k = 0; k < 4; ++k) m.v[4 * q + k] = vp[4 * q + k];
+		}
+}
+
+// NG eights of entries: every gather issued before the first sum.
+template<int NG>
+__device__ __forceinline__ void gs_lds_finish(const gs_lds_row & m, const gs_dir_view & D, int p,
+                                              double dinv, double * xs) {
+	double xv[8 * NG];
+#pragma unroll
+	for (int k = 0; k < 8 * NG; ++k) xv[k] = xs[gs_col16(m.c[k / 8], k % 8)];
+	double rsum = 0.;
+#pragma unroll
+	for (int k = 0; k < 8 * NG; ++k) {
+		const double2 v2 = m.v[k / 2];
+		rsum += ((k & 1) ? v2.y : v2.x) * xv[k];
+	}
+	if constexpr (8 * NG == kLdsRow)
+		for (int j = kLdsRow; j < m.len; ++j)
+			rsum += D.val[(int64_t)p * D.width + j] * xs[D.col[(int64_t)p * D.width + j]];
+	xs[m.r] = dinv * (m.b - rsum);
+}
+
+// One sweep; `base`: the count of finished steps before it.
+__device__ __forceinline__ void gs_lds_sweep(const gs_dir_view & D, const double * __restrict__ b,
+                                             double * xs, unsigned * done, unsigned base) {
+	const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / 64));
+	const int lane = (int)(threadIdx.x % 64);
+	const int S = D.nsteps;
+	gs_step cur{}, nxt{};
+	gs_lds_row m;
+	int rn = 0;
+	auto row_of = [&](const gs_step & d) { return D.row[d.start + min(lane, d.cnt - 1)]; };
+	auto load = [&](int r) {
+		gs_lds_load(m, D, cur.start + min(lane, cur.cnt - 1), r,
+		            __builtin_amdgcn_readfirstlane(cur.groups), b);
+	};
+	if (wave < S) {
+		cur = D.steps[wave];
+		load(row_of(cur));
+		if (wave + kLdsWaves < S) {
+			nxt = D.steps[wave + kLdsWaves];
+			rn = row_of(nxt);
+		}
+	}
+	for (int s = wave; s < S; s += kLdsWaves) {
+		double dinv = 1. / m.diag;
+		asm volatile("" : "+v"(dinv)); // the division stays ahead of the wait
+		const unsigned need = base + (unsigned)__builtin_amdgcn_readfirstlane(cur.need);
+		const int groups = __builtin_amdgcn_readfirstlane(cur.groups);
+		for (;;) {
+			const int behind =
+				(int)(__hip_atomic_load(done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) - need);
+			if (behind >= 0) break;
+			if (behind < -2) __builtin_amdgcn_s_sleep(1);
+		}
+		__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+		if (lane < cur.cnt) {
+			const int p = cur.start + lane;
+			if (groups <= 1) gs_lds_finish<1>(m, D, p, dinv, xs);
+			else if (groups == 2) gs_lds_finish<2>(m, D, p, dinv, xs);
+			else gs_lds_finish<3>(m, D, p, dinv, xs);
+		}
+		__builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+		if (lane == 0)
+			__hip_atomic_fetch_add(done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+		cur = nxt;
+		if (s + kLdsWaves < S) {
+			load(rn);
+			if (s + 2 * kLdsWaves < S) {
+				nxt = D.steps[s + 2 * kLdsWaves];
+				rn = row_of(nxt);
+			}
+		}
+	}
+}
+
+// sweep: 0 forward, 1 backward, 2 symmetric, `nrelax` times
+__global__ __launch_bounds__(kLdsThreads) void gs_lds_kernel(int n, gs_dir_view fw,
+                                                             gs_dir_view bw, int sweep,
+                                                             int nrelax,
+                                                             const double * __restrict__ b,
+                                                             double * __restrict__ x) {
+	extern __shared__ double gs_xs[];
+	unsigned * done = (unsigned *)(gs_xs + n + 1);
+	for (int i = threadIdx.x; i < n; i += kLdsThreads) gs_xs[i] = x[i];
+	if (threadIdx.x == 0) {
+		gs_xs[n] = 0.; // read by padding
+		*done = 0u;
+	}
+	__syncthreads();
+	unsigned base = 0;
+	for (int it = 0; it < nrelax; ++it) {
+		if (sweep != 1) {
+			gs_lds_sweep(fw, b, gs_xs, done, base);
+			base += (unsigned)fw.nsteps;
+		}
+		if (sweep != 0) {
+			gs_lds_sweep(bw, b, gs_xs, done, base);
+			base += (unsigned)bw.nsteps;
+		}
+	}
+	__syncthreads();
+	for (int i = threadIdx.x; i < n; i += kLdsThreads) x[i] = gs_xs[i];
+}
+
+// Largest matrix gs_lds_kernel takes: x, a zero and the count in the 160 KB
+// of a CU.
+constexpr int64_t kGsLdsRows = 160 * 1024 / (int64_t)sizeof(double) - 2;
+
 // Refresh the copy's values from the matrix (entry index per slot, -1 for
 // padding / a missing diagonal).
 __global__ __launch_bounds__(256) void gs_gather_kernel(size_t n, const int64_t * __restrict__ from,
@@ -304,6 +494,7 @@ __global__ __launch_bounds__(kGridThreads) void gs_tile_kernel(
 	}
 	const int me = (li + 1) + H * ((lj + 1) + H * (lk + 1));
 	const int mine = li + lj + lk;
+	const double dinv = 1. / v[3]; // off the diagonals' critical path
 	__syncthreads();
 	for (int L = 0; L < 3 * T - 2; ++L) {
 		if (live && mine == (FWD ? L : 3 * T - 3 - L)) {
@@ -314,7 +505,6 @@ __global__ __launch_bounds__(kGridThreads) void gs_tile_kernel(
 			if (m & 16u) rsum += v[4] * xs[me + 1];
 			if (m & 32u) rsum += v[5] * xs[me + H];
 			if (m & 64u) rsum += v[6] * xs[me + H * H];
-			const double dinv = 1. / v[3];
 			xs[me] = dinv * (br - rsum);
 		}
 		__syncthreads();
@@ -339,7 +529,15 @@ struct fsx_gs {
 		std::vector<int32_t> width; // ELL depth of each level
 		std::unique_ptr<dbuf> srow, slen, sdiag, scol, sval, dfrom, vfrom, dlev, dbase, dwidth;
 		size_t nslots = 0;
+		// gs_lds_kernel's copy: steps, row ids, and per row a record of
+		// `rwidth` columns and values (rfrom: the entry each came from);
+		// rwidth 0: not built
+		std::unique_ptr<dbuf> steps, lrow, rcol, rval, rfrom;
+		size_t nrec = 0;
+		int nsteps = 0, rwidth = 0;
 	} fw, bw;
+	// the whole relaxation in one workgroup with x in LDS
+	bool lds = false;
 	// consecutive levels of at most this many rows (<= kRunThreads) run in
 	// one workgroup (gs_run_kernel); 0: a launch per level
 	int64_t run_rows = 0;
@@ -371,7 +569,7 @@ namespace {
 // sort: ascending row inside a level).
 void schedule(const std::vector<int64_t> & rp, const std::vector<int64_t> & ci,
               const colour_map & cm, bool colours, bool fwd, std::vector<int64_t> & ptr,
-              std::vector<int64_t> & order) {
+              std::vector<int64_t> & order, std::vector<int32_t> * levels = nullptr) {
 	const int64_t n = (int64_t)rp.size() - 1;
 	std::vector<int32_t> lev(n, 0);
 	int32_t maxl = -1;
@@ -393,6 +591,7 @@ void schedule(const std::vector<int64_t> & rp, const std::vector<int64_t> & ci,
 	std::vector<int64_t> fill(ptr.begin(), ptr.end() - 1);
 	order.resize(n);
 	for (int64_t r = 0; r < n; ++r) order[fill[lev[r]]++] = r;
+	if (levels) *levels = std::move(lev);
 }
 
 template<class T>
@@ -484,6 +683,54 @@ void build_tiles(fsx_ctx * ctx, fsx_gs & G) {
 	G.gmask = std::make_unique<dbuf>(std::max<int64_t>(1, n));
 }
 
+// gs_lds_kernel's copy of one sweep direction of a one-colour matrix, if it
+// takes the matrix: x fits LDS, no row is longer than kLdsMaxWidth, and no
+// entry couples rows of one level or a later row of a lower level (earlier
+// rows lie in lower levels by construction).
+template<class I>
+void build_lds_records(fsx_ctx * ctx, const std::vector<int64_t> & rp,
+                       const std::vector<int32_t> & lev, bool fwd,
+                       const std::vector<int64_t> & order, const std::vector<int32_t> & slen,
+                       const std::vector<I> & scol, const std::vector<int64_t> & vfrom,
+                       fsx_gs::dir & D) {
+	const int64_t n = (int64_t)order.size();
+	if (n == 0 || n > kGsLdsRows) return;
+	const int maxlen = *std::max_element(slen.begin(), slen.end());
+	if (maxlen > kLdsMaxWidth) return;
+	const int w = std::max(8, (maxlen + 7) / 8 * 8);
+	const size_t nl = D.lev.size() - 1;
+	std::vector<gs_step> steps;
+	std::vector<int32_t> lrow(n);
+	std::vector<uint16_t> rcol((size_t)n * w, (uint16_t)n);
+	std::vector<int64_t> rfrom((size_t)n * w, -1);
+	for (size_t l = 0; l < nl; ++l) {
+		const int64_t lo = D.lev[l], cnt = D.lev[l + 1] - lo;
+		const int32_t need = (int32_t)steps.size();
+		for (int64_t t0 = 0; t0 < cnt; t0 += 64)
+			steps.push_back({(int32_t)(lo + t0), (int32_t)std::min<int64_t>(64, cnt - t0), need,
+			                 std::max(1, std::min(kLdsRow / 8, (D.width[l] + 7) / 8))});
+		for (int64_t t = 0; t < cnt; ++t) {
+			const int64_t p = lo + t, r = order[p];
+			lrow[p] = (int32_t)r;
+			for (int j = 0; j < slen[p]; ++j) {
+				const int64_t q = D.base[l] + j * cnt + t;
+				const int64_t c = scol[q] >= 0 ? scol[q] : -scol[q] - 1;
+				if ((fwd ? c > r : c < r) && lev[c] <= lev[r]) return;
+				rcol[(size_t)p * w + j] = (uint16_t)c;
+				rfrom[(size_t)p * w + j] = vfrom[q];
+			}
+		}
+	}
+	D.nsteps = (int)steps.size();
+	D.rwidth = w;
+	D.nrec = rcol.size();
+	D.steps = upload(ctx, steps);
+	D.lrow = upload(ctx, lrow);
+	D.rcol = upload(ctx, rcol);
+	D.rfrom = upload(ctx, rfrom);
+	D.rval = std::make_unique<dbuf>(D.nrec * sizeof(double));
+}
+
 // The level-ordered copy of one sweep direction.  Entry order per row: the
 // own colour's off-diagonal entries in CSR order, then the other colours'
 // (gs.hh:94-107); the diagonal is the last entry whose column is the row.
@@ -491,7 +738,8 @@ template<class I>
 void build_dir(fsx_ctx * ctx, const std::vector<int64_t> & rp, const std::vector<int64_t> & ci,
                const colour_map & cm, bool colours, bool fwd, fsx_gs::dir & D) {
 	std::vector<int64_t> order;
-	schedule(rp, ci, cm, colours, fwd, D.lev, order);
+	std::vector<int32_t> lev;
+	schedule(rp, ci, cm, colours, fwd, D.lev, order, &lev);
 	const int64_t n = (int64_t)order.size();
 	const size_t nl = D.lev.size() - 1;
 	std::vector<I> srow(n);
@@ -552,6 +800,7 @@ void build_dir(fsx_ctx * ctx, const std::vector<int64_t> & rp, const std::vector
 		FSX_REQUIRE(width[l] <= std::numeric_limits<int32_t>::max(), "hybrid_gs: row too long");
 		D.width[l] = (int32_t)width[l];
 	}
+	if (!colours) build_lds_records<I>(ctx, rp, lev, fwd, order, slen, scol, vfrom, D);
 	D.dlev = upload(ctx, D.lev);
 	D.dbase = upload(ctx, D.base);
 	D.dwidth = upload(ctx, D.width);
@@ -590,6 +839,10 @@ void refresh_values(const fsx_gs & G) {
 			hipLaunchKernelGGL(gs_gather_kernel, dim3((unsigned)((D->nslots + 255) / 256)),
 			                   dim3(256), 0, s, D->nslots, (const int64_t *)D->vfrom->p, vals,
 			                   (double *)D->sval->p);
+		if (D->rwidth)
+			hipLaunchKernelGGL(gs_gather_kernel, dim3((unsigned)((D->nrec + 255) / 256)),
+			                   dim3(256), 0, s, D->nrec, (const int64_t *)D->rfrom->p, vals,
+			                   (double *)D->rval->p);
 	}
 	FSX_HIP(hipGetLastError());
 }
@@ -654,8 +907,23 @@ void enqueue_sweep(const fsx_gs & G, bool fwd, const double * b, double * x) {
 	FSX_HIP(hipGetLastError());
 }
 
+gs_dir_view dir_view(const fsx_gs::dir & D) {
+	return {(const gs_step *)D.steps->p, (const int32_t *)D.lrow->p,
+	        (const int32_t *)D.slen->p,  (const double *)D.sdiag->p,
+	        (const uint16_t *)D.rcol->p, (const double *)D.rval->p,
+	        D.nsteps,                    D.rwidth};
+}
+
 // sweep kinds: 0 forward, 1 backward, 2 symmetric (mg::relax_sweep)
 void enqueue_relax(const fsx_gs & G, int sweep, int nrelax, const double * b, double * x) {
+	if (G.lds) {
+		const int n = (int)G.A->nrows;
+		hipLaunchKernelGGL(gs_lds_kernel, dim3(1), dim3(kLdsThreads),
+		                   (size_t)(n + 2) * sizeof(double), G.ctx->stream, n, dir_view(G.fw),
+		                   dir_view(G.bw), sweep, nrelax, b, x);
+		FSX_HIP(hipGetLastError());
+		return;
+	}
 	for (int it = 0; it < nrelax; ++it) {
 		auto run = [&](bool fwd) {
 			if (G.A->it == FSX_I32) enqueue_sweep<int32_t>(G, fwd, b, x);
@@ -734,6 +1002,12 @@ int fsx_gs_create(fsx_ctx * ctx, const fsx_csr * A, int ncolours, fsx_gs ** out)
 			else build_dir<int64_t>(ctx, rp, ci, G->cm, ncolours > 1, fwd, D);
 		}
 		if (G->tiles) build_tiles(ctx, *G);
+		// an explicit FSX_GS_RUN_ROWS asks for the launches it shapes
+		G->lds = !re && G->fw.rwidth && G->bw.rwidth;
+		if (G->lds)
+			FSX_HIP(hipFuncSetAttribute((const void *)&gs_lds_kernel,
+			                            hipFuncAttributeMaxDynamicSharedMemorySize,
+			                            (int)((kGsLdsRows + 2) * sizeof(double))));
 		G->xold = std::make_unique<dbuf>(std::max<int64_t>(1, n) * sizeof(double));
 		refresh_values(*G);
 		G->version = A->vals_version;

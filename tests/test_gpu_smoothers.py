@@ -13,6 +13,7 @@ on n^2, 3n - 2 for the 7-point stencil on n^3, 1 for a diagonal matrix).
 """
 import numpy as np
 import pytest
+import scipy.sparse as sp
 
 from flecsolve_amd import fsx
 from flecsolve_amd import problems as P
@@ -200,3 +201,40 @@ def test_errors(ctx):
                    np.array([1.0, 1.0]), ncols=4)
     with pytest.raises(fsx.FsxError):
         fsx.HybridGS(rect)
+
+
+def mirrored_csr(n, per_row, seed, long_rows=0, long_len=60):
+    """Random matrix with a symmetric structure (values not), a full diagonal,
+    columns ascending; `long_rows` rows couple to `long_len` others."""
+    rng = np.random.default_rng(seed)
+    i = rng.integers(0, n, n * per_row // 2)
+    j = np.clip(i + rng.integers(-40, 41, i.size), 0, n - 1)
+    for r in rng.choice(n, long_rows, replace=False):
+        i = np.append(i, np.full(long_len // 2, r))
+        j = np.append(j, rng.choice(n, long_len // 2, replace=False))
+    S = sp.csr_matrix((np.ones(2 * i.size + n),
+                       (np.r_[i, j, np.arange(n)], np.r_[j, i, np.arange(n)])), (n, n))
+    S.sum_duplicates()
+    S.sort_indices()
+    v = rng.uniform(-1.0, 1.0, S.nnz)
+    rows = np.repeat(np.arange(n), np.diff(S.indptr))
+    v[S.indices == rows] = 8.0 + rng.random(n)
+    return S.indptr, S.indices, v
+
+
+@pytest.mark.parametrize("itype", [np.int32, np.int64])
+@pytest.mark.parametrize("n,per_row,long_rows", [
+    (1, 2, 0), (63, 4, 0), (65, 6, 2), (3000, 9, 5), (4000, 20, 9),
+    (20478, 6, 3),   # the largest whose x fits one CU's shared memory
+    (20479, 6, 3),   # the first one past it
+])
+def test_relaxation_in_shared_memory_bit_exact(ctx, itype, n, per_row, long_rows):
+    """Small one-colour matrices run every level of every sweep in one
+    workgroup (levels of more and fewer than 64 rows, rows of more than 8, 16
+    and 24 entries); larger ones, and those whose structure is not symmetric,
+    keep a launch or a run per level: the oracle's bits on both sides."""
+    rp, ci, v = mirrored_csr(n, per_row, 100 + n, min(long_rows, n), min(60, n))
+    for sweep, nrelax in ((0, 1), (1, 1), (2, 3)):
+        got, ref, _ = run_both(ctx, rp.astype(itype), ci.astype(itype), v, sweep, nrelax, 1,
+                               seed=9 + sweep)
+        np.testing.assert_array_equal(got, ref)
