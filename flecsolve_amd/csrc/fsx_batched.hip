@@ -1,4 +1,6 @@
-// fsx_batched.hip -- many independent CG solves in one persistent launch.
+// fsx_batched.hip -- many independent CG solves: one workgroup per system in
+// one persistent launch, or all systems in lockstep (below; use_lockstep says
+// which).
 //
 // Input: the block-diagonal concatenation of the systems (one fsx_csr, global
 // column ids) and the row offsets of each system.  One launch, sized to the
@@ -48,6 +50,14 @@ struct fsx_batch {
 	int lanes = 1;
 	bool tuned = false;
 	double tuned_ms = 0;
+	// a configuration set by the caller names the kernel of one workgroup per
+	// system
+	bool fixed = false;
+	// lockstep solves: the blocks of rows (built by the first one), the
+	// systems' states, the partials, the count of running systems
+	std::unique_ptr<fsx::dbuf> ls_blocks, ls_st, ls_part, ls_active;
+	int64_t nblocks = 0, max_rows = 0, min_rows = 0;
+	int rpt = 0;
 };
 
 namespace fsx {
@@ -646,6 +656,388 @@ __global__ __launch_bounds__(kBatchMaxThreads) void batched_cg_kernel(batch_args
 	}
 }
 
+// ---- lockstep solves: every system advanced by the same launches ------------
+//
+// One workgroup per system leaves most of the GPU idle when the batch holds
+// fewer large systems than workgroups, and its time is the largest system's
+// on one CU.  Here each system is cut into blocks of rows, and three launches
+// over the blocks of all systems advance every system by one iteration:
+//   A  w = A p, partials of w.p per block
+//   B  alpha; r -= alpha w (z = D^-1 r), partials of r.r (r.z)
+//   C  beta, the tolerance test, x += alpha p, p = beta p + z
+// What bounds it is HBM (or MALL) bandwidth over the rows of the systems
+// still running; a block whose system is done returns at entry.  Every block
+// sums its own system's partials itself, in the same order, so the scalars
+// need no launch of their own and depend on nothing but the system.
+//
+// A system is in one phase at a time, and its blocks branch on it:
+//   init     B: r = b - A x, partials of r.r and b.b; C: the first test, then
+//            the first search direction, partials of its rho
+//   start    as iterate, with rho summed from C's partials
+//   iterate  above
+//   segment  (residual replacement) A: x += c S y; B: r = b - A x in FP64,
+//            partials of r.r; C: the test on the true residual, the
+//            replacement, partials of its rho
+//   done
+// Launch k reads the phase and the scalars from slot k & 1 of the system's
+// state; C's first block of the system writes the other slot, so no launch
+// reads what it writes.  The expressions are wg_cg's and wg_cg_segment's.
+//
+// Measured against the kernel of one workgroup per system: use_lockstep.
+constexpr int kLsThreads = 256;
+
+enum ls_phase { LS_INIT = 0, LS_START, LS_ITER, LS_SEG, LS_DONE };
+
+struct ls_state {
+	double rho[2], tol[2];
+	int phase[2], it[2], seg[2];
+	// written by B, read by C
+	double alpha, rho_b, tol_b;
+	int brk, pad;
+	// written by C, read by later launches
+	double c, inv, bnorm, res;
+	int inner;
+};
+
+struct ls_block {
+	int sys;      // system
+	int first;    // the system's first block
+	int count;    // its blocks
+	int pad;
+	int64_t base; // rows base + t (t = 0 .. rows per block - 1) inside [lo, hi)
+	int64_t lo, hi;
+};
+
+struct ls_args {
+	batch_args a;
+	const ls_block * blocks;
+	ls_state * st;
+	double * pa; // A's partials: 1 per block
+	double * pb; // B's: 2 per block
+	double * pc; // C's: 1 per block
+	int * active;
+	int par; // state slot of this launch
+};
+
+template<class V>
+__device__ __forceinline__ double ls_row(const batch_args & a, const V * __restrict__ dg_v,
+                                         int64_t r, const V * __restrict__ x) {
+	const int64_t s = __builtin_amdgcn_readfirstlane((int)(r / kSliceRows));
+	const int lane = (int)(r & (kSliceRows - 1));
+	const int64_t base = a.dg_ptr[s];
+	const int wd = (int)((a.dg_ptr[s + 1] - base) / kSliceRows);
+	const int64_t q0 = base / kSliceRows;
+	double sum = 0.0;
+	for (int j0 = 0; j0 < wd; j0 += kSliceUnroll) {
+		bool pr[kSliceUnroll];
+		V v[kSliceUnroll], xv[kSliceUnroll];
+		int32_t off[kSliceUnroll];
+#pragma unroll
+		for (int k = 0; k < kSliceUnroll; ++k) {
+			const int jj = min(j0 + k, wd - 1);
+			off[k] = a.dg_off[q0 + j0 + k];
+			const uint64_t m = a.dg_mask[q0 + j0 + k];
+			pr[k] = (j0 + k < wd) & (((m >> lane) & 1) != 0);
+			v[k] = ldnt(dg_v + base + (int64_t)jj * kSliceRows + lane);
+		}
+#pragma unroll
+		for (int k = 0; k < kSliceUnroll; ++k) xv[k] = x[pr[k] ? r + off[k] : r];
+#pragma unroll
+		for (int k = 0; k < kSliceUnroll; ++k) {
+			const double t = sum + (double)v[k] * (double)xv[k];
+			sum = pr[k] ? t : sum;
+		}
+	}
+	return sum;
+}
+
+// The rows of a block: RPT per thread, each wave on one slice at a time.
+// f(row, j) runs for the rows of the system only.
+template<int RPT, class F>
+__device__ __forceinline__ void ls_rows(const ls_block & k, F && f) {
+#pragma unroll
+	for (int j = 0; j < RPT; ++j) {
+		const int64_t r = k.base + j * kLsThreads + threadIdx.x;
+		if (r >= k.lo && r < k.hi) f(r, j);
+	}
+}
+
+// The thread's elements of a vector, issued ahead of the partials' sums (B
+// and C wait for those, and would otherwise load their rows only then).
+template<int RPT, class T>
+__device__ __forceinline__ void ls_ahead(const ls_block & k, const T * __restrict__ v,
+                                         T (&out)[RPT]) {
+#pragma unroll
+	for (int j = 0; j < RPT; ++j) {
+		const int64_t r = k.base + j * kLsThreads + threadIdx.x;
+		out[j] = v[min(max(r, k.lo), k.hi - 1)];
+	}
+}
+
+template<bool RR, int RPT>
+__global__ __launch_bounds__(kLsThreads) void ls_a_kernel(ls_args g) {
+	const ls_block k = g.blocks[blockIdx.x];
+	const ls_state & st = g.st[k.sys];
+	const int phase = st.phase[g.par];
+	if (phase == LS_DONE || phase == LS_INIT) return;
+	const batch_args & a = g.a;
+	if (RR && phase == LS_SEG) {
+		const double c = st.c;
+		ls_rows<RPT>(k, [&](int64_t r, int) { a.x[r] = a.x[r] + c * (a.sym[r] * (double)a.fd[r]); });
+		return;
+	}
+	double d[1] = {0.0};
+	ls_rows<RPT>(k, [&](int64_t r, int j) {
+		if constexpr (RR) {
+			const double pv = (double)a.fp[r];
+			const float wi = (float)ls_row<float>(a, a.dg_v32, r, a.fp);
+			a.fw[r] = wi;
+			d[0] += (double)wi * pv;
+		}
+		else {
+			const double pv = a.p[r];
+			const double wi = ls_row<double>(a, a.dg_v64, r, a.p);
+			a.w[r] = wi;
+			d[0] += wi * pv;
+		}
+	});
+	store_block_partials<1>(d, g.pa, blockIdx.x);
+}
+
+template<bool RR, bool JAC, int RPT>
+__global__ __launch_bounds__(kLsThreads) void ls_b_kernel(ls_args g) {
+	const ls_block k = g.blocks[blockIdx.x];
+	ls_state & st = g.st[k.sys];
+	const int phase = st.phase[g.par];
+	if (phase == LS_DONE) return;
+	const batch_args & a = g.a;
+	double d[2] = {0.0, 0.0};
+	if (phase == LS_INIT || (RR && phase == LS_SEG)) {
+		// r = b - A x (x = 0 and r = b from a zero guess)
+		ls_rows<RPT>(k, [&](int64_t r, int j) {
+			const double bi = a.b[r];
+			double ri = bi;
+			if (!RR && a.use_zero_guess) a.x[r] = 0.0;
+			else ri = bi - ls_row<double>(a, a.dg_v64, r, a.x);
+			a.r[r] = ri;
+			d[0] += ri * ri;
+			d[1] += bi * bi;
+		});
+		store_block_partials<2>(d, g.pb, blockIdx.x);
+		return;
+	}
+	using T = std::conditional_t<RR, float, double>;
+	T rv[RPT], wv[RPT], dv[RPT];
+	if constexpr (RR) {
+		ls_ahead<RPT>(k, (const float *)a.fr, rv);
+		ls_ahead<RPT>(k, (const float *)a.fw, wv);
+	}
+	else {
+		ls_ahead<RPT>(k, (const double *)a.r, rv);
+		ls_ahead<RPT>(k, (const double *)a.w, wv);
+		if constexpr (JAC) ls_ahead<RPT>(k, a.dinv64, dv);
+	}
+	double pw[1], rho, tol = st.tol[g.par];
+	sum_partials<1, kLsThreads>(g.pa + k.first, k.count, pw);
+	if (phase == LS_START) {
+		__syncthreads(); // the sums share their scratch
+		double t[1];
+		sum_partials<1, kLsThreads>(g.pc + k.first, k.count, t);
+		rho = t[0];
+		if constexpr (RR) {
+			const double rh0 = sqrt(rho);
+			tol = fmax(a.seg_rtol * rh0, 0.5 * a.rtol_outer * st.bnorm * rh0 / st.res);
+		}
+	}
+	else
+		rho = st.rho[g.par];
+	const double alpha = rho / pw[0];
+	if ((int)blockIdx.x == k.first && threadIdx.x == 0) {
+		st.alpha = alpha;
+		st.rho_b = rho;
+		st.tol_b = tol;
+		st.brk = RR && !(rho > 0.0);
+	}
+	ls_rows<RPT>(k, [&](int64_t r, int j) {
+		if constexpr (RR) {
+			const float ri = (float)((-alpha) * (double)wv[j] + (double)rv[j]);
+			a.fr[r] = ri;
+			d[0] += (double)ri * (double)ri;
+		}
+		else {
+			const double ri = (-alpha) * wv[j] + rv[j];
+			a.r[r] = ri;
+			d[0] += ri * ri;
+			if constexpr (JAC) {
+				const double zi = 0.0 + dv[j] * ri;
+				a.z[r] = zi;
+				d[1] += ri * zi;
+			}
+		}
+	});
+	__syncthreads(); // the reductions share their scratch
+	store_block_partials<2>(d, g.pb, blockIdx.x);
+}
+
+template<bool RR, bool JAC, int RPT>
+__global__ __launch_bounds__(kLsThreads) void ls_c_kernel(ls_args g) {
+	const ls_block k = g.blocks[blockIdx.x];
+	ls_state & st = g.st[k.sys];
+	const batch_args & a = g.a;
+	const int phase = st.phase[g.par], nx = g.par ^ 1;
+	const bool lead = (int)blockIdx.x == k.first && threadIdx.x == 0;
+	if (phase == LS_DONE) {
+		if (lead) st.phase[nx] = LS_DONE;
+		return;
+	}
+	const int seg = st.seg[g.par], it = st.it[g.par];
+	auto finish = [&](int iters, int status, double res) {
+		if (!lead) return;
+		st.phase[nx] = LS_DONE;
+		a.iters[k.sys] = iters;
+		a.status[k.sys] = status;
+		a.res[k.sys] = res;
+		if (a.inner_iters) a.inner_iters[k.sys] = st.inner;
+		atomicSub(g.active, 1);
+	};
+	using T = std::conditional_t<RR, float, double>;
+	T pv[RPT], zv[RPT], xv[RPT];
+	if constexpr (RR) {
+		ls_ahead<RPT>(k, (const float *)a.fp, pv);
+		ls_ahead<RPT>(k, (const float *)a.fr, zv);
+		ls_ahead<RPT>(k, (const float *)a.fd, xv);
+	}
+	else {
+		ls_ahead<RPT>(k, (const double *)a.p, pv);
+		ls_ahead<RPT>(k, (const double *)(JAC ? a.z : a.r), zv);
+		ls_ahead<RPT>(k, (const double *)a.x, xv);
+	}
+	double t[2];
+	sum_partials<2, kLsThreads>(g.pb + 2 * (size_t)k.first, k.count, t);
+	const double res = sqrt(t[0]);
+	if (phase == LS_INIT || (RR && phase == LS_SEG)) {
+		const bool first = phase == LS_INIT;
+		double bnorm = first ? sqrt(t[1]) : st.bnorm;
+		if (bnorm == 0.0) bnorm = 1.0;
+		if constexpr (RR) {
+			const int nseg = first ? 0 : seg + 1;
+			if (res / bnorm <= a.rtol_outer || res == 0.0) {
+				finish(nseg, FSX_CONVERGED_RTOL, res);
+				return;
+			}
+			if (nseg >= a.max_outer) {
+				finish(nseg, FSX_DIVERGED_ITERS, res);
+				return;
+			}
+			const double inv = first ? 1.0 / res : st.inv;
+			// rh <- (float)(S r / c); p = rh, or p += rh_new - rh_old; y = 0
+			double d[1] = {0.0};
+			ls_rows<RPT>(k, [&](int64_t r, int j) {
+				const float vi = (float)(a.sym[r] * (a.r[r] * inv));
+				a.fp[r] = first ? vi : (float)((double)pv[j] + ((double)vi - (double)zv[j]));
+				a.fr[r] = vi;
+				a.fd[r] = 0.0f;
+				d[0] += (double)vi * (double)vi;
+			});
+			__syncthreads();
+			store_block_partials<1>(d, g.pc, blockIdx.x);
+			if (lead) {
+				if (first) {
+					st.c = res;
+					st.inv = inv;
+					st.bnorm = bnorm;
+				}
+				st.res = res;
+				st.phase[nx] = LS_START;
+				st.seg[nx] = nseg;
+				st.it[nx] = 0;
+			}
+		}
+		else {
+			const double tol = a.rtol * bnorm;
+			if (res < tol) {
+				finish(0, FSX_CONVERGED_RTOL, res);
+				return;
+			}
+			if (a.maxiter <= 0) {
+				finish(0, FSX_DIVERGED_ITERS, res);
+				return;
+			}
+			double d[1] = {0.0};
+			ls_rows<RPT>(k, [&](int64_t r, int j) {
+				const double ri = a.r[r];
+				double zi = ri;
+				if constexpr (JAC) {
+					zi = 0.0 + a.dinv64[r] * ri;
+					a.z[r] = zi;
+				}
+				a.p[r] = zi;
+				d[0] += zi * ri;
+			});
+			__syncthreads();
+			store_block_partials<1>(d, g.pc, blockIdx.x);
+			if (lead) {
+				st.tol[nx] = tol;
+				st.phase[nx] = LS_START;
+				st.it[nx] = 0;
+				st.seg[nx] = 0;
+			}
+		}
+		return;
+	}
+	const double alpha = st.alpha, rho = st.rho_b, tol = st.tol_b;
+	if constexpr (RR) {
+		if (st.brk) { // the scaled residual vanished in FP32
+			finish(seg, FSX_DIVERGED_BREAKDOWN, st.res);
+			return;
+		}
+		const double rho1 = t[0], beta = rho1 / rho;
+		ls_rows<RPT>(k, [&](int64_t r, int j) {
+			a.fd[r] = (float)(alpha * (double)pv[j] + (double)xv[j]);
+			a.fp[r] = (float)(beta * (double)pv[j] + (double)zv[j]);
+		});
+		if (lead) {
+			const bool end = res < tol || it + 1 >= a.maxiter;
+			st.rho[nx] = rho1;
+			st.tol[nx] = tol;
+			st.it[nx] = it + 1;
+			st.seg[nx] = seg;
+			st.inner = st.inner + 1;
+			st.phase[nx] = end ? LS_SEG : LS_ITER;
+		}
+	}
+	else {
+		const bool met = res < tol, last = it + 1 >= a.maxiter;
+		const double rho1 = JAC ? t[1] : t[0], beta = rho1 / rho;
+		if (met || last) {
+			ls_rows<RPT>(k, [&](int64_t r, int j) { a.x[r] = alpha * pv[j] + xv[j]; });
+			finish(met ? it + 1 : 0, met ? FSX_CONVERGED_RTOL : FSX_DIVERGED_ITERS, res);
+			return;
+		}
+		ls_rows<RPT>(k, [&](int64_t r, int j) {
+			a.x[r] = alpha * pv[j] + xv[j];
+			a.p[r] = beta * pv[j] + zv[j];
+		});
+		if (lead) {
+			st.rho[nx] = rho1;
+			st.tol[nx] = tol;
+			st.it[nx] = it + 1;
+			st.seg[nx] = 0;
+			st.phase[nx] = LS_ITER;
+		}
+	}
+}
+
+// Every system's state before the first launch: both slots `init`.
+__global__ void ls_start_kernel(int64_t nsys, ls_state * st, int * active) {
+	const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+	if (i == 0) *active = (int)nsys;
+	if (i >= nsys) return;
+	ls_state s{};
+	s.phase[0] = s.phase[1] = LS_INIT;
+	st[i] = s;
+}
+
 // Device check that every row of system s only references columns of s.
 __global__ void batch_check_kernel(int64_t nsys, const int64_t * rows,
                                    const int32_t * rp, const int32_t * ci,
@@ -771,6 +1163,131 @@ void copy_out(fsx_ctx * ctx, const batch_outputs & o, int64_t nsys, int * iters,
 	FSX_HIP(hipStreamSynchronize(ctx->stream));
 }
 
+// Lockstep or one workgroup per system, for the slice-offset mapping of a
+// batch without empty systems.  One workgroup's iteration of a small system
+// takes less than three launches, and while every CU holds a system whose
+// vectors stay in its share of the caches it wastes nothing; lockstep wins
+// where a few systems, or one much larger than the rest, leave CUs idle, and
+// where a system outgrows the caches.  Measured to 1e-10 (ms, residual
+// replacement / FP64 CG, lockstep against the best workgroup size):
+//   160 systems of 8^3 .. 40^3   12.0        against 128 (256 threads)
+//    16 of 24^3                   3.0 /  2.7 against  5.3 /  8.1
+//    16 of 16^3                   1.8 /  1.6 against  1.3 /  1.9
+//   256 of 24^3                  10.3 / 14.2 against  7.7 / 15.0
+//   256 of 16^3                   3.4 /  3.8 against  1.8 /  2.3
+//  2048 of 16^3                  13.8 / 22.2 against 12.0 / 16.3
+//  2048 of 8^3 .. 48^3            259 /  527 against  337 /  546
+bool use_lockstep(const fsx_batch * B, const fsx_csr * A32) {
+	if (B->fixed || B->mapping != 2 || (A32 && !A32->dg_vals)) return false;
+	if (B->min_rows <= 0 || B->max_rows <= 4096) return false;
+	const bool idle = B->max_rows * B->ctx->num_cus > 2 * B->A->nrows;
+	return idle || B->max_rows >= 32768;
+}
+
+// Workgroup size of the kernel of one workgroup per system until the caller
+// sets or tunes one: few systems leave a CU to each, so all its waves serve
+// it (256 systems of 16^3: 1.8 ms at 1024 threads, 4.0 at 256); with many, a
+// CU holds several and small groups synchronise for less (2048 of 8^3: 1.0
+// ms at 256, 2.3 at 1024).
+int default_workgroup(const fsx_batch * B) {
+	if (B->max_rows >= 1536 && B->nsys <= 2 * (int64_t)B->ctx->num_cus) return 1024;
+	return B->max_rows >= 4096 ? 512 : 256;
+}
+
+void ls_prepare(fsx_ctx * ctx, fsx_batch * B) {
+	if (B->ls_blocks) return;
+	// rows per thread: more rows share the sums of a system's partials, fewer
+	// give every CU several blocks (1 / 2 / 4, residual replacement: 16 of
+	// 24^3 3.0 / 3.1 / 3.6 ms; 160 of 8^3 .. 40^3 14.1 / 12.0 / 12.8; 2048 of
+	// 16^3 18.4 / 14.6 / 13.8; 8 was slower than 4 on all)
+	const int64_t per_cu = B->A->nrows / ((int64_t)ctx->num_cus * kLsThreads);
+	const int rpt = per_cu >= 64 ? 4 : per_cu >= 8 ? 2 : 1;
+	const int64_t rows = (int64_t)rpt * kLsThreads;
+	std::vector<ls_block> blk;
+	for (int64_t s = 0; s < B->nsys; ++s) {
+		const int64_t lo = B->h_rows[s], hi = B->h_rows[s + 1];
+		const size_t first = blk.size();
+		for (int64_t base = lo / kSliceRows * kSliceRows; base < hi; base += rows)
+			blk.push_back({(int)s, (int)first, 0, 0, base, lo, hi});
+		for (size_t q = first; q < blk.size(); ++q) blk[q].count = (int)(blk.size() - first);
+	}
+	FSX_REQUIRE(blk.size() < ((size_t)1 << 31), "batch: too many row blocks");
+	auto d = std::make_unique<dbuf>(blk.size() * sizeof(ls_block));
+	FSX_HIP(hipMemcpyAsync(d->p, blk.data(), blk.size() * sizeof(ls_block),
+	                       hipMemcpyHostToDevice, ctx->stream));
+	B->ls_st = std::make_unique<dbuf>(B->nsys * sizeof(ls_state));
+	B->ls_part = std::make_unique<dbuf>(blk.size() * 4 * sizeof(double));
+	B->ls_active = std::make_unique<dbuf>(256);
+	B->rpt = rpt;
+	B->nblocks = (int64_t)blk.size();
+	FSX_HIP(hipStreamSynchronize(ctx->stream)); // blk goes out of scope
+	B->ls_blocks = std::move(d);
+}
+
+template<bool RR, bool JAC, int RPT>
+void ls_round(fsx_ctx * ctx, const fsx_batch * B, const ls_args & g) {
+	const dim3 grid((unsigned)B->nblocks), thr(kLsThreads);
+	hipLaunchKernelGGL((ls_a_kernel<RR, RPT>), grid, thr, 0, ctx->stream, g);
+	hipLaunchKernelGGL((ls_b_kernel<RR, JAC, RPT>), grid, thr, 0, ctx->stream, g);
+	hipLaunchKernelGGL((ls_c_kernel<RR, JAC, RPT>), grid, thr, 0, ctx->stream, g);
+	FSX_HIP(hipGetLastError());
+	ctx->launches += 3;
+}
+
+// Rounds in chunks, one in flight while the host reads the count of running
+// systems after the one before.  Every system ends after at most
+// max_outer (maxiter + 1) + 1 rounds, so the loop does.
+template<bool RR, bool JAC>
+void ls_solve(fsx_ctx * ctx, fsx_batch * B, const batch_args & a) {
+	ls_prepare(ctx, B);
+	ls_args g{};
+	g.a = a;
+	g.blocks = (const ls_block *)B->ls_blocks->p;
+	g.st = (ls_state *)B->ls_st->p;
+	g.pa = (double *)B->ls_part->p;
+	g.pb = g.pa + B->nblocks;
+	g.pc = g.pb + 2 * B->nblocks;
+	g.active = (int *)B->ls_active->p;
+	hipLaunchKernelGGL(ls_start_kernel, dim3((unsigned)((B->nsys + 255) / 256)), dim3(256), 0,
+	                   ctx->stream, B->nsys, g.st, g.active);
+	FSX_HIP(hipGetLastError());
+	ctx->launches++;
+	constexpr int kRounds = 8; // even: the state slot follows the launch
+	int * seen = (int *)ctx->host_scalars; // pinned; one per chunk in flight
+	struct events {
+		hipEvent_t e[2] = {nullptr, nullptr};
+		~events() {
+			for (auto v : e)
+				if (v) (void)hipEventDestroy(v);
+		}
+	} ev;
+	for (auto & v : ev.e) FSX_HIP(hipEventCreateWithFlags(&v, hipEventDisableTiming));
+	auto chunk = [&](int slot) {
+		for (int q = 0; q < kRounds; ++q) {
+			g.par = q & 1;
+			if (B->rpt == 4) ls_round<RR, JAC, 4>(ctx, B, g);
+			else if (B->rpt == 2) ls_round<RR, JAC, 2>(ctx, B, g);
+			else ls_round<RR, JAC, 1>(ctx, B, g);
+		}
+		FSX_HIP(hipMemcpyAsync(&seen[slot], g.active, sizeof(int), hipMemcpyDeviceToHost,
+		                       ctx->stream));
+		FSX_HIP(hipEventRecord(ev.e[slot], ctx->stream));
+	};
+	try {
+		chunk(0);
+		for (int k = 0;; ++k) {
+			chunk((k + 1) & 1);
+			FSX_HIP(hipEventSynchronize(ev.e[k & 1]));
+			ctx->host_syncs++;
+			if (seen[k & 1] <= 0) break;
+		}
+	}
+	catch (...) {
+		(void)hipStreamSynchronize(ctx->stream);
+		throw;
+	}
+}
+
 void set_order(fsx_ctx * ctx, fsx_batch * B, const std::vector<int> & ord) {
 	FSX_HIP(hipMemcpyAsync(B->order->p, ord.data(), ord.size() * sizeof(int),
 	                       hipMemcpyHostToDevice, ctx->stream));
@@ -826,9 +1343,15 @@ int fsx_batch_create(fsx_ctx * ctx, const fsx_csr * A, int64_t nsys,
 		                       ctx->stream));
 		FSX_HIP(hipStreamSynchronize(ctx->stream));
 		FSX_REQUIRE(bad == 0, "a system's rows reference columns of another system");
+		for (int64_t s = 0; s < nsys; ++s) {
+			const int64_t m = sys_rows[s + 1] - sys_rows[s];
+			B->max_rows = std::max(B->max_rows, m);
+			B->min_rows = s ? std::min(B->min_rows, m) : m;
+		}
 		set_order(ctx, B.get(), lpt_order(B.get()));
 		B->mapping = has_sdia(A) ? 2 : has_sliced(A) ? 0 : 1;
 		B->lanes = B->mapping == 1 ? 4 : 1;
+		B->wg = default_workgroup(B.get());
 		ctx_retain(ctx);
 		*out = B.release();
 	});
@@ -872,6 +1395,7 @@ int fsx_batch_set_config(fsx_batch * B, int wg, int mapping, int lanes) {
 		B->wg = wg;
 		B->mapping = mapping;
 		B->lanes = mapping == 1 ? lanes : 1;
+		B->fixed = true;
 	});
 }
 
@@ -896,7 +1420,11 @@ static void batched_cg_run(fsx_ctx * ctx, fsx_batch * B, batch_work & W,
 		a.status = (int *)o.status->p;
 		a.res = (double *)o.res->p;
 		a.inner_iters = nullptr;
-		if (B->nsys > 0) {
+		if (use_lockstep(B, nullptr)) {
+			if (dinv) ls_solve<false, true>(ctx, B, a);
+			else ls_solve<false, false>(ctx, B, a);
+		}
+		else if (B->nsys > 0) {
 			if (dinv) launch<true, false>(ctx, B, a);
 			else launch<false, false>(ctx, B, a);
 		}
@@ -1048,7 +1576,8 @@ int fsx_batched_rr_cg(fsx_ctx * ctx, fsx_batch * B, const fsx_csr * A32,
 		a.status = (int *)o.status->p;
 		a.res = (double *)o.res->p;
 		a.inner_iters = (int *)o.inner->p;
-		if (B->nsys > 0) launch<false, true>(ctx, B, a);
+		if (use_lockstep(B, A32)) ls_solve<true, false>(ctx, B, a);
+		else if (B->nsys > 0) launch<false, true>(ctx, B, a);
 		copy_out(ctx, o, B->nsys, segments, status, res, inner_iters);
 	});
 }
@@ -1094,6 +1623,7 @@ int fsx_batch_tune(fsx_ctx * ctx, fsx_batch * B, const fsx_vec * dinv,
 		std::vector<int> samp(m);
 		for (int64_t i = 0; i < m; ++i) samp[i] = ord[(i * B->nsys) / m];
 		fsx_batch S;
+		S.fixed = true; // the candidates are the one-workgroup kernel's
 		S.ctx = ctx;
 		S.A = B->A;
 		S.nsys = m;

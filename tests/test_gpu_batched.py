@@ -239,3 +239,74 @@ def test_batched_full_edge_range_matches_oracle(ctx):
                          O.Settings(maxiter=1000, rtol=1e-10, use_zero_guess=True),
                          P=O.prec(1, Ao.dinv()))
         assert rel(xg[sl], xo) <= 1e-8, (k, e[k])
+
+
+@pytest.mark.parametrize("edges", [
+    (17,),                      # one system past the lockstep size, one block per slice edge
+    (17, 8, 1, 5, 2),           # tiny systems beside it, none slice-aligned
+    (24,) * 3 + (16,) * 5,      # one row a thread
+    (48, 48, 47, 33, 9),        # two rows a thread
+    (64,) * 16 + (63,) * 2,     # four rows a thread
+])
+def test_lockstep_matches_one_workgroup_per_system(ctx, edges):
+    """Batches solved in lockstep (three launches advance every system) against
+    the kernel of one workgroup per system, which a configuration set by the
+    caller names: FP64 CG with and without Jacobi from zero and other guesses,
+    exhausted iterations, and the FP32 CG with residual replacement.  Both run
+    the same recurrences with sums in another order: iteration counts within
+    two, solutions within the solves' own tolerance."""
+    probs = [P.diffusion3d(e, P.lognormal_field(e, 1.0, 4.0, 900 + k))
+             for k, e in enumerate(edges)]
+    S = sp.block_diag([sp.csr_matrix((v, ci, rp)) for rp, ci, v in probs], format="csr")
+    S.sort_indices()
+    rows = np.concatenate([[0], np.cumsum([e ** 3 for e in edges])]).astype(np.int64)
+    n = int(rows[-1])
+    A = ctx.csr(S.indptr.astype(np.int32), S.indices.astype(np.int32), S.data)
+    A.set_plan(3)
+    A32 = A.convert(fsx.F32)
+    A32.set_values_sym_scaled(A)
+    b = P.uniform(n, 31)
+    x0 = P.uniform(n, 32)
+    bd, d = ctx.vec(b), A.diag_inv()
+    lock, one = fsx.Batch(A, rows), fsx.Batch(A, rows)
+    one.set_config(512, 2, 1)
+
+    def both(f):
+        out = []
+        for B in (lock, one):
+            x = ctx.vec(x0)
+            out.append((f(B, x), x.get()))
+        return out
+
+    for dinv in (d, None):
+        for s in (dict(maxiter=3000, rtol=1e-10, use_zero_guess=True),
+                  dict(maxiter=3000, rtol=1e-10), dict(maxiter=7, rtol=1e-10),
+                  dict(maxiter=0, rtol=1e-10), dict(maxiter=10, rtol=1e6)):
+            (l, xl), (o, xo) = both(lambda B, x: B.cg(bd, x, fsx.Settings(**s), dinv=dinv))
+            np.testing.assert_array_equal(l[1], o[1])
+            # without a preconditioner CG on the lognormal operator loses
+            # orthogonality over ~1000 iterations, and another order of the
+            # sums moves its end by up to 1% (the bar of the single solves)
+            assert (np.abs(l[0] - o[0]) <= (2 if dinv is not None else 2 + 0.01 * o[0])).all()
+            # stopped by the iteration count: the same iterates to rounding;
+            # by the residual: each within the tolerance of the solution
+            assert rel(xl, xo) <= (1e-12 if s["maxiter"] <= 10 else 1e-8)
+            np.testing.assert_allclose(l[2], o[2], rtol=1e-6 if s["maxiter"] <= 10 else 1.0)
+    for s, segs in ((fsx.Settings(maxiter=3000, rtol=3e-2), 100),
+                    (fsx.Settings(maxiter=5, rtol=3e-2), 3), (fsx.Settings(maxiter=9, rtol=0.5), 0)):
+        (l, xl), (o, xo) = both(lambda B, x: B.rr_cg(A32, bd, x, 1e-10, s, max_segments=segs))
+        np.testing.assert_array_equal(l[2], o[2])
+        assert np.abs(l[0] - o[0]).max() <= 1
+        assert (np.abs(l[1] - o[1]) <= 3 + 0.02 * o[1]).all()
+        assert rel(xl, xo) <= (1e-8 if segs == 100 else 1e-5)  # FP32 iterates short of the end
+        if segs == 100:
+            r = b - S @ xl
+            for k in range(len(edges)):
+                sl = slice(rows[k], rows[k + 1])
+                assert np.linalg.norm(r[sl]) / np.linalg.norm(b[sl]) <= 1.01e-10
+    # repeatable, bit for bit
+    x1, x2 = ctx.vec(x0), ctx.vec(x0)
+    s = fsx.Settings(maxiter=3000, rtol=1e-10)
+    lock.cg(bd, x1, s, dinv=d)
+    lock.cg(bd, x2, s, dinv=d)
+    np.testing.assert_array_equal(x1.get(), x2.get())
