@@ -73,6 +73,17 @@ struct epi_cg_spmv {
 		w[i] = wi;
 		d[0] += (double)wi * pv; // w.dot(p)
 	}
+	static constexpr bool runs = true;
+	template<int R, class X>
+	__device__ void row_run(int64_t i, const ACC (&s)[R], double (&d)[NV], const X (&pi)[R]) const {
+		T o[R];
+#pragma unroll
+		for (int j = 0; j < R; ++j) {
+			o[j] = (T)s[j];
+			d[0] += (double)o[j] * (double)pi[j];
+		}
+		st_run<R>(w + i, o);
+	}
 	__device__ void block_end(const double (&d)[NV], unsigned blk,
 	                          unsigned) const {
 		store_block_partials<NV>(d, partials, blk);
@@ -275,6 +286,18 @@ struct epi_cg_spmv2 {
 		d[0] += (double)wi * pv;          // w.dot(p)
 		d[1] += (double)wi * (double)wi;  // w.dot(w)
 	}
+	static constexpr bool runs = true;
+	template<int R, class X>
+	__device__ void row_run(int64_t i, const ACC (&s)[R], double (&d)[NV], const X (&pi)[R]) const {
+		T o[R];
+#pragma unroll
+		for (int j = 0; j < R; ++j) {
+			o[j] = (T)s[j];
+			d[0] += (double)o[j] * (double)pi[j];
+			d[1] += (double)o[j] * (double)o[j];
+		}
+		st_run<R>(w + i, o);
+	}
 	__device__ void block_end(const double (&d)[NV], unsigned blk, unsigned) const {
 		store_block_partials<NV>(d, partials, blk);
 	}
@@ -372,6 +395,18 @@ struct epi_res_norm {
 		const T ri = b[i] - (T)s;
 		r[i] = ri;
 		d[0] += (double)ri * (double)ri;
+	}
+	static constexpr bool runs = true;
+	template<int R, class X>
+	__device__ void row_run(int64_t i, const ACC (&s)[R], double (&d)[NV], const X (&)[R]) const {
+		T o[R];
+		ld_run<R, false>(b, i, o);
+#pragma unroll
+		for (int j = 0; j < R; ++j) {
+			o[j] -= (T)s[j];
+			d[0] += (double)o[j] * (double)o[j];
+		}
+		st_run<R>(r + i, o);
 	}
 	__device__ void block_end(const double (&d)[NV], unsigned blk,
 	                          unsigned) const {
@@ -500,7 +535,7 @@ static void add_layout(entry & e, const fsx_csr * A) {
 	add(X.dg_off);
 	add(X.dg_mask);
 	add(A->dg_vals);
-	add(X.st_mask);
+	add(X.st_bits);
 	add(A->st_vals);
 }
 } // namespace graph_ledger
@@ -550,11 +585,12 @@ static void append_layout(std::vector<const void *> & key, const fsx_csr * A) {
 	const csr_index & X = *A->idx;
 	key.insert(key.end(), {p(X.rowptr), p(X.colind), p(A->vals), p(X.sl_ptr), p(X.sl_col),
 	                       p(A->sl_vals), p(X.dg_ptr), p(X.dg_off), p(X.dg_mask),
-	                       p(A->dg_vals), p(X.st_mask), p(A->st_vals),
+	                       p(A->dg_vals), p(X.st_bits), p(A->st_vals),
 	                       (const void *)(intptr_t)A->nrows,
 	                       (const void *)(intptr_t)A->nnz,
 	                       (const void *)(intptr_t)A->plan_kind,
-	                       (const void *)(intptr_t)A->plan_lanes});
+	                       (const void *)(intptr_t)A->plan_lanes,
+	                       (const void *)(intptr_t)(A->st_full + 2 * A->st_serves)});
 }
 } // namespace fsx
 
@@ -1031,6 +1067,15 @@ struct epi_cg_residual {
 	__device__ void row(int64_t i, ACC s, double (&)[NV], XI &&) const {
 		r[i] = b[i] - (T)s;
 	}
+	static constexpr bool runs = true;
+	template<int R, class X>
+	__device__ void row_run(int64_t i, const ACC (&s)[R], double (&)[NV], const X (&)[R]) const {
+		T o[R];
+		ld_run<R, false>(b, i, o);
+#pragma unroll
+		for (int j = 0; j < R; ++j) o[j] -= (T)s[j];
+		st_run<R>(r + i, o);
+	}
 	__device__ void block_end(const double (&)[NV], unsigned, unsigned) const {}
 };
 
@@ -1246,6 +1291,18 @@ struct epi_bcg_v {
 		v[i] = vi;
 		d[0] += rti * (double)vi; // r_tilde.dot(v)
 	}
+	static constexpr bool runs = true;
+	template<int R, class X>
+	__device__ void row_run(int64_t i, const ACC (&s)[R], double (&d)[NV], const X (&)[R]) const {
+		T o[R], t[R];
+		ld_run<R, false>(rt, i, t);
+#pragma unroll
+		for (int j = 0; j < R; ++j) {
+			o[j] = (T)s[j];
+			d[0] += (double)t[j] * (double)o[j];
+		}
+		st_run<R>(v + i, o);
+	}
 	__device__ void block_end(const double (&d)[NV], unsigned blk, unsigned) const {
 		store_block_partials<NV>(d, partials, blk);
 	}
@@ -1317,6 +1374,19 @@ struct epi_bcg_t {
 		t[i] = ti;
 		d[0] += (double)ti * (double)ti; // t.dot(t)
 		d[1] += (double)ti * si; // t.dot(s)
+	}
+	static constexpr bool runs = true;
+	template<int R, class X>
+	__device__ void row_run(int64_t i, const ACC (&sum)[R], double (&d)[NV], const X (&)[R]) const {
+		T o[R], si[R];
+		ld_run<R, false>(s, i, si);
+#pragma unroll
+		for (int j = 0; j < R; ++j) {
+			o[j] = (T)sum[j];
+			d[0] += (double)o[j] * (double)o[j];
+			d[1] += (double)o[j] * (double)si[j];
+		}
+		st_run<R>(t + i, o);
 	}
 	__device__ void block_end(const double (&d)[NV], unsigned blk, unsigned) const {
 		store_block_partials<NV>(d, partials, blk);
@@ -1581,8 +1651,13 @@ struct gather_dinv {
 	const double * x;
 	__device__ __forceinline__ void init() {}
 	__device__ __forceinline__ double operator()(int64_t c) const { return 0.0 + dinv[c] * x[c]; }
-	__device__ __forceinline__ double at32(uint32_t c) const {
-		return 0.0 + ld32(dinv, c) * ld32(x, c);
+	template<int R, bool O32>
+	__device__ __forceinline__ void run(int64_t off, int64_t r, double (&o)[R]) const {
+		double di[R];
+		ld_run<R, O32>(dinv + off, r, di);
+		ld_run<R, O32>(x + off, r, o);
+#pragma unroll
+		for (int j = 0; j < R; ++j) o[j] = 0.0 + di[j] * o[j];
 	}
 };
 
@@ -1603,6 +1678,20 @@ struct epi_gm_v {
 		if constexpr (LEFTJ) vi = 0.0 + dinv[i] * vi; // P.apply(z, v)
 		v[i] = vi;
 		d[0] += (double)vi * b0i; // v.dot(basis[0])
+	}
+	static constexpr bool runs = true;
+	template<int R, class X>
+	__device__ void row_run(int64_t i, const ACC (&s)[R], double (&d)[NV], const X (&)[R]) const {
+		T o[R], b[R], di[R];
+		ld_run<R, false>(b0, i, b);
+		if constexpr (LEFTJ) ld_run<R, false>(dinv, i, di);
+#pragma unroll
+		for (int j = 0; j < R; ++j) {
+			o[j] = (T)s[j];
+			if constexpr (LEFTJ) o[j] = 0.0 + di[j] * o[j];
+			d[0] += (double)o[j] * (double)b[j];
+		}
+		st_run<R>(v + i, o);
 	}
 	__device__ void block_end(const double (&d)[NV], unsigned blk, unsigned) const {
 		store_block_partials<NV>(d, partials, blk);

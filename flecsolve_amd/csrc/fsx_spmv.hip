@@ -23,6 +23,14 @@ struct epi_store {
 	__device__ bool skip() const { return false; }
 	template<class XI>
 	__device__ void row(int64_t i, ACC s, double (&)[NV], XI &&) const { y[i] = (Y)s; }
+	static constexpr bool runs = true;
+	template<int R, class X>
+	__device__ void row_run(int64_t i, const ACC (&s)[R], double (&)[NV], const X (&)[R]) const {
+		Y o[R];
+#pragma unroll
+		for (int j = 0; j < R; ++j) o[j] = (Y)s[j];
+		st_run<R>(y + i, o);
+	}
 	__device__ void block_end(const double (&)[NV], unsigned, unsigned) const {}
 };
 
@@ -38,6 +46,15 @@ struct epi_residual {
 	template<class XI>
 	__device__ void row(int64_t i, ACC s, double (&)[NV], XI &&) const {
 		r[i] = b[i] - (Y)s;
+	}
+	static constexpr bool runs = true;
+	template<int R, class X>
+	__device__ void row_run(int64_t i, const ACC (&s)[R], double (&)[NV], const X (&)[R]) const {
+		Y o[R];
+		ld_run<R, false>(b, i, o);
+#pragma unroll
+		for (int j = 0; j < R; ++j) o[j] -= (Y)s[j];
+		st_run<R>(r + i, o);
 	}
 	__device__ void block_end(const double (&)[NV], unsigned, unsigned) const {}
 };
@@ -81,6 +98,17 @@ struct epi_dot {
 		const Y wi = (Y)s;
 		w[i] = wi;
 		d[0] += (double)wi * pv;
+	}
+	static constexpr bool runs = true;
+	template<int R, class X>
+	__device__ void row_run(int64_t i, const ACC (&s)[R], double (&d)[NV], const X (&pi)[R]) const {
+		Y o[R];
+#pragma unroll
+		for (int j = 0; j < R; ++j) {
+			o[j] = (Y)s[j];
+			d[0] += (double)o[j] * (double)pi[j];
+		}
+		st_run<R>(w + i, o);
 	}
 	__device__ void block_end(const double (&d)[NV], unsigned blk,
 	                          unsigned) const {
@@ -359,94 +387,97 @@ bool ensure_sdia(fsx_ctx * ctx, fsx_csr * A, const void * host_rowptr,
 	return true;
 }
 
-// ---- symmetric stencil layout ---------------------------------------------
+// ---- stencil layout -------------------------------------------------------
 
 // Host analysis (once per pattern): the ascending union of all rows' column
-// offsets, at most kStencilMax and closed under negation; every entry's
-// mirror present (row r has column r + o exactly when row r + o has column
-// r); the stored slots (offsets >= 0, whole slices) within 25% of the
-// entries they hold (+ one slice).  Builds the lane masks per (slice, offset).
+// offsets, at most kStencilMax; the presence bits of every row; the stored
+// slots (whole slices) within 25% of the entries they hold (+ one slice) in
+// the form that applies.  The structure is symmetric when the list is closed
+// under negation and every entry's mirror is present (row r has column r + o
+// exactly when row r + o has column r).
 template<class I>
-static bool stencil_analyze(fsx_ctx * ctx, int64_t nrows, const I * rp, const I * ci,
-                            csr_index & X) {
+static int stencil_analyze(fsx_ctx * ctx, int64_t nrows, const I * rp, const I * ci,
+                           csr_index & X) {
 	std::vector<int64_t> offs;
 	for (int64_t r = 0; r < nrows; ++r)
 		for (I e = rp[r]; e < rp[r + 1]; ++e) {
 			// columns strictly ascending: the layout sums in offset order
-			if (e > rp[r] && ci[e] <= ci[e - 1]) return false;
+			if (e > rp[r] && ci[e] <= ci[e - 1]) return 0;
 			const int64_t o = (int64_t)ci[e] - r;
-			if (o < INT32_MIN || o > INT32_MAX) return false; // offsets are stored as int32
+			if (o < INT32_MIN || o > INT32_MAX) return 0; // offsets are stored as int32
 			if (std::find(offs.begin(), offs.end(), o) == offs.end()) {
-				if ((int)offs.size() == kStencilMax) return false;
+				if ((int)offs.size() == kStencilMax) return 0;
 				offs.push_back(o);
 			}
 		}
-	if (offs.empty()) return false;
+	if (offs.empty()) return 0;
 	std::sort(offs.begin(), offs.end());
 	const int w = (int)offs.size();
 	auto find = [&](int64_t o) {
 		return (int)(std::lower_bound(offs.begin(), offs.end(), o) - offs.begin());
 	};
 	int jm[kStencilMax];
+	bool sym = true;
 	for (int j = 0; j < w; ++j) {
 		jm[j] = find(-offs[j]);
-		if (jm[j] == w || offs[jm[j]] != -offs[j]) return false;
+		sym = sym && jm[j] < w && offs[jm[j]] == -offs[j];
 	}
 	const int nneg = find(0);
 	const int wu = w - nneg;
-	std::vector<uint8_t> bits((size_t)nrows, 0);
-	int64_t upper = 0;
+	const int64_t ns = (nrows + kSliceRows - 1) / kSliceRows;
+	std::vector<uint8_t> bits((size_t)(ns * kSliceRows), 0);
+	int64_t upper = 0, all = 0;
 	for (int64_t r = 0; r < nrows; ++r)
 		for (I e = rp[r]; e < rp[r + 1]; ++e) {
 			const int64_t o = (int64_t)ci[e] - r;
 			bits[(size_t)r] |= (uint8_t)(1u << find(o));
 			upper += o >= 0;
+			++all;
 		}
-	for (int64_t r = 0; r < nrows; ++r)
+	for (int64_t r = 0; r < nrows && sym; ++r)
 		for (int j = 0; j < w; ++j) {
 			if (!((bits[(size_t)r] >> j) & 1)) continue;
 			const int64_t rr = r + offs[j];
-			if (rr < 0 || rr >= nrows || !((bits[(size_t)rr] >> jm[j]) & 1)) return false;
+			if (rr < 0 || rr >= nrows || !((bits[(size_t)rr] >> jm[j]) & 1)) {
+				sym = false;
+				break;
+			}
 		}
-	const int64_t ns = (nrows + kSliceRows - 1) / kSliceRows;
-	if (ns * kSliceRows * wu > upper + upper / 4 + (int64_t)kSliceRows * wu) return false;
-	std::vector<uint64_t> mask((size_t)(ns * w + kStencilMax), 0);
-	for (int64_t r = 0; r < nrows; ++r)
-		for (int j = 0; j < w; ++j)
-			if ((bits[(size_t)r] >> j) & 1)
-				mask[(size_t)((r / kSliceRows) * w + j)] |= 1ull << (r % kSliceRows);
+	auto fits = [&](int64_t arrays, int64_t held) {
+		return ns * kSliceRows * arrays <= held + held / 4 + (int64_t)kSliceRows * arrays;
+	};
+	if (sym && !fits(wu, upper)) sym = false;
+	if (!sym && !fits(w, all)) return 0;
 	X.st_w = w;
-	X.st_wu = wu;
+	X.st_wu = sym ? wu : w;
 	for (int j = 0; j < kStencilMax; ++j) {
 		X.st_off[j] = j < w ? (int32_t)offs[j] : 0;
-		X.st_ju[j] = j >= w ? 0 : offs[j] >= 0 ? j - nneg : jm[j] - nneg;
+		X.st_ju[j] = j >= w ? 0 : !sym ? j : offs[j] >= 0 ? j - nneg : jm[j] - nneg;
 	}
-	X.st_mask = std::make_unique<dbuf>(mask.size() * sizeof(uint64_t));
-	FSX_HIP(hipMemcpyAsync(X.st_mask->p, mask.data(), mask.size() * sizeof(uint64_t),
-	                       hipMemcpyHostToDevice, ctx->stream));
-	FSX_HIP(hipStreamSynchronize(ctx->stream)); // the host mask goes out of scope
-	return true;
+	X.st_bits = std::make_unique<dbuf>(bits.size());
+	FSX_HIP(hipMemcpyAsync(X.st_bits->p, bits.data(), bits.size(), hipMemcpyHostToDevice,
+	                       ctx->stream));
+	FSX_HIP(hipStreamSynchronize(ctx->stream)); // the host bits go out of scope
+	return sym ? 1 : 2;
 }
 
-// Values of the offsets >= 0 of row r (thread r of the padded slice range)
-// into the layout: zero the row's slots, then place each entry.  Rows and
-// offsets are both ascending, so one forward scan finds them.
+// Stored values of row r (thread r of the padded slice range) into the
+// layout: zero the row's slots, then place each entry.  Rows and offsets are
+// both ascending, so one forward scan finds them.
 template<class I, class V>
-__global__ void stencil_fill_kernel(int64_t nrows, int64_t nslots, const I * __restrict__ rp,
+__global__ void stencil_fill_kernel(int64_t nrows, const I * __restrict__ rp,
                                     const I * __restrict__ ci, const V * __restrict__ v,
                                     stencil_desc sd, V * __restrict__ st_val) {
 	const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-	if (r >= nslots) return;
-	const int64_t s = r / kSliceRows;
-	const int lane = (int)(r % kSliceRows);
-	for (int u = 0; u < sd.wu; ++u) st_val[(s * sd.wu + u) * kSliceRows + lane] = V(0);
+	if (r >= sd.npad) return;
+	for (int u = 0; u < sd.wu; ++u) st_val[u * sd.npad + r] = V(0);
 	if (r >= nrows) return;
 	int j = 0;
 	for (I e = rp[r]; e < rp[r + 1]; ++e) {
 		const int64_t o = (int64_t)ci[e] - r;
 		while (j < sd.w && sd.off[j] != o) ++j;
 		if (j == sd.w) return; // not this layout's structure (cannot happen)
-		if (o >= 0) st_val[(s * sd.wu + sd.ju[j]) * kSliceRows + lane] = v[e];
+		if (sd.sh[j] == 0) st_val[sd.ju[j] * sd.npad + r] = v[e];
 		++j;
 	}
 }
@@ -458,8 +489,8 @@ __device__ __forceinline__ uint64_t value_bits(float a) {
 	return (uint64_t)(uint32_t)__float_as_int(a);
 }
 
-// bad[0] = 1 when an entry at an offset < 0 differs in any bit from its
-// mirror's stored value
+// bad[0] = 1 when a mirrored entry differs in any bit from its mirror's
+// stored value
 template<class I, class V>
 __global__ void stencil_sym_check_kernel(int64_t nrows, const I * __restrict__ rp,
                                          const I * __restrict__ ci, const V * __restrict__ v,
@@ -476,93 +507,113 @@ __global__ void stencil_sym_check_kernel(int64_t nrows, const I * __restrict__ r
 			bad[0] = 1;
 			return;
 		}
-		const int64_t rr = r + o;
-		const V m = st_val[((rr / kSliceRows) * sd.wu + sd.ju[j]) * kSliceRows + rr % kSliceRows];
+		const V m = st_val[sd.ju[j] * sd.npad + r + o];
 		if (value_bits(m) != value_bits(v[e])) bad[0] = 1;
 		++j;
 	}
 }
 
-// Fill A's stencil values from its CSR values and check their symmetry
-// (one host synchronisation); sets A->st_sym.
+// Fill A's stencil values from its CSR values in the form A->st_full names;
+// true unless they are to be symmetric and are not (one host synchronisation).
 template<class I, class V>
-static void stencil_fill_t(fsx_ctx * ctx, fsx_csr * A) {
-	const int64_t nslots = ((A->nrows + kSliceRows - 1) / kSliceRows) * kSliceRows;
-	const stencil_desc sd = make_stencil_desc(*A->idx);
+static bool stencil_fill_t(fsx_ctx * ctx, fsx_csr * A) {
+	const stencil_desc sd = make_stencil_desc(*A->idx, A->st_full, A->nrows);
+	const unsigned g = (unsigned)((sd.npad + 255) / 256);
+	hipLaunchKernelGGL((stencil_fill_kernel<I, V>), dim3(g), dim3(256), 0, ctx->stream,
+	                   A->nrows, (const I *)A->rowptr(), (const I *)A->colind(),
+	                   (const V *)A->vals->p, sd, (V *)A->st_vals->p);
+	FSX_HIP(hipGetLastError());
+	ctx->launches++;
+	if (A->st_full) return true;
 	dbuf flag(sizeof(int));
 	FSX_HIP(hipMemsetAsync(flag.p, 0, sizeof(int), ctx->stream));
-	const unsigned g = (unsigned)((nslots + 255) / 256);
-	hipLaunchKernelGGL((stencil_fill_kernel<I, V>), dim3(g), dim3(256), 0, ctx->stream,
-	                   A->nrows, nslots, (const I *)A->rowptr(), (const I *)A->colind(),
-	                   (const V *)A->vals->p, sd, (V *)A->st_vals->p);
 	hipLaunchKernelGGL((stencil_sym_check_kernel<I, V>), dim3(g), dim3(256), 0, ctx->stream,
 	                   A->nrows, (const I *)A->rowptr(), (const I *)A->colind(),
 	                   (const V *)A->vals->p, sd, (const V *)A->st_vals->p, (int *)flag.p);
 	FSX_HIP(hipGetLastError());
-	ctx->launches += 2;
+	ctx->launches++;
 	int bad = 0;
 	FSX_HIP(hipMemcpyAsync(&bad, flag.p, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
 	FSX_HIP(hipStreamSynchronize(ctx->stream));
 	ctx->host_syncs++;
-	A->st_sym = bad ? 0 : 1;
+	return bad == 0;
 }
 
-static void stencil_fill(fsx_ctx * ctx, fsx_csr * A) {
-	if (A->it == FSX_I32) {
-		if (A->vt == FSX_F64) stencil_fill_t<int32_t, double>(ctx, A);
-		else stencil_fill_t<int32_t, float>(ctx, A);
-	}
-	else {
-		if (A->vt == FSX_F64) stencil_fill_t<int64_t, double>(ctx, A);
-		else stencil_fill_t<int64_t, float>(ctx, A);
-	}
+static bool stencil_fill(fsx_ctx * ctx, fsx_csr * A) {
+	if (A->it == FSX_I32)
+		return A->vt == FSX_F64 ? stencil_fill_t<int32_t, double>(ctx, A)
+		                        : stencil_fill_t<int32_t, float>(ctx, A);
+	return A->vt == FSX_F64 ? stencil_fill_t<int64_t, double>(ctx, A)
+	                        : stencil_fill_t<int64_t, float>(ctx, A);
 }
 
-// The stencil index (analysed once per pattern, from host copies of the
-// structure when given, else downloaded), then A's values in it; true when
-// A's values are symmetric and the layout can serve its products.  A's
-// stencil values are dropped when they are not.
+// A's values in a newly allocated stencil layout of the given form; false
+// (and no values) when they are to be symmetric and are not.
+static bool stencil_build(fsx_ctx * ctx, fsx_csr * A, bool full) {
+	const csr_index & X = *A->idx;
+	const int64_t ns = (A->nrows + kSliceRows - 1) / kSliceRows;
+	const size_t vsz = A->vt == FSX_F64 ? 8 : 4;
+	A->st_vals = std::make_unique<dbuf>((size_t)(ns * kSliceRows) * (full ? X.st_w : X.st_wu) * vsz);
+	A->st_full = full;
+	if (stencil_fill(ctx, A)) return true;
+	A->st_vals.reset();
+	return false;
+}
+
+// The stencil index, analysed once per pattern from host copies of the
+// structure when given, else downloaded.
+static void stencil_index(fsx_ctx * ctx, fsx_csr * A, const void * host_rowptr,
+                          const void * host_colind) {
+	csr_index & X = *A->idx;
+	if (X.st_state >= 0) return;
+	if (A->nrows == 0 || A->nrows != A->ncols) {
+		X.st_state = 0;
+		return;
+	}
+	std::vector<char> hrp, hci;
+	if (!host_rowptr || !host_colind) {
+		const size_t isz = A->it == FSX_I32 ? 4 : 8;
+		hrp.resize((A->nrows + 1) * isz);
+		hci.resize(std::max<int64_t>(1, A->nnz) * isz);
+		FSX_HIP(hipMemcpyAsync(hrp.data(), A->rowptr(), hrp.size(), hipMemcpyDeviceToHost,
+		                       ctx->stream));
+		if (A->nnz)
+			FSX_HIP(hipMemcpyAsync(hci.data(), A->colind(), A->nnz * isz,
+			                       hipMemcpyDeviceToHost, ctx->stream));
+		FSX_HIP(hipStreamSynchronize(ctx->stream));
+		host_rowptr = hrp.data();
+		host_colind = hci.data();
+	}
+	X.st_state = A->it == FSX_I32
+	                 ? stencil_analyze<int32_t>(ctx, A->nrows, (const int32_t *)host_rowptr,
+	                                            (const int32_t *)host_colind, X)
+	                 : stencil_analyze<int64_t>(ctx, A->nrows, (const int64_t *)host_rowptr,
+	                                            (const int64_t *)host_colind, X);
+}
+
+// A's values in the symmetric stencil layout; false (leaving other values as
+// they were) when its structure or values are not symmetric.
 bool ensure_stencil(fsx_ctx * ctx, fsx_csr * A, const void * host_rowptr,
                     const void * host_colind) {
-	csr_index & X = *A->idx;
-	if (X.st_state < 0) {
-		if (A->nrows == 0 || A->nrows != A->ncols) X.st_state = 0;
-		else {
-			std::vector<char> hrp, hci;
-			if (!host_rowptr || !host_colind) {
-				const size_t isz = A->it == FSX_I32 ? 4 : 8;
-				hrp.resize((A->nrows + 1) * isz);
-				hci.resize(std::max<int64_t>(1, A->nnz) * isz);
-				FSX_HIP(hipMemcpyAsync(hrp.data(), A->rowptr(), hrp.size(),
-				                       hipMemcpyDeviceToHost, ctx->stream));
-				if (A->nnz)
-					FSX_HIP(hipMemcpyAsync(hci.data(), A->colind(), A->nnz * isz,
-					                       hipMemcpyDeviceToHost, ctx->stream));
-				FSX_HIP(hipStreamSynchronize(ctx->stream));
-				host_rowptr = hrp.data();
-				host_colind = hci.data();
-			}
-			const bool ok =
-				A->it == FSX_I32
-					? stencil_analyze<int32_t>(ctx, A->nrows, (const int32_t *)host_rowptr,
-					                           (const int32_t *)host_colind, X)
-					: stencil_analyze<int64_t>(ctx, A->nrows, (const int64_t *)host_rowptr,
-					                           (const int64_t *)host_colind, X);
-			X.st_state = ok ? 1 : 0;
-		}
-	}
-	if (X.st_state != 1) return false;
-	if (!A->st_vals) {
-		const int64_t ns = (A->nrows + kSliceRows - 1) / kSliceRows;
-		const size_t vsz = A->vt == FSX_F64 ? 8 : 4;
-		A->st_vals = std::make_unique<dbuf>((size_t)(ns * kSliceRows * X.st_wu) * vsz);
-		stencil_fill(ctx, A);
-	}
-	if (A->st_sym != 1) {
-		A->st_vals.reset();
-		return false;
-	}
-	return true;
+	stencil_index(ctx, A, host_rowptr, host_colind);
+	if (A->idx->st_state != 1) return false;
+	if (A->st_vals && !A->st_full) return true;
+	auto old = std::move(A->st_vals);
+	const bool was_full = A->st_full;
+	if (stencil_build(ctx, A, false)) return true;
+	A->st_vals = std::move(old);
+	A->st_full = was_full;
+	return false;
+}
+
+// A's values in the stencil layout, in the symmetric form where they allow
+// it; false when its structure has none.
+static bool ensure_stencil_any(fsx_ctx * ctx, fsx_csr * A, const void * host_rowptr,
+                               const void * host_colind) {
+	stencil_index(ctx, A, host_rowptr, host_colind);
+	if (A->idx->st_state <= 0) return false;
+	if (A->st_vals) return true;
+	return (A->idx->st_state == 1 && stencil_build(ctx, A, false)) || stencil_build(ctx, A, true);
 }
 
 void ensure_dg_fresh(fsx_ctx * ctx, const fsx_csr * A) {
@@ -574,15 +625,21 @@ void ensure_dg_fresh(fsx_ctx * ctx, const fsx_csr * A) {
 
 void refresh_sliced_values(fsx_ctx * ctx, fsx_csr * A) {
 	++A->vals_version;
-	if (A->idx->dg_ptr && A->dg_vals) sdia_fill(ctx, A);
-	A->dg_stale = false;
-	if (A->idx->st_state == 1 && A->st_vals) {
-		// refilled in place; values that are no longer symmetric send the
-		// products to the slice-offset layout
-		stencil_fill(ctx, A);
-		if (A->st_sym != 1) {
-			A->st_vals.reset();
-			if (A->plan_kind == 4) A->plan_kind = 3;
+	if (A->st_vals && A->idx->st_state > 0 && !stencil_fill(ctx, A)) {
+		// no longer symmetric: the full form serves the products of plan 3
+		A->st_vals.reset();
+		if (A->plan_kind == 4) {
+			A->plan_kind = 3;
+			A->st_serves = true;
+		}
+		if (A->st_serves) stencil_build(ctx, A, true);
+	}
+	if (A->idx->dg_ptr && A->dg_vals) {
+		// rebuilt when next read where the products run on the stencil layout
+		if (on_stencil(A)) A->dg_stale = true;
+		else {
+			sdia_fill(ctx, A);
+			A->dg_stale = false;
 		}
 	}
 	if (!(A->idx->sl_ptr && A->sl_vals)) return;
@@ -597,8 +654,8 @@ void refresh_sliced_values(fsx_ctx * ctx, fsx_csr * A) {
 }
 
 // Short rows whose slices share few column offsets (stencils) -> slice
-// offsets, or the symmetric stencil layout when all rows draw on one short
-// offset list and the values are symmetric; other short rows of similar length -> sliced rows (padding <= 10%,
+// offsets, or the stencil layout when all rows draw on one short offset list;
+// other short rows of similar length -> sliced rows (padding <= 10%,
 // addressable with the index type); other short-row matrices -> LDS-staged
 // row blocks; long rows -> LANES lanes per row with LANES the next power of
 // two of the mean row length (2..64).
@@ -622,12 +679,12 @@ void choose_plan(fsx_ctx * ctx, fsx_csr * A, const void * host_rowptr,
 	const double per_row_budget = (double)kStreamCap / kStreamRows;
 	if (A->avg_row <= per_row_budget) {
 		if (host_colind && ensure_sdia(ctx, A, host_rowptr, host_colind, true)) {
-			// symmetric FP64 stencils: the stencil layout, the slice-offset
-			// one kept for a later change of values.  FP32 matrices stay on
-			// slice offsets, measured faster there (256^3 FP32 CG K1: 0.119
-			// against 0.123-0.130 ms for the stencil variants)
-			A->plan_kind =
-				A->vt == FSX_F64 && ensure_stencil(ctx, A, host_rowptr, host_colind) ? 4 : 3;
+			// one short offset list: the products run on the stencil layout,
+			// reported as plan 4 for symmetric FP64 matrices and as plan 3
+			// otherwise; the slice-offset layout is kept for the batched
+			// solves and for values that change
+			A->st_serves = ensure_stencil_any(ctx, A, host_rowptr, host_colind);
+			A->plan_kind = A->st_serves && A->vt == FSX_F64 && !A->st_full ? 4 : 3;
 			A->plan_lanes = 0;
 			return;
 		}
@@ -825,19 +882,17 @@ __global__ void shift_scale_sdia_kernel(int64_t nslots_total, const uint64_t * _
 	a[k] = off[q] == 0 ? alpha + v : v;
 }
 
-// The same on the stencil layout shared by f and a: slot k holds column
-// u = (k / 64) % wu, offset off[w - wu + u], of row (slice k / 64 / wu,
-// lane k % 64) when that lane's mask bit is set (absent slots stay zero).
-__global__ void shift_scale_stencil_kernel(int64_t nslots_total, const uint64_t * __restrict__ mask,
+// The same on the stencil layout shared by f and a: slot k holds row k % npad
+// at offset off[w - wu + k / npad] when that row's bit is set (absent slots
+// stay zero).
+__global__ void shift_scale_stencil_kernel(int64_t nslots_total, const uint8_t * __restrict__ bits,
                                            stencil_desc sd, const double * __restrict__ f,
                                            double alpha, double beta, double * __restrict__ a) {
 	const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
 	if (k >= nslots_total) return;
-	const int64_t c = k / kSliceRows;
-	const int64_t s = c / sd.wu;
-	const int j = sd.w - sd.wu + (int)(c % sd.wu);
-	const int lane = (int)(k % kSliceRows);
-	if (!((mask[s * sd.w + j] >> lane) & 1ull)) return;
+	const int64_t u = k / sd.npad;
+	const int j = sd.w - sd.wu + (int)u;
+	if (!((bits[k - u * sd.npad] >> j) & 1)) return;
 	const double v = beta * f[k];
 	a[k] = sd.off[j] == 0 ? alpha + v : v;
 }
@@ -1033,13 +1088,13 @@ int fsx_csr_convert(fsx_ctx * ctx, const fsx_csr * A, fsx_dtype vt,
 		if (A->dg_vals) B->dg_vals = cast_copy(*A->dg_vals, A->dg_vals->bytes / avsz);
 		else if (B->plan_kind == 3)
 			B->plan_kind = 0;
-		// FP32 copies default to slice offsets (as at creation); the stencil
-		// values are built on request (fsx_csr_set_plan)
-		if (A->st_vals && vt == FSX_F64) {
+		// a cast of symmetric values is symmetric; FP32 copies report plan 3
+		if (A->st_vals) {
 			B->st_vals = cast_copy(*A->st_vals, A->st_vals->bytes / avsz);
-			B->st_sym = A->st_sym;
+			B->st_full = A->st_full;
+			B->st_serves = A->st_serves || (A->plan_kind == 4 && vt == FSX_F32);
 		}
-		else if (B->plan_kind == 4)
+		if (B->plan_kind == 4 && (vt == FSX_F32 || !B->st_vals))
 			B->plan_kind = B->dg_vals ? 3 : 0;
 		FSX_HIP(hipStreamSynchronize(ctx->stream));
 		ctx_retain(ctx);
@@ -1115,6 +1170,7 @@ int fsx_csr_set_plan(fsx_csr * A, int kind, int lanes) {
 		}
 		A->plan_kind = kind;
 		A->plan_lanes = kind == 1 ? lanes : 0;
+		A->st_serves = false;
 	});
 }
 
@@ -1316,7 +1372,8 @@ int fsx_csr_shift_scale(fsx_ctx * ctx, const fsx_csr * F, double alpha, double b
 		// F's stencil values exist, so they are symmetric) leaves its
 		// slice-offset values behind, rebuilt when next needed.
 		++A->vals_version;
-		const bool st_serves = A->plan_kind == 4 && ix.st_state == 1 && A->st_vals && F->st_vals;
+		const bool st_same = A->st_vals && F->st_vals && A->st_full == F->st_full;
+		const bool st_serves = on_stencil(A) && st_same;
 		if (ix.dg_ptr && A->dg_vals) {
 			if (st_serves)
 				A->dg_stale = true;
@@ -1336,25 +1393,25 @@ int fsx_csr_shift_scale(fsx_ctx * ctx, const fsx_csr * F, double alpha, double b
 				A->dg_stale = false;
 			}
 		}
-		if (ix.st_state == 1 && A->st_vals) {
-			if (F->st_vals) {
-				// F's stencil values exist only when they are symmetric, and
-				// alpha I + beta F keeps that
-				const int64_t t = (int64_t)(A->st_vals->bytes / sizeof(double));
-				hipLaunchKernelGGL(shift_scale_stencil_kernel, dim3((unsigned)((t + 255) / 256)),
-				                   dim3(256), 0, ctx->stream, t, (const uint64_t *)ix.st_mask->p,
-				                   make_stencil_desc(ix), (const double *)F->st_vals->p, alpha,
-				                   beta, (double *)A->st_vals->p);
-				FSX_HIP(hipGetLastError());
-				ctx->launches++;
-				A->st_sym = 1;
+		if (st_same) {
+			// alpha I + beta F keeps the symmetry of F
+			const stencil_desc sd = make_stencil_desc(ix, A->st_full, n);
+			const int64_t t = sd.npad * sd.wu;
+			hipLaunchKernelGGL(shift_scale_stencil_kernel, dim3((unsigned)((t + 255) / 256)),
+			                   dim3(256), 0, ctx->stream, t, (const uint8_t *)ix.st_bits->p, sd,
+			                   (const double *)F->st_vals->p, alpha, beta,
+			                   (double *)A->st_vals->p);
+			FSX_HIP(hipGetLastError());
+			ctx->launches++;
+		}
+		else if (A->st_vals && !stencil_fill(ctx, A)) {
+			A->st_vals.reset();
+			if (A->plan_kind == 4) {
+				A->plan_kind = 3;
+				A->st_serves = true;
 			}
-			else
-				stencil_fill(ctx, A);
-			if (A->st_sym != 1) {
-				A->st_vals.reset();
-				if (A->plan_kind == 4) A->plan_kind = 3;
-			}
+			if (A->st_serves) stencil_build(ctx, A, true);
+			ensure_dg_fresh(ctx, A);
 		}
 		if (ix.sl_ptr && A->sl_vals) {
 			if (A->it == FSX_I32) refresh_sliced_t<int32_t, double>(ctx, A);
@@ -1539,10 +1596,10 @@ int fsx_csr_layout_bytes(const fsx_csr * A, size_t x_bytes, uint64_t * bytes) {
 		const uint64_t n = (uint64_t)A->nrows, nsl = (n + kSliceRows - 1) / kSliceRows;
 		const uint64_t vec = n * x_bytes * 2; // x read once, y written once
 		const csr_index & X = *A->idx;
-		if (A->plan_kind == 4) {
-			// value slots of the offsets >= 0; per slice one 8-byte lane mask
-			// per offset (entries at offsets < 0 re-read stored slots)
-			*bytes = nsl * kSliceRows * (uint64_t)X.st_wu * vb + nsl * (uint64_t)X.st_w * 8 + vec;
+		if (on_stencil(A)) {
+			// value slots of the stored offsets and a byte of presence bits per
+			// row (mirrored entries re-read stored slots)
+			*bytes = nsl * kSliceRows * ((uint64_t)(A->st_full ? X.st_w : X.st_wu) * vb + 1) + vec;
 		}
 		else if (A->plan_kind == 3) {
 			// value slots; per slice one 8-byte pointer; per offset entry (64

@@ -107,6 +107,13 @@ struct is_offdiag : std::false_type {};
 template<class E>
 struct is_offdiag<E, std::void_t<decltype(E::offdiag)>> : std::bool_constant<E::offdiag> {};
 
+// Epilogues with row_run take R consecutive rows at once (their vector loads
+// and stores are then as wide as the product's).
+template<class E, class = void>
+struct has_row_run : std::false_type {};
+template<class E>
+struct has_row_run<E, std::void_t<decltype(E::runs)>> : std::bool_constant<E::runs> {};
+
 constexpr int kSpmvThreads = 256;
 constexpr int kStreamRows = 256;   // rows per workgroup (LDS-staged mapping)
 constexpr int kStreamCap = 2048;   // nonzeros staged per workgroup
@@ -116,23 +123,50 @@ __device__ __forceinline__ T ldnt(const T * p) {
 	return __builtin_nontemporal_load(p);
 }
 
-// Element c of p through a 32-bit byte offset from the (uniform) base: one
-// address register per lane instead of two.  Valid while c * sizeof(T)
-// stays below 2^32.
-template<class T>
-__device__ __forceinline__ T ld32(const T * p, uint32_t c) {
-	return *(const T *)((const char *)p + c * (uint32_t)sizeof(T));
+// R consecutive elements in one access, aligned to the element only (vector
+// loads and stores of global memory need no more on gfx9).
+template<class T, int R>
+struct run_type {
+	typedef T type __attribute__((ext_vector_type(R), aligned(sizeof(T))));
+};
+
+// o = p[r .. r + R): p uniform.  O32: through a 32-bit byte offset, so that
+// the loads of a row at every stencil offset share one address register
+// (valid while r * sizeof(T) stays below 2^32).  NT: not read again.
+template<int R, bool O32, bool NT = false, class T>
+__device__ __forceinline__ void ld_run(const T * p, int64_t r, T (&o)[R]) {
+	const T * q;
+	if constexpr (O32) q = (const T *)((const char *)p + (uint32_t)r * (uint32_t)sizeof(T));
+	else q = p + r;
+	if constexpr (R == 1) o[0] = NT ? ldnt(q) : *q;
+	else {
+		using run = typename run_type<T, R>::type;
+		const run v = NT ? __builtin_nontemporal_load((const run *)q) : *(const run *)q;
+#pragma unroll
+		for (int j = 0; j < R; ++j) o[j] = v[j];
+	}
 }
 
-// Gather policies: the value of the multiplied vector at column c (at32:
-// the same through a 32-bit offset).
+template<int R, class T>
+__device__ __forceinline__ void st_run(T * q, const T (&o)[R]) {
+	typename run_type<T, R>::type v;
+#pragma unroll
+	for (int j = 0; j < R; ++j) v[j] = o[j];
+	*(typename run_type<T, R>::type *)q = v;
+}
+
+// Gather policies: the value of the multiplied vector at column c.
 template<class X>
 struct gather_x {
 	using value_type = X;
 	const X * x;
 	__device__ __forceinline__ void init() {}
 	__device__ __forceinline__ X operator()(int64_t c) const { return x[c]; }
-	__device__ __forceinline__ X at32(uint32_t c) const { return ld32(x, c); }
+	// R consecutive elements from off + r (off uniform)
+	template<int R, bool O32>
+	__device__ __forceinline__ void run(int64_t off, int64_t r, X (&o)[R]) const {
+		ld_run<R, O32>(x + off, r, o);
+	}
 };
 
 // Sum of the thread's row for the LDS-staged mapping.  Valid when
@@ -397,131 +431,248 @@ __global__ __launch_bounds__(BT) void spmv_sdia_kernel(
 	epi.block_end(d, blockIdx.x, gridDim.x);
 }
 
-// Symmetric stencil layout: one ascending offset list for the whole matrix,
-// passed by value, so a wave loads no per-slice pointer or offsets -- only
-// the slice's lane masks (w consecutive words, one scalar load).  Values are
-// stored for the offsets >= 0 only; the entry of row r at offset o < 0 is
-// the stored entry of row r + o at offset -o, read from that row's slot (a
-// recently streamed slice: an L2 hit, not HBM traffic).  The layout is used
-// only when the CSR values are bitwise symmetric, so each row is still
-// summed over its own entries' values in CSR order: bit-identical to the
-// serial loop.
+// Stencil layout: one ascending offset list for the whole matrix, passed by
+// value, a byte per row whose bit k tells whether the row has the entry at
+// offset k, and one array of values per stored offset, indexed by row.
+// Symmetric form (bitwise symmetric values): only the offsets >= 0 are
+// stored, and the entry of row r at offset o < 0 is read as row r + o's value
+// at -o (a recently streamed line: an L2 hit, not HBM traffic).  Full form:
+// every offset is stored.  Each row sums its own entries' values in CSR order
+// either way: bit-identical to the serial loop.
+//
+// What bounds it: the FP64 products on the layout before this one (values
+// entry-major in slices of 64 rows, a row per lane, sixteen 8-byte accesses a
+// row) kept the address and L1 path busy (89-94%), not HBM, and the FP32
+// ones its misses in flight.  A lane therefore owns R consecutive rows (two
+// of FP64, four of FP32): values and vector elements come 16 bytes at a time
+// through one address register -- an offset only moves the uniform base --
+// and the -1 / +1 neighbours inside the run are the centre's own elements, so
+// that two FP64 rows take 14 accesses instead of 32, four FP32 rows 14
+// instead of 64.
 struct stencil_desc {
 	int w;  // offsets in the list (<= kStencilMax)
-	int wu; // offsets >= 0: stored values per row
+	int wu; // stored offsets
 	int32_t off[kStencilMax];
-	int32_t ju[kStencilMax]; // value column of entry j (of its mirror for off < 0)
+	int32_t ju[kStencilMax]; // value array of entry k
+	int32_t sh[kStencilMax]; // its row there, minus the row: off[k] for a mirror
+	int64_t at[kStencilMax]; // where entry k of row r lies, minus r
+	int64_t npad;            // elements of a value array
+	int64_t lo, hi;          // the first and last offset, 0 among them
 };
 
-inline stencil_desc make_stencil_desc(const csr_index & X) {
+// The last wu offsets are stored: wu == w is the full form.
+inline stencil_desc make_stencil_desc(const csr_index & X, bool full, int64_t nrows) {
 	stencil_desc sd{};
 	sd.w = X.st_w;
-	sd.wu = X.st_wu;
+	sd.wu = full ? X.st_w : X.st_wu;
 	for (int k = 0; k < kStencilMax; ++k) {
-		sd.off[k] = X.st_off[k];
-		sd.ju[k] = X.st_ju[k];
+		const bool in = k < X.st_w, mirror = in && !full && X.st_off[k] < 0;
+		sd.off[k] = in ? X.st_off[k] : 0;
+		sd.ju[k] = !in ? 0 : full ? k : X.st_ju[k];
+		sd.sh[k] = mirror ? X.st_off[k] : 0;
 	}
+	sd.npad = (nrows + kSliceRows - 1) / kSliceRows * kSliceRows;
+	for (int k = 0; k < kStencilMax; ++k) sd.at[k] = sd.ju[k] * sd.npad + sd.sh[k];
+	sd.lo = std::min(sd.off[0], 0);
+	sd.hi = std::max(sd.off[std::max(0, sd.w - 1)], 0);
 	return sd;
 }
 
-// The slices are dealt to waves exactly as in the slice-offset kernel (same
-// grid, same grid stride), so each block's partials cover the same rows and
-// a whole solve runs bit for bit as on that layout.  Per slice, every value
-// load is issued before the gathers and every gather before the first sum
-// (scheduling barriers keep that order).  O32: value and gather addresses
-// are the array base (uniform) plus a 32-bit byte offset per lane.
-// MW: the minimum waves per SIMD the register allocation must allow (1: the
-// compiler's own choice).  With 32-bit offsets every instance fits 8
-// without spills.
-template<class Epi, class ACC, class V, class G, int BT, bool O32, int MW>
-__global__ __launch_bounds__(BT) __attribute__((amdgpu_waves_per_eu(MW))) void
-spmv_stencil_kernel(
-	int64_t nrows, stencil_desc sd, const uint64_t * __restrict__ st_mask,
-	const V * __restrict__ st_val, G x, Epi epi) {
+// Rows per lane R: 16 bytes of values on large matrices.  Small ones take one
+// row per lane: more would leave too few waves, and the waves at the ends of
+// the vector, which load element by element, would end last.  CG's FP64
+// product at one / two rows a lane: 48^3 4.4 / 4.2 us, 72^3 (373 k rows) 7.3 /
+// 5.7; the FP32 one at one / four: 48^3 3.9 / 6.4 us, 128^3 (2.1 M rows) 19 /
+// 15.6, 161^3 25.7 / 21.9.
+constexpr int64_t kStencilWideF64 = (int64_t)1 << 17;
+constexpr int64_t kStencilWideF32 = (int64_t)1 << 20;
+
+inline int stencil_run(fsx_dtype vt, int64_t nrows) {
+	if (vt == FSX_F64) return nrows >= kStencilWideF64 ? 2 : 1;
+	return nrows >= kStencilWideF32 ? 4 : 1;
+}
+
+// W > 0: a list of exactly W offsets whose middle three are -1, 0, +1; 0: any
+// list.  O32: 32-bit byte offsets per lane.
+template<class Epi, class ACC, class V, class G, int R, int W, bool SYM, bool O32>
+__global__ __launch_bounds__(kSpmvThreads) void
+spmv_stencil_kernel(int64_t nrows, stencil_desc sd, const uint8_t * __restrict__ bits,
+                    const V * __restrict__ val, G x, Epi epi) {
 	if (epi.skip()) return;
 	x.init();
 	using XV = typename G::value_type;
-	const int lane = threadIdx.x & (kSliceRows - 1);
+	constexpr int BT = kSpmvThreads;
+	constexpr int N = W ? W : kStencilMax, C = W ? W / 2 : -1;
+	const int lane = threadIdx.x & 63;
 	double d[Epi::NV];
 #pragma unroll
 	for (int i = 0; i < Epi::NV; ++i) d[i] = 0.0;
-	constexpr int kWaves = BT / kSliceRows;
-	const int64_t nslices = (nrows + kSliceRows - 1) / kSliceRows;
-	const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kSliceRows));
-	const int64_t sstride = (int64_t)gridDim.x * kWaves;
-	const int sw = sd.wu * kSliceRows; // values per slice
-	for (int64_t s = (int64_t)blockIdx.x * kWaves + wave; s < nslices; s += sstride) {
-		const int64_t r = s * kSliceRows + lane;
-		const uint64_t * mp = st_mask + s * sd.w;
-		V v[kStencilMax];
-		XV xv[kStencilMax];
-		// No load waits for the lane masks: a slot or vector element whose
-		// row lies in [0, nrows) is read whether or not the entry exists
-		// (the sum below skips absent entries), so every load of the slice
-		// issues at once.  Entry k of row r sits in the slot of row q at
-		// column ju[k]: q = r for offsets >= 0, the mirror row r + off[k]
-		// for offsets < 0 (rows before the first read their own slot).
-		// Row indices are 32-bit under O32 (nrows < 2^29 there).
-		using RI = std::conditional_t<O32, int32_t, int64_t>;
-		using RU = std::conditional_t<O32, uint32_t, uint64_t>;
-		const RI ri = (RI)r;
+	const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / 64));
+	const int64_t nruns = (nrows + 64 * R - 1) / (64 * R);
+	for (int64_t q = (int64_t)blockIdx.x * (BT / 64) + wave; q < nruns;
+	     q += (int64_t)gridDim.x * (BT / 64)) {
+		const int64_t base = q * 64 * R;
+		const int64_t r = base + R * lane;
+		V v[N][R];
+		XV xv[N][R];
+		uint32_t pr = 0;
+		if (base + sd.lo >= 0 && base + 64 * R + sd.hi <= nrows) {
+			[[maybe_unused]] V vm[1];
+			[[maybe_unused]] XV xm[1], xp[1];
+			if constexpr (R == 4) pr = *(const uint32_t *)(bits + r);
+			else if constexpr (R == 2) pr = *(const uint16_t *)(bits + r);
+			else pr = bits[r];
 #pragma unroll
-		for (int k = 0; k < kStencilMax; ++k) {
-			const RI rr = ri + (RI)sd.off[k];
-			const bool inb = (RU)rr < (RU)nrows;
-			const RI q = (sd.off[k] < 0 && inb) ? rr : ri;
-			const RU e = (RU)(q >> 6) * (RU)sw + (RU)(sd.ju[k] * kSliceRows) + (RU)(q & 63);
-			if constexpr (O32)
-				v[k] = ld32(st_val, e);
-			else
-				v[k] = st_val[e];
-		}
-		__builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-		for (int k = 0; k < kStencilMax; ++k) {
-			const RI rr = ri + (RI)sd.off[k];
-			const bool inb = (RU)rr < (RU)nrows;
-			if constexpr (O32)
-				xv[k] = x.at32(inb ? (uint32_t)rr : 0u);
-			else
-				xv[k] = x(inb ? (int64_t)rr : 0);
-		}
-		__builtin_amdgcn_sched_barrier(0);
-		bool pr[kStencilMax];
-#pragma unroll
-		for (int k = 0; k < kStencilMax; ++k) {
-			// the mask array carries kStencilMax words of padding; entries
-			// past w have offset 0 and column 0 and are never present
-			const uint64_t m = mp[k];
-			pr[k] = (k < sd.w) & (((m >> lane) & 1) != 0);
-		}
-		ACC sum = ACC(0);
-		XV xself{};
-		bool has_self = false;
-		double dgv = 0.; // diagonal value (offdiag epilogues)
-#pragma unroll
-		for (int k = 0; k < kStencilMax; ++k) {
-			const ACC t = sum + (ACC)v[k] * (ACC)xv[k];
-			const bool isd = pr[k] && sd.off[k] == 0;
-			if constexpr (is_offdiag<Epi>::value) {
-				sum = pr[k] && !isd ? t : sum;
-				dgv = isd ? (double)v[k] : dgv;
+			for (int k = 0; k < N; ++k) {
+				if constexpr (W == 0)
+					if (k >= sd.w) break;
+				const V * vp = val + sd.at[k];
+				if (W && SYM && k == C - 1) ld_run<1, O32>(vp, r, vm);
+				else ld_run<R, O32, W && !SYM>(vp, r, v[k]);
 			}
-			else
-				sum = pr[k] ? t : sum;
-			if (isd) {
-				xself = xv[k];
-				has_self = true;
+#pragma unroll
+			for (int k = 0; k < N; ++k) {
+				if constexpr (W == 0)
+					if (k >= sd.w) break;
+				if (W && k == C - 1) x.template run<1, O32>(-1, r, xm);
+				else if (W && k == C + 1) x.template run<1, O32>(R, r, xp);
+				else x.template run<R, O32>(sd.off[k], r, xv[k]);
+			}
+			if constexpr (W > 0) {
+#pragma unroll
+				for (int j = 0; j < R; ++j) {
+					xv[C - 1][j] = j ? xv[C][j - 1] : xm[0];
+					xv[C + 1][j] = j + 1 < R ? xv[C][j + 1] : xp[0];
+					// the mirror of row r's -1 entry is row r - 1's +1 entry
+					if constexpr (SYM) v[C - 1][j] = j ? v[C + 1][j - 1] : vm[0];
+				}
 			}
 		}
-		if (r < nrows) {
-			if constexpr (is_offdiag<Epi>::value)
-				epi.row_offdiag(r, sum, dgv, [&] { return has_self ? xself : x(r); });
-			else
-				epi.row(r, sum, d, [&] { return has_self ? xself : x(r); });
+		else {
+			// rows near the ends, element by element: what lies outside the
+			// vector is replaced by the row's own slot and element (rows past
+			// the end by the last row's) and never summed.  No load waits for
+			// the presence bits, so these waves end with the others.
+#pragma unroll
+			for (int j = 0; j < R; ++j) {
+				const int64_t rj = min(r + j, nrows - 1);
+				pr |= (uint32_t)bits[rj] << (8 * j);
+#pragma unroll
+				for (int k = 0; k < N; ++k) {
+					if constexpr (W == 0)
+						if (k >= sd.w) break;
+					const int64_t c = rj + sd.off[k];
+					const bool in = c >= 0 && c < nrows;
+					v[k][j] = val[sd.at[k] + rj - (in ? 0 : sd.sh[k])];
+					xv[k][j] = x(in ? c : rj);
+				}
+			}
 		}
+		ACC sum[R];
+		[[maybe_unused]] double dg[R];
+		[[maybe_unused]] bool self[R];
+		XV xs[R];
+#pragma unroll
+		for (int j = 0; j < R; ++j) {
+			sum[j] = ACC(0);
+			dg[j] = 0.;
+			self[j] = W > 0;
+			if constexpr (W > 0) xs[j] = xv[C][j];
+			else xs[j] = XV{};
+		}
+#pragma unroll
+		for (int k = 0; k < N; ++k) {
+			if constexpr (W == 0)
+				if (k >= sd.w) break;
+			const bool zero = W ? k == C : sd.off[k] == 0;
+#pragma unroll
+			for (int j = 0; j < R; ++j) {
+				const bool p = (pr >> (8 * j + k)) & 1u;
+				const ACC t = sum[j] + (ACC)v[k][j] * (ACC)xv[k][j];
+				if constexpr (is_offdiag<Epi>::value) {
+					sum[j] = p && !zero ? t : sum[j];
+					dg[j] = p && zero ? (double)v[k][j] : dg[j];
+				}
+				else
+					sum[j] = p ? t : sum[j];
+				if (W == 0 && zero) {
+					xs[j] = xv[k][j];
+					self[j] = true;
+				}
+			}
+		}
+		if (has_row_run<Epi>::value && base + 64 * R <= nrows) {
+			if constexpr (has_row_run<Epi>::value) {
+				if constexpr (W == 0) {
+#pragma unroll
+					for (int j = 0; j < R; ++j)
+						if (!self[j]) xs[j] = x(r + j);
+				}
+				epi.template row_run<R>(r, sum, d, xs);
+			}
+			continue;
+		}
+#pragma unroll
+		for (int j = 0; j < R; ++j)
+			if (r + j < nrows) {
+				auto xi = [&] { return self[j] ? xs[j] : x(r + j); };
+				if constexpr (is_offdiag<Epi>::value) epi.row_offdiag(r + j, sum[j], dg[j], xi);
+				else epi.row(r + j, sum[j], d, xi);
+			}
 	}
 	epi.block_end(d, blockIdx.x, gridDim.x);
+}
+
+// Workgroups of a stencil product: a run of 64 R rows per wave.  Reducing
+// FP32 products stride over a capped grid, which leaves fewer partials to
+// finalize (256^3: product 89 us at 8192 blocks, 93 at all 16384); the FP64
+// ones lose more to the stride (161 us at all 32768, 175 at 8192).
+constexpr unsigned kStencilMaxBlocksF32 = 8192;
+inline unsigned stencil_blocks(fsx_dtype vt, int64_t nrows, bool reduces) {
+	const int64_t rows = (int64_t)kSpmvThreads * stencil_run(vt, nrows);
+	const int64_t g = (nrows + rows - 1) / rows;
+	return (unsigned)(reduces && vt == FSX_F32 ? std::min<int64_t>(g, kStencilMaxBlocksF32) : g);
+}
+
+// Products on the stencil layout: plan 4 (symmetric, FP64 by default), and
+// the matrices planned on slice offsets that have it too.
+inline bool on_stencil(const fsx_csr * A) {
+	return A->st_vals && (A->plan_kind == 4 || (A->plan_kind == 3 && A->st_serves));
+}
+
+template<class Epi, class ACC, class V, class G>
+void stencil_launch(hipStream_t st, const fsx_csr * A, const G & x, const Epi & epi) {
+	const csr_index & X = *A->idx;
+	const stencil_desc sd = make_stencil_desc(X, A->st_full, A->nrows);
+	// 32-bit offsets while a row's byte offset in a vector (at most 8-byte
+	// elements) fits
+	const bool o32 = (uint64_t)A->nrows * 8 < ((uint64_t)1 << 32);
+	const int c = sd.w / 2;
+	const bool tri = sd.w % 2 && sd.w >= 3 && sd.off[c - 1] == -1 && sd.off[c] == 0 &&
+	                 sd.off[c + 1] == 1;
+	const unsigned g = stencil_blocks(A->vt, A->nrows, Epi::reduces);
+	auto launch = [&](auto r_c, auto w_c, auto sym_c, auto o32_c) {
+		constexpr int R = decltype(r_c)::value, W = decltype(w_c)::value;
+		constexpr bool SYM = decltype(sym_c)::value, O32 = decltype(o32_c)::value;
+		hipLaunchKernelGGL((spmv_stencil_kernel<Epi, ACC, V, G, R, W, SYM, O32>), dim3(g),
+		                   dim3(kSpmvThreads), 0, st, A->nrows, sd,
+		                   (const uint8_t *)X.st_bits->p, (const V *)A->st_vals->p, x, epi);
+	};
+	auto go = [&](auto w_c, auto sym_c, auto o32_c) {
+		constexpr int wide = sizeof(V) == 8 ? 2 : 4;
+		if (stencil_run(A->vt, A->nrows) == wide)
+			launch(std::integral_constant<int, wide>{}, w_c, sym_c, o32_c);
+		else launch(std::integral_constant<int, 1>{}, w_c, sym_c, o32_c);
+	};
+	using std::integral_constant;
+	using yes = std::true_type;
+	using no = std::false_type;
+	if (!o32) go(integral_constant<int, 0>{}, no{}, no{});
+	else if (tri && sd.w == 7 && !A->st_full) go(integral_constant<int, 7>{}, yes{}, yes{});
+	else if (tri && sd.w == 7) go(integral_constant<int, 7>{}, no{}, yes{});
+	else if (tri && sd.w == 5 && !A->st_full) go(integral_constant<int, 5>{}, yes{}, yes{});
+	else if (tri && sd.w == 5) go(integral_constant<int, 5>{}, no{}, yes{});
+	else go(integral_constant<int, 0>{}, no{}, yes{});
 }
 
 // Epilogues that leave per-block partials cap the grid (fewer partials for
@@ -572,39 +723,7 @@ void spmv_launch_gather(hipStream_t st, const fsx_csr * A, const G & x,
 	const I * ci = (const I *)A->colind();
 	const V * vv = (const V *)A->vals->p;
 	if (A->nrows == 0) return;
-	if (A->plan_kind == 4) {
-		const csr_index & X = *A->idx;
-		const stencil_desc sd = make_stencil_desc(X);
-		// 32-bit offsets when the value array and the gathered vector (at
-		// most 8-byte elements) span less than 4 GiB
-		const bool o32 = A->st_vals->bytes < ((size_t)1 << 32) &&
-		                 (uint64_t)A->ncols * 8 < ((uint64_t)1 << 32) &&
-		                 (uint64_t)A->nrows * 8 < ((uint64_t)1 << 32);
-		// Reducing products at 8 waves per SIMD (FP64 CG K1 at 256^3: 0.198
-		// against 0.215 ms), plain products at the compiler's choice (FP64
-		// y = A x: 0.196 against 0.229 ms)
-		constexpr int MW = Epi::reduces ? 8 : 1;
-		auto go = [&](auto bt_c, unsigned g) {
-			constexpr int BT = decltype(bt_c)::value;
-			if (o32)
-				hipLaunchKernelGGL((spmv_stencil_kernel<Epi, ACC, V, G, BT, true, MW>), dim3(g),
-				                   dim3(BT), 0, st, A->nrows, sd, (const uint64_t *)X.st_mask->p,
-				                   (const V *)A->st_vals->p, x, epi);
-			else
-				hipLaunchKernelGGL((spmv_stencil_kernel<Epi, ACC, V, G, BT, false, 1>), dim3(g),
-				                   dim3(BT), 0, st, A->nrows, sd, (const uint64_t *)X.st_mask->p,
-				                   (const V *)A->st_vals->p, x, epi);
-		};
-		if constexpr (!Epi::reduces)
-			go(std::integral_constant<int, kSpmvThreads>{},
-			   sdia_blocks(A->nrows, false, 0, 0));
-		else {
-			const sdia_reduce_shape sh = sdia_reduce(A->vt, A->nrows);
-			const unsigned g = sdia_blocks(A->nrows, true, sh.threads, sh.max_blocks);
-			if (sh.threads == 512) go(std::integral_constant<int, 512>{}, g);
-			else go(std::integral_constant<int, 256>{}, g);
-		}
-	}
+	if (on_stencil(A)) stencil_launch<Epi, ACC, V, G>(st, A, x, epi);
 	else if (A->plan_kind == 3) {
 		FSX_REQUIRE(!A->dg_stale, "slice-offset values lag the CSR values");
 		auto go = [&](auto bt_c, unsigned g) {
@@ -667,7 +786,8 @@ void spmv_launch_typed(hipStream_t st, const fsx_csr * A, const X * x,
 
 // Number of partials (each NV doubles) a reducing product on A leaves.
 inline unsigned spmv_blocks(const fsx_csr * A) {
-	if (A->plan_kind == 3 || A->plan_kind == 4) {
+	if (on_stencil(A)) return stencil_blocks(A->vt, A->nrows, true);
+	if (A->plan_kind == 3) {
 		const sdia_reduce_shape sh = sdia_reduce(A->vt, A->nrows);
 		return sdia_blocks(A->nrows, true, sh.threads, sh.max_blocks);
 	}

@@ -5,6 +5,7 @@ sliced, slice-offset and symmetric stencil layouts bit-identical to the
 reference's serial CSR loop (each sums every row serially in CSR order); the
 vector-per-row mapping within 1e-13 relative (tree order inside a row).
 """
+import ctypes as C
 from pathlib import Path
 
 import numpy as np
@@ -423,3 +424,96 @@ def test_set_values_refreshes_layouts(ctx):
     with pytest.raises(fsx.FsxError):   # unrelated structure
         B32 = ctx.csr(rp, ci, v1).convert(fsx.F32)
         B32.set_values_from(A)
+
+
+def box_stencil(dims, seed, symmetric, extra=0):
+    """Stencil matrix on a box (natural order, x fastest) with random values;
+    `extra`: one more offset pair, so that the list is no 3/5/7-point one."""
+    rng = np.random.default_rng(seed)
+    n = int(np.prod(dims))
+    idx = np.arange(n)
+    coord = [idx % dims[0]]
+    step = [1]
+    for d in range(1, len(dims)):
+        step.append(step[-1] * dims[d - 1])
+        coord.append(idx // step[d] % dims[d])
+    rows, cols, vals = [idx], [idx], [4.0 + rng.random(n)]
+    pairs = [(coord[d] + 1 < dims[d], step[d]) for d in range(len(dims))]
+    if extra:
+        pairs.append((idx + extra < n, extra))
+    for ok, o in pairs:
+        r = idx[ok]
+        up, lo = rng.uniform(-1, 1, r.size), rng.uniform(-1, 1, r.size)
+        rows += [r, r + o]
+        cols += [r + o, r]
+        vals += [up, up if symmetric else lo]
+    S = sp.csr_matrix((np.concatenate(vals), (np.concatenate(rows), np.concatenate(cols))), (n, n))
+    S.sort_indices()
+    return S.indptr.astype(np.int32), S.indices.astype(np.int32), S.data
+
+
+@pytest.mark.parametrize("symmetric", [True, False])
+@pytest.mark.parametrize("dims,extra", [
+    ((500,), 0),            # 3 offsets: the general list
+    ((129, 1024), 0),       # two rows a lane, a last run that is not whole
+    ((61, 53, 41), 0),      # odd lines: no run aligned past its elements
+    ((300, 7), 0),          # every run near an end
+    ((370, 360), 5),        # seven offsets that are no 7-point list
+    ((127, 101, 83), 0),    # FP32: four rows a lane
+])
+def test_stencil_runs_bit_exact(ctx, symmetric, dims, extra):
+    """Runs of consecutive rows per lane on the stencil layout, symmetric and
+    full form: products, residuals, SpMV+dot and Jacobi sweeps bit for bit the
+    serial loop's, FP64 and FP32, from vectors aligned to their elements only,
+    and with infinities and NaN in x at rows that no other row reads."""
+    rp, ci, v = box_stencil(dims, 7 + len(dims), symmetric, extra)
+    n = rp.size - 1
+    A = ctx.csr(rp, ci, v)
+    assert A.plan()[0] == (4 if symmetric else 3)
+    Ao = O.Csr(rp, ci, v)
+    x = np.random.default_rng(3).standard_normal(n)
+    b = np.random.default_rng(4).standard_normal(n)
+    ref = Ao.spmv(x)
+    bd, yd = ctx.vec(b), ctx.zeros(n)
+    xd = ctx.vec(x)
+    A.spmv(xd, yd)
+    np.testing.assert_array_equal(yd.get(), ref)
+    pw = fsx.spmv_dot(A, xd, yd)
+    assert abs(pw - O.dot(ref, x)) <= 1e-12 * np.abs(ref * x).sum()
+    # aligned to 8 bytes only
+    off = ctx.vec(np.r_[0.0, x])
+    p = C.c_void_p()
+    fsx.check(fsx.lib().fsx_vec_device_ptr(off.h, C.byref(p)))
+    h = C.c_void_p()
+    fsx.check(fsx.lib().fsx_vec_wrap(ctx.h, p.value + 8, n, fsx.F64, C.byref(h)))
+    A.residual(bd, fsx.Vector(ctx, n, fsx.F64, _handle=h), yd)
+    np.testing.assert_array_equal(yd.get(), b - ref)
+    # one weighted Jacobi sweep
+    w = ctx.vec(x)
+    fsx.check(fsx.lib().fsx_jacobi_relax(ctx.h, A.h, 0.5, 1, bd.h, w.h))
+    np.testing.assert_array_equal(w.get(), Ao.jacobi_relax(b, x, 0.5, 1))
+    # a NaN and an infinity reach exactly the rows that couple to them
+    z = x.copy()
+    z[n // 2], z[0] = np.inf, np.nan
+    A.spmv(ctx.vec(z), yd)
+    np.testing.assert_array_equal(yd.get(), Ao.spmv(z))
+    # FP32 values with FP32 and FP64 vectors: the layouts agree bit for bit
+    A32 = A.convert(fsx.F32)
+    outs = []
+    for plan in (None, 3, 0):
+        if plan is not None and A.plan()[0] >= 3:
+            A32.set_plan(plan)
+        y32, y64 = ctx.zeros(n, fsx.F32), ctx.zeros(n)
+        A32.spmv(ctx.vec(x.astype(np.float32)), y32)
+        A32.spmv(xd, y64)
+        outs.append((y32.get(), y64.get()))
+    for o in outs[1:]:
+        np.testing.assert_array_equal(o[0], outs[0][0])
+        np.testing.assert_array_equal(o[1], outs[0][1])
+    # values that lose (and regain) their symmetry
+    v2 = v.copy()
+    v2[ci > np.repeat(np.arange(n), np.diff(rp))] *= 1.5
+    for vals in (v2, v):
+        A.set_values(vals)
+        A.spmv(xd, yd)
+        np.testing.assert_array_equal(yd.get(), O.Csr(rp, ci, vals).spmv(x))
