@@ -657,8 +657,11 @@ void refresh_sliced_values(fsx_ctx * ctx, fsx_csr * A) {
 // offsets, or the stencil layout when all rows draw on one short offset list;
 // other short rows of similar length -> sliced rows (padding <= 10%,
 // addressable with the index type); other short-row matrices -> LDS-staged
-// row blocks; long rows -> LANES lanes per row with LANES the next power of
-// two of the mean row length (2..64).
+// row blocks; long rows -> LANES lanes per row with LANES the largest power of
+// two within the mean row length (2..64): fewer idle lanes than the next one
+// costs trips (us at lanes 8 / 16 / 32 / 64: mean 9.4 entries 70 / 77 / 105 /
+// 202, 13.4 33 / 34 / 44 / 84, 19.3 147 / 121 / 140 / 210, 34.1 127 / 98 /
+// 89 / 112).
 void choose_plan(fsx_ctx * ctx, fsx_csr * A, const void * host_rowptr,
                  const void * host_colind) {
 	int64_t maxr = 0;
@@ -705,7 +708,7 @@ void choose_plan(fsx_ctx * ctx, fsx_csr * A, const void * host_rowptr,
 	else {
 		A->plan_kind = 1;
 		int l = 2;
-		while (l < 64 && l < A->avg_row) l <<= 1;
+		while (l < 64 && 2 * l <= A->avg_row) l <<= 1;
 		A->plan_lanes = l;
 	}
 }

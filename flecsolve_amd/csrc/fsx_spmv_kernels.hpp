@@ -220,23 +220,53 @@ __device__ __forceinline__ ACC stream_rows(int64_t r0, int nr,
 	return sum;
 }
 
-// LANES lanes per row; returns the row sum in every lane of the group.
-template<int LANES, class ACC, class V, class I, class G>
-__device__ __forceinline__ ACC vector_row(int64_t row, int64_t nrows,
-                                          const I * __restrict__ rowptr,
-                                          const I * __restrict__ colind,
-                                          const V * __restrict__ vals,
-                                          const G & x) {
+// LANES lanes per row, NR rows row0, row0 + stride, ... per group; sum[i]: row
+// i's sum in every lane of the group.  The rows' first entries go through
+// memory together (row pointers, then columns and values, then the gathers):
+// one row alone is three dependent trips for a few bytes.  A lane's entries
+// and the tree are those of a row alone.
+template<int LANES, int NR, class ACC, class V, class I, class G>
+__device__ __forceinline__ void vector_rows(int64_t row0, int64_t stride, int64_t nrows,
+                                            const I * __restrict__ rowptr,
+                                            const I * __restrict__ colind,
+                                            const V * __restrict__ vals, const G & x,
+                                            ACC (&sum)[NR]) {
 	const int sub = threadIdx.x & (LANES - 1);
-	ACC s = ACC(0);
-	if (row < nrows) {
-		const I lo = rowptr[row], hi = rowptr[row + 1];
-		for (I e = lo + sub; e < hi; e += LANES)
-			s += (ACC)ldnt(vals + e) * (ACC)x(ldnt(colind + e));
+	I e[NR], hi[NR];
+#pragma unroll
+	for (int i = 0; i < NR; ++i) {
+		const int64_t row = row0 + i * stride;
+		e[i] = row < nrows ? rowptr[row] + sub : I(0);
+		hi[i] = row < nrows ? rowptr[row + 1] : I(0);
+		sum[i] = ACC(0);
+	}
+	for (;;) {
+		bool more = false;
+		I c[NR];
+		V v[NR];
+#pragma unroll
+		for (int i = 0; i < NR; ++i)
+			if (e[i] < hi[i]) {
+				c[i] = ldnt(colind + e[i]);
+				v[i] = ldnt(vals + e[i]);
+				more = true;
+			}
+		if (!more) break;
+		typename G::value_type xv[NR];
+#pragma unroll
+		for (int i = 0; i < NR; ++i)
+			if (e[i] < hi[i]) xv[i] = x(c[i]);
+#pragma unroll
+		for (int i = 0; i < NR; ++i)
+			if (e[i] < hi[i]) {
+				sum[i] += (ACC)v[i] * (ACC)xv[i];
+				e[i] += LANES;
+			}
 	}
 #pragma unroll
-	for (int o = LANES / 2; o > 0; o >>= 1) s += __shfl_xor(s, o, LANES);
-	return s;
+	for (int i = 0; i < NR; ++i)
+#pragma unroll
+		for (int o = LANES / 2; o > 0; o >>= 1) sum[i] += __shfl_xor(sum[i], o, LANES);
 }
 
 // ---- kernels -------------------------------------------------------------
@@ -263,6 +293,15 @@ __global__ __launch_bounds__(kSpmvThreads) void spmv_stream_kernel(
 	epi.block_end(d, blk, gridDim.x);
 }
 
+// Rows per group of lanes.  What bounds this mapping on ragged rows is the
+// rate of the gathers (3.8 cycles each and CU at 19 entries a row), then the
+// memory trips of a row: two rows at once, and lanes no more than the mean
+// row has entries (plan rule), 160 -> 120 us at 1 M rows of 3 .. 60 entries
+// (mean 19.3).  Four rows 127 us, eight 177 (registers); larger workgroups
+// walking contiguous rows, so that a CU's gathers stay in one window of x,
+// 126 us at best.
+constexpr int kVectorRows = 2;
+
 template<int LANES, class Epi, class ACC, class V, class I, class G>
 __global__ __launch_bounds__(kSpmvThreads) void spmv_vector_kernel(
 	int64_t nrows, const I * __restrict__ rowptr, const I * __restrict__ colind,
@@ -271,13 +310,19 @@ __global__ __launch_bounds__(kSpmvThreads) void spmv_vector_kernel(
 	x.init();
 	constexpr int RPB = kSpmvThreads / LANES;
 	const unsigned blk = blockIdx.x;
-	const int64_t row = (int64_t)blk * RPB + threadIdx.x / LANES;
-	ACC sum = vector_row<LANES, ACC>(row, nrows, rowptr, colind, vals, x);
+	const int64_t row0 = (int64_t)blk * RPB * kVectorRows + threadIdx.x / LANES;
+	ACC sum[kVectorRows];
+	vector_rows<LANES, kVectorRows, ACC>(row0, RPB, nrows, rowptr, colind, vals, x, sum);
 	double d[Epi::NV];
 #pragma unroll
 	for (int i = 0; i < Epi::NV; ++i) d[i] = 0.0;
-	if ((threadIdx.x & (LANES - 1)) == 0 && row < nrows)
-		epi.row(row, sum, d, [&] { return x(row); });
+	if ((threadIdx.x & (LANES - 1)) == 0) {
+#pragma unroll
+		for (int i = 0; i < kVectorRows; ++i) {
+			const int64_t row = row0 + (int64_t)i * RPB;
+			if (row < nrows) epi.row(row, sum[i], d, [&] { return x(row); });
+		}
+	}
 	epi.block_end(d, blk, gridDim.x);
 }
 
@@ -759,7 +804,7 @@ void spmv_launch_gather(hipStream_t st, const fsx_csr * A, const G & x,
 	else {
 		auto go = [&](auto lanes_c) {
 			constexpr int L = decltype(lanes_c)::value;
-			constexpr int RPB = kSpmvThreads / L;
+			constexpr int RPB = kSpmvThreads / L * kVectorRows;
 			unsigned g = (unsigned)((A->nrows + RPB - 1) / RPB);
 			hipLaunchKernelGGL((spmv_vector_kernel<L, Epi, ACC, V, I, G>), dim3(g),
 			                   dim3(kSpmvThreads), 0, st, A->nrows, rp, ci, vv, x,
@@ -794,7 +839,7 @@ inline unsigned spmv_blocks(const fsx_csr * A) {
 	if (A->plan_kind == 2) return sliced_blocks(A->nrows);
 	if (A->plan_kind == 0)
 		return (unsigned)((A->nrows + kStreamRows - 1) / kStreamRows);
-	const int rpb = kSpmvThreads / A->plan_lanes;
+	const int rpb = kSpmvThreads / A->plan_lanes * kVectorRows;
 	return (unsigned)((A->nrows + rpb - 1) / rpb);
 }
 

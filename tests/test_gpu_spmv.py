@@ -517,3 +517,22 @@ def test_stencil_runs_bit_exact(ctx, symmetric, dims, extra):
         A.set_values(vals)
         A.spmv(xd, yd)
         np.testing.assert_array_equal(yd.get(), O.Csr(rp, ci, vals).spmv(x))
+
+
+@pytest.mark.parametrize("lanes", [2, 8, 64])
+@pytest.mark.parametrize("n", [1, 7, 255, 513, 4099])
+def test_lanes_per_row_several_rows_a_group(ctx, lanes, n):
+    """Lanes-per-row mapping with two rows a group: row counts around a
+    workgroup's rows, empty rows and rows of many passes beside short ones;
+    tree sums, so 1e-13 relative to the row's terms, and SpMV+dot."""
+    rp, ci, v = ragged(n, 60 + n)
+    A = ctx.csr(rp, ci, v, ncols=n)
+    A.set_plan(1, lanes)
+    x = np.random.default_rng(5).standard_normal(n)
+    S = sp.csr_matrix((v, ci, rp), (n, n))
+    ref, mag = S @ x, abs(S) @ np.abs(x)
+    y = ctx.zeros(n)
+    A.spmv(ctx.vec(x), y)
+    assert (np.abs(y.get() - ref) <= 1e-13 * mag).all()
+    pw = fsx.spmv_dot(A, ctx.vec(x), y)
+    assert abs(pw - ref @ x) <= 1e-12 * (mag * np.abs(x)).sum()
