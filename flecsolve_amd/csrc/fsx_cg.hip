@@ -1622,21 +1622,29 @@ static void bcg_run_chunks(fsx_ctx * ctx, const bcg_bufs & B, bcg_state & st_hos
 
 // ---- fused GMRES (op::gmres::apply, solvers/gmres.hh:79-258) -------------
 //
-// Same Arnoldi sequence, modified Gram-Schmidt order, Givens rotations
-// (Bindel et al.), restart rule, back_solve and correct as the reference,
-// with the Hessenberg column, rotations and least-squares right-hand side
-// on the device.  Step k of a restart cycle:
-//   G0  v = A P b_k (right; P = D^-1 enters as a scaled gather
-//       0 + dinv[c] b_k[c], bitwise the z the reference forms) or
-//       v = P A b_k (left); partials of v.b_0
-//   F0  a one-block kernel stores h_0k
-//   then for j = 0..k:
-//   Gj  v = v - h_jk b_j; partials of v.b_{j+1} (j < k) or |v|^2 (j = k);
-//       for j > 0 each block first sums G(j-1)'s partials into h_jk itself
-//   GN  h_{k+1,k} = |v| from Gk's partials (each block); b_{k+1} = v / |v|
-//       (v if |v| = 0)
+// Same Arnoldi sequence, Givens rotations (Bindel et al.), restart rule,
+// back_solve and correct as the reference, with the Hessenberg column,
+// rotations and least-squares right-hand side on the device.  Step k of a
+// restart cycle:
+//   G0  v = A z, z = P b_k (right; formed by GN beside b_k) or v = P A b_k
+//       (left)
+//   G1  one pass over the basis: partials of s_i = b_i.v (i <= k) and of
+//       l_i = b_i.b_k (i < k)
+//   F1  a block per sum: s and row k of L
+//   G2  h from (I + L) h = s by forward substitution (every block, same
+//       order); v -= sum_i h_i b_i in order; partials of |v|^2
+//   GN  h_{k+1,k} = |v| from G2's partials (each block); b_{k+1} = v / |v|
+//       (v if |v| = 0); right Jacobi: z = 0 + D^-1 b_{k+1}
 //   GR  one thread: previous rotations on column k, the new rotation, the
 //       rhs update, |dw_{k+1}| test, iteration count, end of cycle.
+// This is modified Gram-Schmidt with its k + 1 reductions taken at once
+// (K. Swirydowicz, J. Langou, S. Ananthan, U. Yang, S. Thomas, Numer. Linear
+// Algebra Appl. 28 (2021) e2343): the reference's h_j = b_j.(v - sum_{i<j}
+// h_i b_i) equals s_j - sum_{i<j} (b_j.b_i) h_i, with L the computed inner
+// products of the basis, so the loss of orthogonality is that of the
+// one-at-a-time form.  What bounds it is the passes over the basis: 2 k + 6
+// vectors a step instead of 4 k + 6, in 6 launches instead of k + 5.
+// 104 x 100 x 96, GMRES(30): see kGmPerThread.
 // A cycle's m steps are captured in one graph; the host runs back_solve,
 // correct and the restart residual between cycles (every m iterations).
 
@@ -1645,135 +1653,185 @@ struct gm_state {
 	int iter, k, m, maxiter, done, status, iters, cycle_end;
 };
 
-struct gather_dinv {
-	using value_type = double;
-	const double * dinv;
-	const double * x;
-	__device__ __forceinline__ void init() {}
-	__device__ __forceinline__ double operator()(int64_t c) const { return 0.0 + dinv[c] * x[c]; }
-	template<int R, bool O32>
-	__device__ __forceinline__ void run(int64_t off, int64_t r, double (&o)[R]) const {
-		double di[R];
-		ld_run<R, O32>(dinv + off, r, di);
-		ld_run<R, O32>(x + off, r, o);
-#pragma unroll
-		for (int j = 0; j < R; ++j) o[j] = 0.0 + di[j] * o[j];
-	}
-};
-
 template<class ACC, class T, bool LEFTJ>
 struct epi_gm_v {
 	static constexpr int NV = 1;
-	static constexpr bool reduces = true;
+	static constexpr bool reduces = false;
 	T * v;
-	const T * b0;
 	const T * dinv;
-	double * partials;
 	const gm_state * st;
 	__device__ bool skip() const { return st->done != 0; }
 	template<class XI>
-	__device__ void row(int64_t i, ACC s, double (&d)[NV], XI &&) const {
-		const double b0i = (double)b0[i]; // load before the store
+	__device__ void row(int64_t i, ACC s, double (&)[NV], XI &&) const {
 		T vi = (T)s;
 		if constexpr (LEFTJ) vi = 0.0 + dinv[i] * vi; // P.apply(z, v)
 		v[i] = vi;
-		d[0] += (double)vi * b0i; // v.dot(basis[0])
 	}
 	static constexpr bool runs = true;
 	template<int R, class X>
-	__device__ void row_run(int64_t i, const ACC (&s)[R], double (&d)[NV], const X (&)[R]) const {
-		T o[R], b[R], di[R];
-		ld_run<R, false>(b0, i, b);
+	__device__ void row_run(int64_t i, const ACC (&s)[R], double (&)[NV], const X (&)[R]) const {
+		T o[R], di[R];
 		if constexpr (LEFTJ) ld_run<R, false>(dinv, i, di);
 #pragma unroll
 		for (int j = 0; j < R; ++j) {
 			o[j] = (T)s[j];
 			if constexpr (LEFTJ) o[j] = 0.0 + di[j] * o[j];
-			d[0] += (double)o[j] * (double)b[j];
 		}
 		st_run<R>(v + i, o);
 	}
-	__device__ void block_end(const double (&d)[NV], unsigned blk, unsigned) const {
-		store_block_partials<NV>(d, partials, blk);
-	}
+	__device__ void block_end(const double (&)[NV], unsigned, unsigned) const {}
 };
 
-// H(row, col) = sum (or its square root for the norm), column-major with
-// leading dimension ld (mdcolex of the reference)
-struct fin_gm_h {
-	const gm_state * st;
-	double * H;
-	int idx;
-	bool norm;
-	__device__ bool skip() const { return st->done != 0; }
-	__device__ void operator()(const double (&t)[1]) const {
-		H[idx] = norm ? sqrt(t[0]) : t[0];
-	}
-};
+// rows per thread of the Gram-Schmidt passes
+constexpr int kGmPerThread = 4;
+constexpr int kGmMaxDim = 101; // basis vectors at most (max_krylov_dim + 1)
+constexpr int kGmAhead = 4;    // basis vectors whose loads are in flight together
 
-// rows per thread of the Gram-Schmidt passes (fewer blocks: fewer partials
-// for every block of the next pass to sum)
-constexpr int kGmPerThread = 8;
-
-// v = v - h_jk b_j; partials of v.b_next (or |v|^2 when b_next is null)
-// into `partials`.  h_jk is *hjk (j = 0: stored by the product's finalize)
-// or, when `prev` is given, the sum of the previous pass's nprev partials,
-// which every block forms in the same order while its vector loads are in
-// flight (block 0 stores it at *hjk for the rotations): no finalize launch
-// between passes.
-__global__ __launch_bounds__(kUpdThreads) void gm_mgs_kernel(
-	size_t n, double * __restrict__ v, const double * __restrict__ bj,
-	const double * __restrict__ bnext, const double * __restrict__ prev, unsigned nprev,
-	double * hjk, double * __restrict__ partials, const gm_state * st) {
-	if (st->done) return;
-	const unsigned blk = blockIdx.x;
-	const size_t base = (size_t)blk * kUpdThreads * kGmPerThread + threadIdx.x;
-	double bv[kGmPerThread], vv[kGmPerThread], nv[kGmPerThread];
+// The thread's elements of p: element j at base + j * kUpdThreads (past the
+// end: zero, which adds nothing).
+__device__ __forceinline__ void gm_load(size_t n, size_t base, const double * __restrict__ p,
+                                        double (&o)[kGmPerThread]) {
 #pragma unroll
 	for (int j = 0; j < kGmPerThread; ++j) {
 		const size_t i = base + (size_t)j * kUpdThreads;
-		if (i < n) {
-			bv[j] = bj[i];
-			vv[j] = v[i];
-			nv[j] = bnext ? bnext[i] : 0.0;
+		o[j] = i < n ? p[i] : 0.0;
+	}
+}
+
+// G1: sum q (q <= k: b_q.v; k + 1 + q: b_q.b_k) of block blk at
+// partials[q * gridDim.x + blk]
+__global__ __launch_bounds__(kUpdThreads) void gm_dots_kernel(
+	size_t n, const double * __restrict__ v, const double * const * __restrict__ basis, int k,
+	double * __restrict__ partials, const gm_state * st) {
+	if (st->done) return;
+	__shared__ double sh[2 * kGmMaxDim][kUpdThreads / 64];
+	const size_t base = (size_t)blockIdx.x * kUpdThreads * kGmPerThread + threadIdx.x;
+	const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+	double vv[kGmPerThread], bk[kGmPerThread];
+	gm_load(n, base, v, vv);
+	gm_load(n, base, basis[k], bk);
+	for (int i0 = 0; i0 <= k; i0 += kGmAhead) {
+		double bi[kGmAhead][kGmPerThread];
+#pragma unroll
+		for (int q = 0; q < kGmAhead; ++q) gm_load(n, base, basis[min(i0 + q, k)], bi[q]);
+#pragma unroll
+		for (int q = 0; q < kGmAhead; ++q) {
+			double s = 0.0, l = 0.0;
+#pragma unroll
+			for (int j = 0; j < kGmPerThread; ++j) {
+				s += bi[q][j] * vv[j];
+				l += bi[q][j] * bk[j];
+			}
+			s = wave_sum(s);
+			l = wave_sum(l);
+			const int i = i0 + q;
+			if (lane == 0 && i <= k) {
+				sh[i][wave] = s;
+				if (i < k) sh[k + 1 + i][wave] = l;
+			}
 		}
 	}
-	double h;
-	if (prev) {
-		double t[1];
-		sum_partials<1, kUpdThreads>(prev, nprev, t);
-		h = t[0];
-		if (blk == 0 && threadIdx.x == 0) *hjk = h;
+	__syncthreads();
+	for (int q = threadIdx.x; q < 2 * k + 1; q += kUpdThreads) {
+		double t = sh[q][0];
+#pragma unroll
+		for (int w = 1; w < kUpdThreads / 64; ++w) t += sh[q][w];
+		partials[(size_t)q * gridDim.x + blockIdx.x] = t;
 	}
-	else
-		h = *hjk;
+}
+
+// F1: block q sums G1's q-th partials into s[q] or L(k, q - k - 1)
+__global__ __launch_bounds__(kUpdThreads) void gm_sums_kernel(
+	const double * __restrict__ partials, unsigned nblk, int k, double * s, double * L, int ld,
+	const gm_state * st) {
+	if (st->done) return;
+	const int q = blockIdx.x;
+	double t[1];
+	sum_partials<1, kUpdThreads>(partials + (size_t)q * nblk, nblk, t);
+	if (threadIdx.x == 0) {
+		if (q <= k) s[q] = t[0];
+		else L[k + (size_t)ld * (q - k - 1)] = t[0];
+	}
+}
+
+// G2: h, v -= sum h_i b_i, partials of |v|^2; block 0 stores h in H(0..k, k)
+__global__ __launch_bounds__(kUpdThreads) void gm_update_kernel(
+	size_t n, double * __restrict__ v, const double * const * __restrict__ basis, int k,
+	const double * __restrict__ s, const double * __restrict__ L, int ld, double * hcol,
+	double * __restrict__ partials, const gm_state * st) {
+	if (st->done) return;
+	__shared__ double h[kGmMaxDim];
+	const size_t base = (size_t)blockIdx.x * kUpdThreads * kGmPerThread + threadIdx.x;
+	double vv[kGmPerThread];
+	gm_load(n, base, v, vv);
+	if (threadIdx.x < 64) {
+		// forward substitution, unknowns lane and lane + 64
+		const int a = threadIdx.x, c = a + 64;
+		double sa = a <= k ? s[a] : 0.0, sc = c <= k ? s[c] : 0.0;
+		for (int i0 = 0; i0 <= k; i0 += 8) {
+			double la[8], lc[8];
+#pragma unroll
+			for (int q = 0; q < 8; ++q) {
+				const int i = min(i0 + q, k);
+				la[q] = a > i && a <= k ? L[a + (size_t)ld * i] : 0.0;
+				lc[q] = c > i && c <= k ? L[c + (size_t)ld * i] : 0.0;
+			}
+#pragma unroll
+			for (int q = 0; q < 8; ++q) {
+				const int i = i0 + q;
+				if (i > k) break;
+				const double hi = __shfl(i < 64 ? sa : sc, i & 63, 64);
+				if (a > i) sa -= la[q] * hi;
+				if (c > i) sc -= lc[q] * hi;
+			}
+		}
+		if (a <= k) h[a] = sa;
+		if (c <= k) h[c] = sc;
+		if (blockIdx.x == 0) {
+			if (a <= k) hcol[a] = sa;
+			if (c <= k) hcol[c] = sc;
+		}
+	}
+	__syncthreads();
+	for (int i0 = 0; i0 <= k; i0 += kGmAhead) {
+		double bi[kGmAhead][kGmPerThread];
+#pragma unroll
+		for (int q = 0; q < kGmAhead; ++q) gm_load(n, base, basis[min(i0 + q, k)], bi[q]);
+#pragma unroll
+		for (int q = 0; q < kGmAhead; ++q)
+			if (i0 + q <= k) {
+				const double hi = h[i0 + q];
+#pragma unroll
+				for (int j = 0; j < kGmPerThread; ++j)
+					vv[j] = (-hi) * bi[q][j] + vv[j]; // v.axpy(-h_ik, basis[i], v)
+			}
+	}
 	double acc = 0.0;
 #pragma unroll
 	for (int j = 0; j < kGmPerThread; ++j) {
 		const size_t i = base + (size_t)j * kUpdThreads;
 		if (i < n) {
-			const double vi = (-h) * bv[j] + vv[j]; // v.axpy(-h_jk, basis[j], v)
-			v[i] = vi;
-			acc += bnext ? vi * nv[j] : vi * vi;
+			v[i] = vv[j];
+			acc += vv[j] * vv[j];
 		}
 	}
 	double d[1] = {acc};
-	store_block_partials<1>(d, partials, blk);
+	store_block_partials<1>(d, partials, blockIdx.x);
 }
 
 // h_{k+1,k} = |v| from the last pass's nprev partials (every block, same
-// order; block 0 stores it) and b_{k+1} = v scaled by 1/|v| (gmres.hh:140-146)
+// order; block 0 stores it) and b_{k+1} = v scaled by 1/|v| (gmres.hh:140-146);
+// z (optional): the next product's z = D^-1 b_{k+1}, formed here instead of in
+// that product's gathers, which would read D^-1 as often as b_{k+1}
 __global__ __launch_bounds__(kUpdThreads) void gm_scale_kernel(
 	size_t n, const double * __restrict__ v, double * __restrict__ bnext,
+	const double * __restrict__ dinv, double * __restrict__ z,
 	const double * __restrict__ prev, unsigned nprev, double * hnorm, const gm_state * st) {
 	if (st->done) return;
 	const size_t base = (size_t)blockIdx.x * kUpdThreads * kGmPerThread + threadIdx.x;
-	double vv[kGmPerThread];
-#pragma unroll
-	for (int j = 0; j < kGmPerThread; ++j) {
-		const size_t i = base + (size_t)j * kUpdThreads;
-		if (i < n) vv[j] = v[i];
-	}
+	double vv[kGmPerThread], dv[kGmPerThread];
+	gm_load(n, base, v, vv);
+	if (z) gm_load(n, base, dinv, dv);
 	double t[1];
 	sum_partials<1, kUpdThreads>(prev, nprev, t);
 	const double vn = sqrt(t[0]);
@@ -1781,7 +1839,11 @@ __global__ __launch_bounds__(kUpdThreads) void gm_scale_kernel(
 #pragma unroll
 	for (int j = 0; j < kGmPerThread; ++j) {
 		const size_t i = base + (size_t)j * kUpdThreads;
-		if (i < n) bnext[i] = vn != 0.0 ? (1.0 / vn) * vv[j] : vv[j];
+		if (i < n) {
+			const double b = vn != 0.0 ? (1.0 / vn) * vv[j] : vv[j];
+			bnext[i] = b;
+			if (z) z[i] = 0.0 + dv[j] * b;
+		}
 	}
 }
 
@@ -1868,15 +1930,22 @@ __global__ __launch_bounds__(256) void gm_correct_kernel(size_t n, double * __re
 
 struct gm_bufs {
 	const fsx_csr * A;
-	double * v;
+	double *v, *z;
 	const double * const * basis_dev; // device array of basis pointers
 	std::vector<double *> basis;      // host copy
 	const double * dinv;
 	bool right;
 	double *H, *cs, *sn, *dw;
+	double *L, *s; // inner products of the basis (ld x ld), a step's b_i.v
 	int ld, m;
 	size_t n;
 };
+
+// Doubles of partials a cycle's steps need: G1's sums and G2's, a block each.
+static size_t gm_partials_need(size_t n, int m) {
+	const size_t per = (size_t)kUpdThreads * kGmPerThread;
+	return (2 * (size_t)m + 1) * std::max<size_t>(1, (n + per - 1) / per);
+}
 
 template<class V, class I>
 static void gm_enqueue_cycle(fsx_ctx * ctx, const gm_bufs & B, gm_state * st) {
@@ -1884,35 +1953,33 @@ static void gm_enqueue_cycle(fsx_ctx * ctx, const gm_bufs & B, gm_state * st) {
 	double * part = ctx->ws.partials;
 	const size_t per = (size_t)kUpdThreads * kGmPerThread;
 	const unsigned gu = (unsigned)((B.n + per - 1) / per);
-	// the passes' partials alternate between two buffers, so that a pass
-	// never overwrites the ones its blocks are still summing
-	double * pp[2] = {part, part + gu};
 	for (int k = 0; k < B.m; ++k) {
 		const double * bk = B.basis[k];
-		// G0: v = A P b_k / P A b_k, partials of v.b_0
+		// G0: v = A P b_k / P A b_k
 		if (B.right && B.dinv) {
-			epi_gm_v<double, double, false> e{B.v, B.basis[0], nullptr, part, st};
-			spmv_launch_gather<decltype(e), double, V, I>(s, B.A, gather_dinv{B.dinv, bk}, e);
+			epi_gm_v<double, double, false> e{B.v, nullptr, st};
+			spmv_launch_typed<decltype(e), double, V, I, double>(s, B.A, (const double *)B.z, e);
 		}
 		else if (!B.right && B.dinv) {
-			epi_gm_v<double, double, true> e{B.v, B.basis[0], B.dinv, part, st};
+			epi_gm_v<double, double, true> e{B.v, B.dinv, st};
 			spmv_launch_typed<decltype(e), double, V, I, double>(s, B.A, bk, e);
 		}
 		else {
-			epi_gm_v<double, double, false> e{B.v, B.basis[0], nullptr, part, st};
+			epi_gm_v<double, double, false> e{B.v, nullptr, st};
 			spmv_launch_typed<decltype(e), double, V, I, double>(s, B.A, bk, e);
 		}
-		// h_0k from the product's partials
-		spmv_finalize<1>(s, B.A, part, fin_gm_h{st, B.H, B.ld * k, false});
-		for (int j = 0; j <= k; ++j)
-			hipLaunchKernelGGL(gm_mgs_kernel, dim3(gu), dim3(kUpdThreads), 0, s, B.n, B.v,
-			                   (const double *)B.basis[j],
-			                   j < k ? (const double *)B.basis[j + 1] : nullptr,
-			                   j > 0 ? (const double *)pp[(j - 1) & 1] : nullptr, gu,
-			                   B.H + j + (size_t)B.ld * k, pp[j & 1], (const gm_state *)st);
+		// G1, F1, G2
+		hipLaunchKernelGGL(gm_dots_kernel, dim3(gu), dim3(kUpdThreads), 0, s, B.n,
+		                   (const double *)B.v, B.basis_dev, k, part, (const gm_state *)st);
+		hipLaunchKernelGGL(gm_sums_kernel, dim3(2 * k + 1), dim3(kUpdThreads), 0, s,
+		                   (const double *)part, gu, k, B.s, B.L, B.ld, (const gm_state *)st);
+		hipLaunchKernelGGL(gm_update_kernel, dim3(gu), dim3(kUpdThreads), 0, s, B.n, B.v,
+		                   B.basis_dev, k, (const double *)B.s, (const double *)B.L, B.ld,
+		                   B.H + (size_t)B.ld * k, part, (const gm_state *)st);
 		// GN: h_{k+1,k} = |v|; b_{k+1} = v / |v|
 		hipLaunchKernelGGL(gm_scale_kernel, dim3(gu), dim3(kUpdThreads), 0, s, B.n,
-		                   (const double *)B.v, B.basis[k + 1], (const double *)pp[k & 1], gu,
+		                   (const double *)B.v, B.basis[k + 1], B.dinv,
+		                   B.right && B.dinv ? B.z : nullptr, (const double *)part, gu,
 		                   B.H + k + 1 + (size_t)B.ld * k, (const gm_state *)st);
 		// GR
 		hipLaunchKernelGGL(gm_givens_kernel, dim3(1), dim3(64), 0, s, B.H, B.ld, B.cs, B.sn,
@@ -2578,14 +2645,16 @@ int fsx_gmres_solve(fsx_ctx * ctx, const fsx_csr * A, const fsx_vec * dinv,
 			bvec[i] = pooled(ctx, n, FSX_F64, 40 + i);
 			basis[i] = (double *)bvec[i]->ptr();
 		}
-		const size_t small = (size_t)ld * ld + 4 * (size_t)ld;
+		const size_t small = 2 * (size_t)ld * ld + 5 * (size_t)ld;
 		fsx_vec * smallv = pooled(ctx, small + (size_t)ld, FSX_F64, 39); // + basis ptrs
 		double * H = (double *)smallv->ptr();
 		double * cs = H + (size_t)ld * ld;
 		double * sn = cs + ld;
 		double * dw = sn + ld;
 		double * dy = dw + ld;
-		double ** bptr = (double **)(dy + ld);
+		double * gs = dy + ld; // a step's b_i.v
+		double * L = gs + ld;  // inner products of the basis
+		double ** bptr = (double **)(L + (size_t)ld * ld);
 		// gmres reset(): H, cos, sin, dw, dy zero
 		FSX_HIP(hipMemsetAsync(H, 0, small * sizeof(double), ctx->stream));
 		FSX_HIP(hipMemcpyAsync(bptr, basis.data(), ld * sizeof(double *),
@@ -2631,18 +2700,18 @@ int fsx_gmres_solve(fsx_ctx * ctx, const fsx_csr * A, const fsx_vec * dinv,
 			int rc = fsx_scale(ctx, 1.0 / bt, res);
 			if (rc) throw error(rc, get_error());
 			launch_copy(ctx, res, b0);
+			if (right && dinv) precond(b0, z);
 			FSX_HIP(hipMemcpyAsync(dw, &bt, sizeof(double), hipMemcpyHostToDevice, ctx->stream));
 			FSX_HIP(hipStreamSynchronize(ctx->stream)); // bt is a host local
 		};
 		start_cycle(beta);
-		gm_bufs B{A, (double *)v->ptr(), bptr, basis, dinv ? (const double *)dinv->ptr() : nullptr,
-		          right, H, cs, sn, dw, ld, max_dim, n};
+		gm_bufs B{A, (double *)v->ptr(), (double *)z->ptr(), bptr, basis, dinv ? (const double *)dinv->ptr() : nullptr,
+		          right, H, cs, sn, dw, L, gs, ld, max_dim, n};
 		auto & cache = cache_of(ctx);
 		gm_state * st = (gm_state *)cache.statebuf->p;
 		gm_state * pinned = (gm_state *)ctx->host_scalars;
 		static_assert(sizeof(gm_state) <= sizeof(cg_state) * 4, "");
-		const size_t per = (size_t)kUpdThreads * kGmPerThread;
-		ensure_partials(ctx, std::max<size_t>(spmv_partials_size(A, 1), 2 * ((n + per - 1) / per)));
+		ensure_partials(ctx, gm_partials_need(n, max_dim));
 		gm_state sh{};
 		sh.tol = tol;
 		sh.m = max_dim;
@@ -2700,7 +2769,8 @@ int fsx_gmres_solve(fsx_ctx * ctx, const fsx_csr * A, const fsx_vec * dinv,
 				hipGraphExec_t ge = nullptr;
 				if (use_graphs()) {
 					std::vector<const void *> key{(const void *)&gm_enqueue_cycle<V, I>,
-					                              (const void *)B.v, (const void *)H,
+					                              (const void *)B.v, (const void *)B.z,
+					                              (const void *)H,
 					                              (const void *)B.dinv,
 					                              (const void *)ctx->ws.partials,
 					                              (const void *)st,
@@ -2734,7 +2804,7 @@ int fsx_gmres_solve(fsx_ctx * ctx, const fsx_csr * A, const fsx_vec * dinv,
 				if (ge) FSX_HIP(hipGraphLaunch(ge, ctx->stream));
 				else gm_enqueue_cycle<V, I>(ctx, B, st);
 			});
-			ctx->launches += (size_t)max_dim * (max_dim + 9) / 2;
+			ctx->launches += (size_t)max_dim * 6;
 			FSX_HIP(hipMemcpyAsync(pinned, st, sizeof(gm_state), hipMemcpyDeviceToHost,
 			                       ctx->stream));
 			FSX_HIP(hipStreamSynchronize(ctx->stream));

@@ -9,6 +9,7 @@ gmres test (flecsolve/solvers/test/gmres.cc:88-110); settings validation
 """
 import numpy as np
 import pytest
+import scipy.sparse as sp
 
 from flecsolve_amd import fsx
 from flecsolve_amd import problems as P
@@ -84,3 +85,30 @@ def test_validation_exhaustion_zero_rhs(ctx):
                            fsx.Settings(maxiter=5, rtol=1e-8, max_krylov_dim=30,
                                         restart=True, use_zero_guess=True))
     assert info.reason == "converged_rtol" and info.iters == 0
+
+
+@pytest.mark.parametrize("dim", [1, 2, 63, 64, 65, 100])
+@pytest.mark.parametrize("n", [4, 11, 17])
+def test_basis_sizes_iteration_matched(ctx, dim, n):
+    """The Gram-Schmidt pass at basis sizes around a wave's lanes and the
+    largest, on vectors of less than a workgroup to several: cycles stopped by
+    maxiter give the oracle's iterates (sums in another order: the Hessenberg
+    column is off by rounding times the condition of the least-squares
+    problem, so x to 1e-9), an orthogonal basis on an ill-conditioned matrix."""
+    rp, ci, v = P.diffusion3d(n, P.lognormal_field(n, 2.0, 4.0, 55))
+    N = n ** 3
+    Ao = O.Csr(rp, ci, v)
+    b = P.uniform(N, 2105)
+    its = min(2 * dim, 130)
+    s = dict(maxiter=its, rtol=1e-14, use_zero_guess=True, max_krylov_dim=dim, restart=True,
+             pre_side=1)
+    xo, io, _ = O.gmres(Ao, b, np.zeros(N), O.Settings(**s), P=O.prec(1, Ao.dinv()))
+    A = ctx.csr(rp, ci, v)
+    x = ctx.zeros(N)
+    info = fsx.gmres_solve(A, ctx.vec(b), x, fsx.Settings(**s), dinv=A.diag_inv())
+    S = sp.csr_matrix((v, ci, rp))
+    ro, rg = np.linalg.norm(b - S @ xo), np.linalg.norm(b - S @ x.get())
+    assert rg <= 1.01 * ro + 1e-11 * np.linalg.norm(b)
+    if N > dim:  # the basis does not span the whole space
+        assert info.reason == io.reason and info.restarts == io.restarts
+        assert rel(x.get(), xo) <= 1e-9
