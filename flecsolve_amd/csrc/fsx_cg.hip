@@ -638,6 +638,8 @@ struct cg_work {
 	// the single-reduction iteration (unpreconditioned solves of the
 	// refinement only): K1 with w.p and w.w, one finalize, one fused update
 	bool single_reduction = false;
+	// small stencil systems in one launch (cg_resident_kernel)
+	bool resident = true;
 };
 
 // Partials a CG solve on A over n rows needs: the SpMV+dot (1 per block),
@@ -973,6 +975,433 @@ static void run_cg_loop_pipelined(fsx_ctx * ctx, const cg_bufs & B, cg_state * s
 	(void)hipEventDestroy(ev[1]);
 }
 
+// ---- resident CG: small stencil systems, all iterations in one launch -------
+//
+// On small systems an iteration is five launches (three in the
+// single-reduction form) of 2-4 us each, whatever the rows: bound by launches
+// and by each kernel's first trip to memory.  Here every row of the system
+// belongs to a thread of one launch: r, x, p, D^-1 and its
+// matrix entries stay in registers, and the iteration's two global
+// reductions are exchanges between the workgroups.
+//
+// An exchange: each workgroup stores its partial sums into its slots of a
+// buffer that held a sentinel, polls the others' slots until none holds the
+// sentinel, and sums them.  It orders memory as a barrier would: what a
+// neighbour gathers (p and z, or p) is written with device-scope stores, which
+// a wave waits for before its workgroup's partials leave, and read with
+// device-scope loads; no cache is written back or invalidated.  Three buffers
+// in turn: after exchange e everyone has read buffer e - 1, whose slots their
+// owners reset before storing for exchange e + 1.
+//
+// The products, partial sums, totals and updates are those of the launched
+// kernels, in their order (blocks of 256 rows for the product's dot, of 1024
+// for the update's): the same bits as the launched loop takes on systems that
+// use one row per lane.
+//
+// FP64, two gathers per entry: p = beta p_old + z is formed for the neighbour
+// instead of stored and exchanged once more.
+//
+// Every wait ends.  At most one workgroup per CU is launched, and one resident
+// solve at a time in a process and device (a second thread's takes the launched
+// loop), so all of them start once other streams' kernels leave the CUs; a
+// poll that lasts kResWaitTicks all the same gives up, sets the abort flag and
+// returns without storing anything, and the host runs the launched loop.
+constexpr int kResThreads = 256;
+constexpr int kResRows = 4;                    // rows per thread
+constexpr int kResMaxBlocks = 256;
+constexpr uint64_t kResWaitTicks = 100000000;  // of the 100 MHz counter: 1 s
+constexpr uint64_t kResSentinel = 0xFFF8DEADBEEF5A5Aull;
+constexpr int kResItersPerLaunch = 4096;
+static_assert(kResMaxBlocks * kResRows * 2 <= kXchSlots, "exchange slots");
+
+struct res_args {
+	int64_t n;
+	stencil_desc sd;
+	const uint8_t * bits;
+	const void * val;
+	void *x, *r, *p;     // p: also the FP64 form's gathered copy
+	void * z;            // FP64: gathered z (r without a preconditioner)
+	void * q;            // single reduction: gathered p
+	const void * dinv;
+	cg_state * st;
+	double * hist;
+	double * xch;
+	int iters;           // iterations of this launch at most
+};
+
+template<class T>
+__device__ __forceinline__ T dev_load(const T * p) {
+	return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template<class T>
+__device__ __forceinline__ void dev_store(T * p, T v) {
+	__hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// All slots the sentinel, the abort flag clear.
+__global__ void res_reset_kernel(double * xch) {
+	const int i = blockIdx.x * blockDim.x + threadIdx.x;
+	if (i < 3 * kXchSlots) ((uint64_t *)xch)[i] = kResSentinel;
+	else if (i < kXchDoubles) ((uint64_t *)xch)[i] = 0;
+}
+
+// Totals of NV sums whose partials are one per group of rows: this workgroup
+// holds GRP groups (d[g][i], per thread), `count` groups in all.  The block
+// sums are store_block_partials', the total finalize_kernel's with its 1024
+// threads.  False when a wait gave up.
+template<int NV, int GRP>
+__device__ __forceinline__ bool res_exchange(const double (&d)[GRP][NV], int count, double * xch,
+                                             int & turn, int prev_slots, double (&tot)[NV]) {
+	__shared__ double sh[GRP][NV][kResThreads / 64];
+	__shared__ double red[NV][kFinThreads / 64];
+	__shared__ int gave_up;
+	const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+	uint64_t * buf = (uint64_t *)xch + (size_t)turn * kXchSlots;
+	uint64_t * old = (uint64_t *)xch + (size_t)(turn + 2 - (turn > 0 ? 3 : 0)) * kXchSlots;
+	int * abortf = (int *)(xch + 3 * kXchSlots);
+#pragma unroll
+	for (int g = 0; g < GRP; ++g)
+#pragma unroll
+		for (int i = 0; i < NV; ++i) {
+			const double s = wave_sum(d[g][i]);
+			if (lane == 0) sh[g][i][wave] = s;
+		}
+	if (tid == 0) gave_up = 0;
+	// this wave's device-scope stores have arrived before its partials leave
+	asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+	__syncthreads();
+	if (tid < GRP * NV) {
+		const int g = tid / NV, i = tid % NV, at = (int)blockIdx.x * GRP + g;
+		double t = sh[g][i][0];
+#pragma unroll
+		for (int w = 1; w < kResThreads / 64; ++w) t += sh[g][i][w];
+		uint64_t b = (uint64_t)__double_as_longlong(t);
+		if (b == kResSentinel) b = 0x7FF8000000000000ull;
+		if (at < count) dev_store(buf + at * NV + i, b);
+	}
+	// thread t sums group t, t + 1024, ... of each 256-wide quarter m
+	constexpr int Q = kFinThreads / kResThreads;
+	constexpr int DEPTH = (kResMaxBlocks * GRP + kFinThreads - 1) / kFinThreads;
+	uint64_t v[Q][DEPTH][NV];
+	bool live = true;
+	uint64_t t0 = 0;
+	for (int spin = 0;; ++spin) {
+		bool all = true;
+#pragma unroll
+		for (int m = 0; m < Q; ++m)
+#pragma unroll
+			for (int e = 0; e < DEPTH; ++e)
+#pragma unroll
+				for (int i = 0; i < NV; ++i) {
+					const int at = m * kResThreads + tid + e * kFinThreads;
+					v[m][e][i] = at < count ? dev_load(buf + at * NV + i) : 0ull;
+				}
+#pragma unroll
+		for (int m = 0; m < Q; ++m)
+#pragma unroll
+			for (int e = 0; e < DEPTH; ++e)
+#pragma unroll
+				for (int i = 0; i < NV; ++i) all = all && v[m][e][i] != kResSentinel;
+		if (__all(all)) break;
+		if ((spin & 255) == 255) {
+			const uint64_t now = wall_clock64();
+			if (!t0) t0 = now;
+			if (now - t0 > kResWaitTicks || dev_load(abortf)) {
+				live = false;
+				break;
+			}
+		}
+	}
+	if (!live && lane == 0) {
+		gave_up = 1;
+		dev_store(abortf, 1);
+	}
+#pragma unroll
+	for (int m = 0; m < Q; ++m)
+#pragma unroll
+		for (int i = 0; i < NV; ++i) {
+			double a = 0.0;
+#pragma unroll
+			for (int e = 0; e < DEPTH; ++e) a += __longlong_as_double((long long)v[m][e][i]);
+			const double s = wave_sum(a);
+			if (lane == 0) red[i][m * (kResThreads / 64) + wave] = s;
+		}
+	__syncthreads();
+	if (gave_up) return false;
+#pragma unroll
+	for (int i = 0; i < NV; ++i) {
+		double s = 0.0;
+		for (int w = 0; w < kFinThreads / 64; ++w) s += red[i][w];
+		tot[i] = s;
+	}
+	// everyone has read the previous buffer: reset this workgroup's slots there
+	if (tid < prev_slots) dev_store(old + blockIdx.x * prev_slots + tid, kResSentinel);
+	turn = turn == 2 ? 0 : turn + 1;
+	__syncthreads(); // the shared sums are reused
+	return true;
+}
+
+// SR: the single-reduction form (FP32, no preconditioner), else the
+// reference's sequence (FP64).
+template<class T, bool SR, bool JAC, int W>
+__global__ __launch_bounds__(kResThreads) __attribute__((amdgpu_waves_per_eu(1, 1))) void
+cg_resident_kernel(res_args a) {
+	constexpr int RPT = kResRows, N = W;
+	constexpr int UPD = RPT / kUpdPerThread; // update blocks of 1024 rows
+	cg_state & st = *a.st;
+	if (st.done) return;
+	const int64_t base = (int64_t)blockIdx.x * kResThreads * RPT + threadIdx.x;
+	const int count1 = (int)((a.n + kResThreads - 1) / kResThreads);
+	const int count2 = (int)((a.n + kResThreads * kUpdPerThread - 1) / (kResThreads * kUpdPerThread));
+	const T * val = (const T *)a.val;
+	T * gq = SR ? (T *)a.q : (T *)a.p; // gathered p
+	T * gz = (T *)a.z;                 // gathered z
+	T r[RPT], x[RPT], p[RPT], w[RPT], z[RPT], dv[RPT];
+	unsigned pr[RPT];
+	T v[RPT][N];
+#pragma unroll
+	for (int j = 0; j < RPT; ++j) {
+		const int64_t row = base + j * kResThreads;
+		const bool in = row < a.n;
+		const int64_t c = in ? row : 0;
+		r[j] = in ? ((const T *)a.r)[c] : T(0);
+		x[j] = in ? ((const T *)a.x)[c] : T(0);
+		p[j] = in ? ((const T *)a.p)[c] : T(0);
+		dv[j] = JAC && in ? ((const T *)a.dinv)[c] : T(0);
+		z[j] = T(0);
+		pr[j] = in ? a.bits[c] : 0u;
+#pragma unroll
+		for (int k = 0; k < N; ++k)
+			v[j][k] = val[a.sd.at[k] + c - ((pr[j] >> k) & 1u ? 0 : a.sd.sh[k])];
+	}
+	double rho = st.rho1, rho0 = st.rho0, alpha = st.alpha, beta = 0.0, res = st.res, pw = st.pw;
+	const double tol = st.tol;
+	const int maxiter = st.maxiter;
+	int it = st.iter, ncurv = st.ncurv, done = 0, status = st.status, iters = st.iters;
+	const int last = a.iters < maxiter - it ? it + a.iters : maxiter;
+	int turn = 0, prev = 0;
+	bool first = true, ok = true;
+	if constexpr (SR) {
+		// p to where it is gathered from
+#pragma unroll
+		for (int j = 0; j < RPT; ++j) {
+			const int64_t row = base + j * kResThreads;
+			if (row < a.n) dev_store(gq + row, p[j]);
+		}
+		double none[1][1] = {{0.0}}, t[1];
+		ok = res_exchange<1, 1>(none, (int)gridDim.x, a.xch, turn, prev, t);
+		prev = 1;
+	}
+	while (ok && it < last) {
+		// w = A p, the dot products of each 256-row block
+		constexpr int NA = SR ? 2 : 1;
+		double da[RPT][NA];
+#pragma unroll
+		for (int j = 0; j < RPT; ++j) {
+			const int64_t row = base + j * kResThreads;
+			// 32-bit offsets, formed here in every iteration: kept, the addresses
+			// of all gathers would take more registers than the row's data
+			uint32_t own = row < a.n ? (uint32_t)row : 0u;
+			asm volatile("" : "+v"(own));
+			T g[N], gp[N];
+#pragma unroll
+			for (int k = 0; k < N; ++k) {
+				const bool on = (pr[j] >> k) & 1u;
+				const uint32_t c = (own + (on ? (uint32_t)a.sd.off[k] : 0u)) * (uint32_t)sizeof(T);
+				gp[k] = dev_load((const T *)((const char *)gq + c));
+				if (!SR && !first) g[k] = dev_load((const T *)((const char *)gz + c));
+			}
+			T sum = T(0);
+#pragma unroll
+			for (int k = 0; k < N; ++k) {
+				T pn = gp[k];
+				if (!SR && !first) pn = (T)(beta * (double)gp[k] + (double)g[k]);
+				const T t = sum + v[j][k] * pn;
+				sum = ((pr[j] >> k) & 1u) ? t : sum;
+			}
+			w[j] = sum;
+			da[j][0] = 0.0;
+			if constexpr (SR) da[j][1] = 0.0;
+			if (row < a.n) {
+				da[j][0] += (double)sum * (double)p[j];
+				if constexpr (SR) da[j][1] += (double)sum * (double)sum;
+			}
+		}
+		double ta[NA];
+		ok = res_exchange<NA, RPT>(da, count1, a.xch, turn, prev, ta);
+		prev = RPT * NA;
+		if (!ok) break;
+		pw = ta[0];
+		if (pw <= 0.0) ++ncurv;
+		alpha = rho / pw;
+		constexpr int NB = SR ? 1 : 2;
+		double db[UPD][NB];
+#pragma unroll
+		for (int u = 0; u < UPD; ++u)
+#pragma unroll
+			for (int i = 0; i < NB; ++i) db[u][i] = 0.0;
+		if constexpr (SR) {
+			const double rho_next = alpha * alpha * ta[1] - rho;
+			beta = rho_next / rho;
+			rho0 = rho;
+#pragma unroll
+			for (int j = 0; j < RPT; ++j) {
+				const int64_t row = base + j * kResThreads;
+				if (row < a.n) {
+					const double pi = (double)p[j];
+					const T ri = (T)((-alpha) * (double)w[j] + (double)r[j]);
+					r[j] = ri;
+					db[j / kUpdPerThread][0] += (double)ri * (double)ri;
+					x[j] = (T)(alpha * pi + (double)x[j]);
+					p[j] = (T)(beta * pi + (double)ri);
+					dev_store(gq + row, p[j]);
+				}
+			}
+		}
+		else {
+#pragma unroll
+			for (int j = 0; j < RPT; ++j) {
+				const int64_t row = base + j * kResThreads;
+				if (row < a.n) {
+					const T ri = (-alpha) * w[j] + r[j];
+					r[j] = ri;
+					db[j / kUpdPerThread][0] += ri * ri;
+					z[j] = ri;
+					if constexpr (JAC) {
+						z[j] = 0.0 + dv[j] * ri;
+						db[j / kUpdPerThread][1] += ri * z[j];
+					}
+					dev_store(gz + row, z[j]);
+					if (!first) dev_store(gq + row, p[j]);
+				}
+			}
+		}
+		double tb[NB];
+		ok = res_exchange<NB, UPD>(db, count2, a.xch, turn, prev, tb);
+		prev = UPD * NB;
+		if (!ok) break;
+		res = sqrt(tb[0]);
+		if (a.hist && blockIdx.x == 0 && threadIdx.x == 0) a.hist[it] = res;
+		++it;
+		if constexpr (!SR) {
+#pragma unroll
+			for (int j = 0; j < RPT; ++j) x[j] = alpha * p[j] + x[j];
+		}
+		if (res < tol) {
+			iters = it;
+			status = FSX_CONVERGED_RTOL;
+			done = 1;
+		}
+		else if (it >= maxiter) done = 1;
+		if constexpr (SR) rho = tb[0];
+		if (done) break;
+		if constexpr (!SR) {
+			rho0 = rho;
+			rho = JAC ? tb[1] : tb[0];
+			beta = rho / rho0;
+#pragma unroll
+			for (int j = 0; j < RPT; ++j) p[j] = beta * p[j] + z[j];
+		}
+		first = false;
+	}
+	if (!ok) return;
+#pragma unroll
+	for (int j = 0; j < RPT; ++j) {
+		const int64_t row = base + j * kResThreads;
+		if (row < a.n) {
+			((T *)a.r)[row] = r[j];
+			((T *)a.x)[row] = x[j];
+			((T *)a.p)[row] = p[j];
+		}
+	}
+	if (blockIdx.x == 0 && threadIdx.x == 0) {
+		st.rho0 = rho0;
+		st.rho1 = rho;
+		st.alpha = alpha;
+		st.beta = beta;
+		st.res = res;
+		st.pw = pw;
+		st.iter = it;
+		st.ncurv = ncurv;
+		st.done = done;
+		st.status = status;
+		st.iters = iters;
+	}
+}
+
+// Whether a system's iterations run in resident launches: the 5- and 7-point
+// stencil lists, at most kResRows rows for each thread of a workgroup per CU.
+static bool fits_resident(const fsx_csr * A, size_t n) {
+	const size_t blocks = (size_t)std::min(kResMaxBlocks, A->ctx->num_cus);
+	return n > 0 && on_stencil(A) && (A->idx->st_w == 5 || A->idx->st_w == 7) &&
+	       n <= blocks * kResThreads * kResRows;
+}
+
+static bool use_resident() {
+	static bool g = [] {
+		const char * e = getenv("FSX_CG_RESIDENT");
+		return !(e && e[0] == '0');
+	}();
+	return g;
+}
+
+template<class T, bool SR, bool JAC>
+static void launch_resident(fsx_ctx * ctx, res_args a) {
+	const int64_t per = (int64_t)kResThreads * kResRows;
+	const dim3 grid((unsigned)((a.n + per - 1) / per));
+	if (a.sd.w == 7)
+		hipLaunchKernelGGL((cg_resident_kernel<T, SR, JAC, 7>), grid, dim3(kResThreads), 0,
+		                   ctx->stream, a);
+	else
+		hipLaunchKernelGGL((cg_resident_kernel<T, SR, JAC, 5>), grid, dim3(kResThreads), 0,
+		                   ctx->stream, a);
+}
+
+// One launch of at most `iters` iterations.
+template<class T, bool SR>
+static void enqueue_resident(fsx_ctx * ctx, const cg_bufs & B, cg_state * st, double * hist,
+                             int iters) {
+	const fsx_csr * A = B.A;
+	res_args a{};
+	a.n = (int64_t)B.n;
+	a.sd = make_stencil_desc(*A->idx, A->st_full, A->nrows);
+	a.bits = (const uint8_t *)A->idx->st_bits->p;
+	a.val = A->st_vals->p;
+	a.x = B.x;
+	a.r = B.r;
+	a.p = B.p;
+	a.z = B.z;
+	a.q = B.w;
+	a.dinv = B.dinv;
+	a.st = st;
+	a.hist = hist;
+	a.xch = ctx->ws.xch;
+	a.iters = iters;
+	hipLaunchKernelGGL(res_reset_kernel, dim3((kXchDoubles + 255) / 256), dim3(256), 0,
+	                   ctx->stream, ctx->ws.xch);
+	if constexpr (SR) launch_resident<T, true, false>(ctx, a);
+	else if (B.dinv) launch_resident<T, false, true>(ctx, a);
+	else launch_resident<T, false, false>(ctx, a);
+	FSX_HIP(hipGetLastError());
+	ctx->launches += 2;
+}
+
+// The resident solve of a device, held from its launch to the read of its
+// state; one that is not free is not waited for.
+constexpr int kResMaxDevices = 64;
+static std::mutex g_resident_mu[kResMaxDevices];
+
+// Reads the state after a resident launch; false when the launch gave up.
+static bool read_resident(fsx_ctx * ctx, const cg_state * st, cg_state * pinned) {
+	int * abortf = (int *)(ctx->host_scalars + kScalarSlots - 1);
+	FSX_HIP(hipMemcpyAsync(pinned, st, sizeof(cg_state), hipMemcpyDeviceToHost, ctx->stream));
+	FSX_HIP(hipMemcpyAsync(abortf, ctx->ws.xch + 3 * kXchSlots, sizeof(int),
+	                       hipMemcpyDeviceToHost, ctx->stream));
+	FSX_HIP(hipStreamSynchronize(ctx->stream));
+	ctx->host_syncs++;
+	return *abortf == 0;
+}
+
 // Iteration loop with a user diagnostic (cg.hh:112-116): one iteration at a
 // time, the host reading |r| after each and calling diag(x, |r|) before the
 // tolerance test takes effect -- a true return stops the solve with
@@ -1012,10 +1441,34 @@ static void run_cg_loop_diag(fsx_ctx * ctx, const cg_bufs & B, cg_state * st,
 	*pinned = *flag;
 }
 
+// The iteration loop in resident launches: all iterations in one (or one at a
+// time, the host calling the diagnostic after each).  False when a launch gave
+// up waiting: its vectors are not updated (FP64: r, z and p are overwritten).
+template<class T, bool SR>
+static bool run_cg_loop_resident(fsx_ctx * ctx, const cg_bufs & B, cg_state * st,
+                                 cg_state * pinned, double * hist, fsx_vec * xv,
+                                 fsx_diag_fn fn, void * user) {
+	const int maxit = pinned->maxiter;
+	while (!pinned->done && pinned->iter < maxit) {
+		enqueue_resident<T, SR>(ctx, B, st, hist, fn ? 1 : kResItersPerLaunch);
+		if (!read_resident(ctx, st, pinned)) return false;
+		if (!fn) continue;
+		const int d = fn(user, xv, pinned->res);
+		if (d < 0) throw error(FSX_ERR_STATE, "cg: the user diagnostic reported an error");
+		if (d > 0) {
+			pinned->iters = pinned->iter;
+			pinned->status = FSX_CONVERGED_USER;
+			pinned->done = 1;
+		}
+	}
+	return true;
+}
+
 // Runs the iteration loop on the device.  `st_host` holds the initial state
-// and receives the final one; *x2_out receives |x|^2 of the final x.
+// and receives the final one; *x2_out receives |x|^2 of the final x.  False
+// when a resident launch gave up and the solve has to be set up again.
 template<class T, class V, class I>
-static void run_cg_loop(fsx_ctx * ctx, const cg_bufs & B, const cg_work & wk,
+static bool run_cg_loop(fsx_ctx * ctx, const cg_bufs & B, const cg_work & wk,
                         cg_state & st_host, fsx_vec * xv, double * x2_out,
                         fsx_diag_fn diag, void * user) {
 	cg_state * st = wk.st;
@@ -1024,6 +1477,36 @@ static void run_cg_loop(fsx_ctx * ctx, const cg_bufs & B, const cg_work & wk,
 	std::memcpy(pinned, &st_host, sizeof(cg_state));
 	FSX_HIP(hipMemcpyAsync(st, pinned, sizeof(cg_state), hipMemcpyHostToDevice,
 	                       ctx->stream));
+	bool ran = false;
+	if constexpr (std::is_same_v<T, V>) {
+		constexpr bool SR = std::is_same_v<T, float>;
+		std::unique_lock<std::mutex> mine;
+		if (wk.resident && use_resident() && SR == (B.part2 != nullptr) &&
+		    fits_resident(B.A, B.n) && ctx->device < kResMaxDevices)
+			mine = std::unique_lock<std::mutex>(g_resident_mu[ctx->device], std::try_to_lock);
+		if (mine.owns_lock()) {
+			ran = run_cg_loop_resident<T, SR>(ctx, B, st, pinned, wk.hist, xv, diag, user);
+			if (!ran) {
+				if (!SR) return false;
+				std::memcpy(pinned, &st_host, sizeof(cg_state));
+				FSX_HIP(hipMemcpyAsync(st, pinned, sizeof(cg_state), hipMemcpyHostToDevice,
+				                       ctx->stream));
+			}
+		}
+	}
+	if (ran) {
+		st_host = *pinned;
+		if (x2_out) *x2_out = 0.0;
+		if (xv && B.n > 0 && x2_out) {
+			double * x2slot = wk.slots + 4;
+			reduce_raw(ctx, RED_L2SQ, xv->dt, B.n, xv->ptr(), nullptr, x2slot, wk.part);
+			FSX_HIP(hipMemcpyAsync(ctx->host_scalars + kCgHostSlot + 4, x2slot, sizeof(double),
+			                       hipMemcpyDeviceToHost, ctx->stream));
+			FSX_HIP(hipStreamSynchronize(ctx->stream));
+			*x2_out = ctx->host_scalars[kCgHostSlot + 4];
+		}
+		return true;
+	}
 	if (diag) run_cg_loop_diag<T, V, I>(ctx, B, st, pinned, wk.hist, xv, diag, user);
 	else if (wk.graphs && B.part2)
 		run_cg_loop_pipelined<T, V, I, true>(ctx, B, st, pinned, wk.hist, st_host);
@@ -1052,6 +1535,7 @@ static void run_cg_loop(fsx_ctx * ctx, const cg_bufs & B, const cg_work & wk,
 	FSX_HIP(hipStreamSynchronize(ctx->stream));
 	std::memcpy(&st_host, pinned, sizeof(cg_state));
 	if (x2_out) *x2_out = (xv && B.n > 0) ? ctx->host_scalars[kCgHostSlot + 4] : 0.0;
+	return true;
 }
 
 // r = b - A x (op::core::residual, operators/core.hh:129-142: apply, then
@@ -1178,11 +1662,18 @@ static void cg_solve_impl(fsx_ctx * ctx, const fsx_csr * A, const fsx_vec * dinv
 		const bool sr = wk.single_reduction && !dinv && !diag;
 		cg_bufs B{A, x->ptr(), r, zz, wk.p, wk.w, dinv ? dinv->ptr() : nullptr, wk.part,
 		          sr ? wk.part + spmv_partials_size(A, 2) : nullptr, n};
+		bool ran = true;
 		by_matrix_type(A, [&](auto * vtag, auto * itag) {
 			using V = std::remove_pointer_t<decltype(vtag)>;
 			using I = std::remove_pointer_t<decltype(itag)>;
-			run_cg_loop<T, V, I>(ctx, B, wk, st, x, &xf2, diag, user);
+			ran = run_cg_loop<T, V, I>(ctx, B, wk, st, x, &xf2, diag, user);
 		});
+		if (!ran) { // from the guess again, in launches
+			cg_work again = wk;
+			again.resident = false;
+			cg_solve_impl<T>(ctx, A, dinv, b, x, s, info, again, hist_count, diag, user);
+			return;
+		}
 		current_res = st.res;
 		info->iters = st.iters;
 		if (st.iters) info->status = st.status;

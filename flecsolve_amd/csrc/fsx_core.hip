@@ -465,10 +465,11 @@ int fsx_ctx_create(int device, fsx_ctx ** out) {
 		FSX_HIP(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
 		// the no-allocation CG's scratch address on this device
 		noalloc_init(device);
-		size_t ws_bytes = sizeof(double) * kScalarSlots;
+		size_t ws_bytes = sizeof(double) * (kScalarSlots + kXchDoubles);
 		c->ws_buf = std::make_unique<dbuf>(ws_bytes);
 		char * base = (char *)c->ws_buf->p;
 		c->ws.scalars = (double *)base;
+		c->ws.xch = c->ws.scalars + kScalarSlots;
 		ensure_partials(c.get(), (size_t)kRedBlocks * 4);
 		FSX_HIP(hipMemsetAsync(base, 0, ws_bytes, c->stream));
 		FSX_HIP(hipHostMalloc((void **)&c->host_scalars,

@@ -409,3 +409,68 @@ def test_cg_user_diagnostic(ctx):
     x5 = ctx.zeros(n * n)
     i5 = fsx.cg_solve(A, ctx.vec(b), x5, fsx.Settings(**s), dinv=d)
     assert i5.as_dict() == i1.as_dict()
+
+
+@pytest.mark.parametrize("dims", [(3, 5, 4), (32, 32), (33, 31), (181, 180), (512, 512), (513, 512),
+                                  (64, 64, 64), (65, 64, 64)])
+def test_resident_solves_iteration_matched(ctx, dims):
+    """Small stencil systems run all iterations in one launch, a thread per
+    four rows: row counts below, at and past a workgroup's 1024, and at and
+    past the largest system (262144 rows); 25 iterations with Jacobi and
+    without, from a nonzero guess, against the oracle's trajectory."""
+    S = None
+    for m in dims:
+        L = sp.diags([2.0 * np.ones(m), -np.ones(m - 1), -np.ones(m - 1)], [0, 1, -1])
+        S = L if S is None else sp.kron(sp.eye(m), S) + sp.kron(L, sp.eye(S.shape[0]))
+    S = sp.csr_matrix(S)
+    n = S.shape[0]
+    # a varying diagonal, so that Jacobi differs from the identity
+    S = sp.csr_matrix(S + sp.diags(P.uniform(n, 71, 0.0, 2.0)))
+    S.sort_indices()
+    rp, ci, v = S.indptr.astype(np.int32), S.indices.astype(np.int32), S.data
+    Ao = O.Csr(rp, ci, v)
+    A = ctx.csr(rp, ci, v)
+    assert A.plan() == (4, 0) or n < 1000
+    b, x0 = P.uniform(n, 72), P.uniform(n, 73)
+    s = dict(maxiter=25, rtol=1e-15)
+    for jac in (True, False):
+        xo, io, ho = O.cg(Ao, b, x0, O.Settings(**s), P=O.prec(1, Ao.dinv()) if jac else None,
+                          hist_cap=25)
+        xd = ctx.vec(x0)
+        info = fsx.cg_solve(A, ctx.vec(b), xd, fsx.Settings(**s),
+                            dinv=A.diag_inv() if jac else None)
+        assert info.reason == io.reason
+        np.testing.assert_allclose(fsx.cg_history(ctx), ho, rtol=1e-9)
+        assert rel(xd.get(), xo) <= 1e-12
+
+
+def test_solves_from_two_threads(ctx):
+    """Two threads, each on a context of its own, solve small systems at once:
+    one resident solve runs at a time and the other thread's takes the
+    launched loop, with the same bits."""
+    import threading
+    n = 48
+    rp, ci, v = P.poisson2d(n)
+    b = P.uniform(n * n, 81)
+    s = dict(maxiter=2000, rtol=1e-10, use_zero_guess=True)
+
+    def solve(c, out, reps):
+        A = c.csr(rp, ci, v)
+        d, bd, x = A.diag_inv(), c.vec(b), c.zeros(n * n)
+        for _ in range(reps):
+            i = fsx.cg_solve(A, bd, x, fsx.Settings(**s), dinv=d)
+            out.append((i.iters, x.get()))
+
+    want, got = [], [[], []]
+    solve(ctx, want, 1)
+    ctxs = [fsx.Context(0), fsx.Context(0)]
+    th = [threading.Thread(target=solve, args=(ctxs[k], got[k], 15)) for k in range(2)]
+    for t in th:
+        t.start()
+    for t in th:
+        t.join()
+    for out in got:
+        assert len(out) == 15
+        for it, x in out:
+            assert it == want[0][0]
+            np.testing.assert_array_equal(x, want[0][1])
