@@ -34,29 +34,14 @@
 //    reference's loop.  Measured on the 256^3 7-point matrix this moves the
 //    kernel from ~64% (best LDS-staged CSR variant) to ~70% of HBM peak.
 //
-//  * Symmetric stencil (structurally and bitwise symmetric matrices whose
-//    rows all draw on one list of at most 8 column offsets: the 3-D 7-point
-//    and 2-D 5-point stencils): the offsets travel as kernel arguments, each
-//    64-row slice keeps one lane mask per offset, and values are stored only
-//    for the offsets >= 0 (the diagonal and the entries above it); the entry
-//    of row r at a negative offset o is read from row r + o's stored entry at
-//    -o.  FP64 at 256^3: y = A x 0.227 -> 0.198 ms and the CG K1 0.232 ->
-//    0.200 ms against the slice-offset layout; the FP32 CG K1 measured
-//    0.123-0.184 ms against 0.119-0.124 there across launch shapes, so FP32
-//    matrices stay on slice offsets.  Measured and not kept: mirroring only
-//    the offsets that are whole slices (-256, -65536; the -1 entry stored,
-//    so no mirror load straddles lanes): FP32 0.159 ms, FP64 0.206 ms;
-//    non-temporal loads for the last use of a value (mirror reads, the
-//    diagonal): FP32 0.157 ms, FP64 K1 0.214 ms; XCD-major block order:
-//    FP64 0.202 / 0.209 ms; other shapes for the FP64 K1 (256- or
-//    1024-thread blocks one slice per wave, 256 or 512 threads striding over
-//    2-4 slices): 0.196-0.207 ms against 0.196 ms, steady state, for a plain
-//    product of 0.192 ms; x at -1 and +1 and the -1 mirror value taken from
-//    the neighbouring lanes (DPP wave shifts, one uniform load per slice
-//    edge; three of the fourteen loads a row issues): product 0.197 ->
-//    0.229 ms and CG K1 0.200 -> 0.513 ms (the reducing instance at 8 waves
-//    per SIMD).  Rows keep their CSR order: bit-identical to the serial
-//    loop.
+//  * Stencil (matrices whose rows all draw on one list of at most 8 column
+//    offsets): offsets as kernel arguments, one value array per stored offset,
+//    a lane owning a run of rows; described at spmv_stencil_kernel.  Measured
+//    on the layout before it (values entry-major in slices, a row per lane)
+//    and not kept: mirroring only the offsets that are whole slices (FP32
+//    0.159 ms, FP64 0.206); non-temporal loads for the last use of a mirrored
+//    value (0.157, 0.214); XCD-major block order (FP64 0.202 / 0.209); the
+//    +-1 neighbours from other lanes by DPP wave shifts (FP64 0.229 / 0.513).
 //
 // Workgroups are dealt to XCDs round-robin by block id.  Measured: keeping
 // that default order is faster than remapping blocks to give each XCD a
