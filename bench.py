@@ -300,13 +300,17 @@ def bench_diffusion(a, fsx, P):
               2: "spmv_sliced_kernel (sliced rows)",
               3: "spmv_sdia_kernel (slice-offset layout)",
               4: "spmv_stencil_kernel (symmetric stencil layout)"}
+    # an FP32 matrix of plan 3 is on the symmetric stencil layout when its
+    # layout holds fewer value bytes than the matrix has entries
+    plan32, plan64 = A32.plan()[0], A64.plan()[0]
+    if plan32 == 3 and k1_bytes - 8 * N < 4 * nnz:
+        plan32 = 4
     bases = {3: "compulsory bytes of the slice-offset layout (values, offsets, lane masks, "
                 "slice pointers; input read once, output written once)",
              4: "compulsory bytes of the symmetric stencil layout (values at offsets >= 0 and "
-                "lane masks; entries below the diagonal re-read from stored values, counted "
+                "a byte per row; entries below the diagonal re-read from stored values, counted "
                 "once; input read once, output written once)"}
     csr_basis = "CSR bytes (values, int32 columns, row pointers; input read once, output written once)"
-    plan32, plan64 = A32.plan()[0], A64.plan()[0]
     kname, basis = knames[plan32], bases.get(plan32, csr_basis)
     roofline = {
         "bound": "hbm",

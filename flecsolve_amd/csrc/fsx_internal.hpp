@@ -99,7 +99,7 @@ struct dbuf {
 // scalars.
 constexpr int kRedBlocks = 2048;   // maximum blocks of a reduction grid
 constexpr int kScalarSlots = 64;   // device scalar slots per context
-constexpr int kStencilMax = 8;     // offsets of the symmetric stencil layout
+constexpr int kStencilMax = 8;     // offsets of the stencil layout
 // Exchange slots of the resident CG (three buffers and an abort flag).
 constexpr int kXchSlots = 4096;
 constexpr int kXchDoubles = 3 * kXchSlots + 8;
