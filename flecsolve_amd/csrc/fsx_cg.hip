@@ -47,6 +47,7 @@ struct cg_state {
 	double rho0, rho1, alpha, beta, res, tol, pw;
 	int iter, done, status, iters, maxiter, ncurv;
 	int xpend; // the last iteration's x += alpha p is still to be applied
+	int base;  // iterations done before the launched loop took over
 };
 
 // ---- K1: w = A p and the partials of w.p; F1: alpha ----------------------
@@ -303,20 +304,22 @@ struct epi_cg_spmv2 {
 	}
 };
 
-// F1s: rho_k = |r_k|^2 (the previous fused pass's partials; the setup's rho
-// at k = 0) with r_k's tolerance test and maxiter, then alpha_k and beta_k.
+// F1s: rho_k = |r_k|^2 (the previous fused pass's partials; the state's rho,
+// already tested, at the loop's first iteration) with r_k's tolerance test and
+// maxiter, then alpha_k and beta_k.
 __global__ __launch_bounds__(kFinThreads) void sr_finalize_kernel(
 	const double * part1, unsigned nblk1, const double * part2, unsigned nblk2,
 	cg_state * st, double * hist) {
 	if (st->done) return;
 	const int it = st->iter; // completed updates
+	const bool tested = it == st->base;
 	double t[2];
 	sum_partials<2>(part1, nblk1, t);
 	double u[1] = {0.0};
-	if (it > 0) sum_partials<1>(part2, nblk2, u);
+	if (!tested) sum_partials<1>(part2, nblk2, u);
 	if (threadIdx.x != 0) return;
-	const double rho = it > 0 ? u[0] : st->rho1;
-	if (it > 0) {
+	const double rho = tested ? st->rho1 : u[0];
+	if (!tested) {
 		const double res = sqrt(rho);
 		st->res = res;
 		if (hist) hist[it - 1] = res;
@@ -605,6 +608,7 @@ struct cg_bufs {
 	void * x;
 	void * r;
 	void * z; // == r for identity
+	void * zpub; // FP64: where the resident form publishes z (never r)
 	void * p;
 	void * w;
 	const void * dinv;
@@ -628,6 +632,7 @@ static_assert(sizeof(cg_state) * 3 <= sizeof(double) * kCgHostSlot,
 // into its static scratch array.
 struct cg_work {
 	void *r, *z, *p, *w; // z: null without a preconditioner
+	void * zpub;         // FP64 systems the resident form takes: z or its stand-in
 	double * part;       // partials: at least cg_partials_need(A, n) doubles
 	double * slots;      // 5 device scalars (setup reductions, final |x|^2)
 	cg_state * st;       // device iteration state
@@ -638,8 +643,6 @@ struct cg_work {
 	// the single-reduction iteration (unpreconditioned solves of the
 	// refinement only): K1 with w.p and w.w, one finalize, one fused update
 	bool single_reduction = false;
-	// small stencil systems in one launch (cg_resident_kernel)
-	bool resident = true;
 };
 
 // Partials a CG solve on A over n rows needs: the SpMV+dot (1 per block),
@@ -801,6 +804,19 @@ static fsx_vec * pooled(fsx_ctx * ctx, size_t n, fsx_dtype dt, int slot) {
 	return v;
 }
 
+// The resident CG's launch shape: at most one workgroup per CU.
+constexpr int kResThreads = 256;
+constexpr int kResRows = 4; // rows per thread
+constexpr int kResMaxBlocks = 256;
+
+// Whether a system's iterations run in resident launches: the 5- and 7-point
+// stencil lists, at most kResRows rows for each thread of a workgroup per CU.
+static bool fits_resident(const fsx_csr * A, size_t n) {
+	const size_t blocks = (size_t)std::min(kResMaxBlocks, A->ctx->num_cus);
+	return n > 0 && on_stencil(A) && (A->idx->st_w == 5 || A->idx->st_w == 7) &&
+	       n <= blocks * kResThreads * kResRows;
+}
+
 // Work of an allocating CG solve: pooled context vectors in slots slot0 ..
 // slot0 + 3 (r, z, p, w), the context's partials grown to what the solve
 // needs, the cache's state buffer and a history buffer for maxiter entries.
@@ -809,6 +825,7 @@ static cg_work pooled_work(fsx_ctx * ctx, const fsx_csr * A, size_t n, fsx_dtype
 	cg_work wk{};
 	wk.r = pooled(ctx, n, dt, slot0 + 0)->ptr();
 	wk.z = jac ? pooled(ctx, n, dt, slot0 + 1)->ptr() : nullptr;
+	wk.zpub = dt == FSX_F64 && fits_resident(A, n) ? pooled(ctx, n, dt, slot0 + 1)->ptr() : nullptr;
 	wk.p = pooled(ctx, n, dt, slot0 + 2)->ptr();
 	wk.w = pooled(ctx, n, dt, slot0 + 3)->ptr();
 	wk.single_reduction = sr && !jac;
@@ -830,7 +847,7 @@ static void run_cg_loop_direct(fsx_ctx * ctx, const cg_bufs & B, cg_state * st,
 	const int K = chunk_size();
 	const long maxit = pinned->maxiter;
 	cg_state * flag = pinned + 1;
-	long launched_it = 0;
+	long launched_it = pinned->iter;
 	while (launched_it < maxit) {
 		const int len = (int)std::min<long>(K, maxit - launched_it);
 		for (int k = 0; k < len; ++k) enqueue_iteration<T, V, I>(ctx, B, st, hist, k);
@@ -934,7 +951,7 @@ static void run_cg_loop_pipelined(fsx_ctx * ctx, const cg_bufs & B, cg_state * s
 	};
 	const long maxit = st0.maxiter;
 	const double res0 = st0.res, tol = st0.tol;
-	long launched_it = 0; // iterations launched
+	long launched_it = st0.iter; // iterations launched
 	long want = -1;       // iterations predicted beyond those launched (-1: unknown)
 	int launched = 0, checked = 0;
 	try {
@@ -956,8 +973,8 @@ static void run_cg_loop_pipelined(fsx_ctx * ctx, const cg_bufs & B, cg_state * s
 			if (f.done) break;
 			// remaining iterations at the mean contraction per iteration so far
 			want = -1;
-			if (f.iter > 0 && f.res > 0 && res0 > 0 && tol > 0) {
-				const double rate = std::pow(f.res / res0, 1.0 / f.iter);
+			if (f.iter > st0.iter && f.res > 0 && res0 > 0 && tol > 0) {
+				const double rate = std::pow(f.res / res0, 1.0 / (f.iter - st0.iter));
 				if (rate > 0 && rate < 1) {
 					const double m = std::ceil(std::log(tol / f.res) / std::log(rate));
 					if (m < 1e9) want = std::max<long>(0, (long)m - (launched_it - f.iter));
@@ -1007,15 +1024,21 @@ static void run_cg_loop_pipelined(fsx_ctx * ctx, const cg_bufs & B, cg_state * s
 //
 // Every wait ends.  At most one workgroup per CU is launched, and one resident
 // solve at a time in a process and device (a second thread's takes the launched
-// loop), so all of them start once other streams' kernels leave the CUs; a
-// poll that lasts kResWaitTicks all the same gives up, sets the abort flag and
-// returns without storing anything, and the host runs the launched loop.
-constexpr int kResThreads = 256;
-constexpr int kResRows = 4;                    // rows per thread
-constexpr int kResMaxBlocks = 256;
+// loop), so all of them start once other streams' and processes' kernels leave
+// the CUs; a poll that lasts kResWaitTicks all the same gives up.
+//
+// A launch ends as a whole: one word says whether it gave up or finished, and
+// the first workgroup to reach either end decides it.  Whoever has passed the
+// last exchange claims the word before it stores r, x, p or the state; whoever
+// has waited too long claims it before it leaves, and goes on polling when the
+// other has been first (the last partials have then all been seen by someone,
+// so they are there for it too).  The vectors others gather from during the
+// launch are w and zpub.  A launch that gave up therefore leaves r, x, p and the
+// state as the launch before left them, and the launched loop goes on from
+// there.
 constexpr uint64_t kResWaitTicks = 100000000;  // of the 100 MHz counter: 1 s
 constexpr uint64_t kResSentinel = 0xFFF8DEADBEEF5A5Aull;
-constexpr int kResItersPerLaunch = 4096;
+enum res_verdict { RES_RUNNING = 0, RES_GAVE_UP, RES_FINISHED };
 static_assert(kResMaxBlocks * kResRows * 2 <= kXchSlots, "exchange slots");
 
 struct res_args {
@@ -1023,9 +1046,9 @@ struct res_args {
 	stencil_desc sd;
 	const uint8_t * bits;
 	const void * val;
-	void *x, *r, *p;     // p: also the FP64 form's gathered copy
-	void * z;            // FP64: gathered z (r without a preconditioner)
-	void * q;            // single reduction: gathered p
+	void *x, *r, *p;
+	void * z;            // FP64: gathered z (without a preconditioner r's copy)
+	void * q;            // gathered p (FP64: after the first iteration)
 	const void * dinv;
 	cg_state * st;
 	double * hist;
@@ -1042,11 +1065,21 @@ __device__ __forceinline__ void dev_store(T * p, T v) {
 	__hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// All slots the sentinel, the abort flag clear.
-__global__ void res_reset_kernel(double * xch) {
+// All slots the sentinel; the verdict open (or already that it gave up).
+__global__ void res_reset_kernel(double * xch, int verdict) {
 	const int i = blockIdx.x * blockDim.x + threadIdx.x;
 	if (i < 3 * kXchSlots) ((uint64_t *)xch)[i] = kResSentinel;
 	else if (i < kXchDoubles) ((uint64_t *)xch)[i] = 0;
+	if (i == 3 * kXchSlots) *(int *)(xch + i) = verdict;
+}
+
+// The launch's verdict, `mine` if none was reached before.
+__device__ __forceinline__ int res_claim(double * xch, int mine) {
+	int * word = (int *)(xch + 3 * kXchSlots);
+	int was = RES_RUNNING;
+	__hip_atomic_compare_exchange_strong(word, &was, mine, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+	                                     __HIP_MEMORY_SCOPE_AGENT);
+	return was == RES_RUNNING ? mine : was;
 }
 
 // Totals of NV sums whose partials are one per group of rows: this workgroup
@@ -1062,7 +1095,6 @@ __device__ __forceinline__ bool res_exchange(const double (&d)[GRP][NV], int cou
 	const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
 	uint64_t * buf = (uint64_t *)xch + (size_t)turn * kXchSlots;
 	uint64_t * old = (uint64_t *)xch + (size_t)(turn + 2 - (turn > 0 ? 3 : 0)) * kXchSlots;
-	int * abortf = (int *)(xch + 3 * kXchSlots);
 #pragma unroll
 	for (int g = 0; g < GRP; ++g)
 #pragma unroll
@@ -1110,16 +1142,16 @@ __device__ __forceinline__ bool res_exchange(const double (&d)[GRP][NV], int cou
 		if ((spin & 255) == 255) {
 			const uint64_t now = wall_clock64();
 			if (!t0) t0 = now;
-			if (now - t0 > kResWaitTicks || dev_load(abortf)) {
+			int verdict = dev_load((const int *)(xch + 3 * kXchSlots));
+			if (verdict == RES_RUNNING && now - t0 > kResWaitTicks)
+				verdict = res_claim(xch, RES_GAVE_UP);
+			if (__any(verdict == RES_GAVE_UP)) {
 				live = false;
 				break;
 			}
 		}
 	}
-	if (!live && lane == 0) {
-		gave_up = 1;
-		dev_store(abortf, 1);
-	}
+	if (!live && lane == 0) gave_up = 1;
 #pragma unroll
 	for (int m = 0; m < Q; ++m)
 #pragma unroll
@@ -1158,8 +1190,8 @@ cg_resident_kernel(res_args a) {
 	const int count1 = (int)((a.n + kResThreads - 1) / kResThreads);
 	const int count2 = (int)((a.n + kResThreads * kUpdPerThread - 1) / (kResThreads * kUpdPerThread));
 	const T * val = (const T *)a.val;
-	T * gq = SR ? (T *)a.q : (T *)a.p; // gathered p
-	T * gz = (T *)a.z;                 // gathered z
+	T * gq = (T *)a.q; // gathered p
+	T * gz = (T *)a.z; // gathered z
 	T r[RPT], x[RPT], p[RPT], w[RPT], z[RPT], dv[RPT];
 	unsigned pr[RPT];
 	T v[RPT][N];
@@ -1207,12 +1239,13 @@ cg_resident_kernel(res_args a) {
 			// of all gathers would take more registers than the row's data
 			uint32_t own = row < a.n ? (uint32_t)row : 0u;
 			asm volatile("" : "+v"(own));
+			const T * gsrc = !SR && first ? (const T *)a.p : gq;
 			T g[N], gp[N];
 #pragma unroll
 			for (int k = 0; k < N; ++k) {
 				const bool on = (pr[j] >> k) & 1u;
 				const uint32_t c = (own + (on ? (uint32_t)a.sd.off[k] : 0u)) * (uint32_t)sizeof(T);
-				gp[k] = dev_load((const T *)((const char *)gq + c));
+				gp[k] = dev_load((const T *)((const char *)gsrc + c));
 				if (!SR && !first) g[k] = dev_load((const T *)((const char *)gz + c));
 			}
 			T sum = T(0);
@@ -1276,7 +1309,7 @@ cg_resident_kernel(res_args a) {
 						db[j / kUpdPerThread][1] += ri * z[j];
 					}
 					dev_store(gz + row, z[j]);
-					if (!first) dev_store(gq + row, p[j]);
+					dev_store(gq + row, p[j]);
 				}
 			}
 		}
@@ -1309,6 +1342,10 @@ cg_resident_kernel(res_args a) {
 		first = false;
 	}
 	if (!ok) return;
+	__shared__ int verdict;
+	if (threadIdx.x == 0) verdict = res_claim(a.xch, RES_FINISHED);
+	__syncthreads();
+	if (verdict != RES_FINISHED) return;
 #pragma unroll
 	for (int j = 0; j < RPT; ++j) {
 		const int64_t row = base + j * kResThreads;
@@ -1333,22 +1370,6 @@ cg_resident_kernel(res_args a) {
 	}
 }
 
-// Whether a system's iterations run in resident launches: the 5- and 7-point
-// stencil lists, at most kResRows rows for each thread of a workgroup per CU.
-static bool fits_resident(const fsx_csr * A, size_t n) {
-	const size_t blocks = (size_t)std::min(kResMaxBlocks, A->ctx->num_cus);
-	return n > 0 && on_stencil(A) && (A->idx->st_w == 5 || A->idx->st_w == 7) &&
-	       n <= blocks * kResThreads * kResRows;
-}
-
-static bool use_resident() {
-	static bool g = [] {
-		const char * e = getenv("FSX_CG_RESIDENT");
-		return !(e && e[0] == '0');
-	}();
-	return g;
-}
-
 template<class T, bool SR, bool JAC>
 static void launch_resident(fsx_ctx * ctx, res_args a) {
 	const int64_t per = (int64_t)kResThreads * kResRows;
@@ -1365,6 +1386,7 @@ static void launch_resident(fsx_ctx * ctx, res_args a) {
 template<class T, bool SR>
 static void enqueue_resident(fsx_ctx * ctx, const cg_bufs & B, cg_state * st, double * hist,
                              int iters) {
+	const bool give_up = ++ctx->res_launches == (uint64_t)ctx->res_give_up;
 	const fsx_csr * A = B.A;
 	res_args a{};
 	a.n = (int64_t)B.n;
@@ -1374,7 +1396,7 @@ static void enqueue_resident(fsx_ctx * ctx, const cg_bufs & B, cg_state * st, do
 	a.x = B.x;
 	a.r = B.r;
 	a.p = B.p;
-	a.z = B.z;
+	a.z = B.zpub;
 	a.q = B.w;
 	a.dinv = B.dinv;
 	a.st = st;
@@ -1382,7 +1404,7 @@ static void enqueue_resident(fsx_ctx * ctx, const cg_bufs & B, cg_state * st, do
 	a.xch = ctx->ws.xch;
 	a.iters = iters;
 	hipLaunchKernelGGL(res_reset_kernel, dim3((kXchDoubles + 255) / 256), dim3(256), 0,
-	                   ctx->stream, ctx->ws.xch);
+	                   ctx->stream, ctx->ws.xch, (int)(give_up ? RES_GAVE_UP : RES_RUNNING));
 	if constexpr (SR) launch_resident<T, true, false>(ctx, a);
 	else if (B.dinv) launch_resident<T, false, true>(ctx, a);
 	else launch_resident<T, false, false>(ctx, a);
@@ -1397,13 +1419,13 @@ static std::mutex g_resident_mu[kResMaxDevices];
 
 // Reads the state after a resident launch; false when the launch gave up.
 static bool read_resident(fsx_ctx * ctx, const cg_state * st, cg_state * pinned) {
-	int * abortf = (int *)(ctx->host_scalars + kScalarSlots - 1);
+	int * verdict = (int *)(ctx->host_scalars + kScalarSlots - 1);
 	FSX_HIP(hipMemcpyAsync(pinned, st, sizeof(cg_state), hipMemcpyDeviceToHost, ctx->stream));
-	FSX_HIP(hipMemcpyAsync(abortf, ctx->ws.xch + 3 * kXchSlots, sizeof(int),
+	FSX_HIP(hipMemcpyAsync(verdict, ctx->ws.xch + 3 * kXchSlots, sizeof(int),
 	                       hipMemcpyDeviceToHost, ctx->stream));
 	FSX_HIP(hipStreamSynchronize(ctx->stream));
 	ctx->host_syncs++;
-	return *abortf == 0;
+	return *verdict != RES_GAVE_UP;
 }
 
 // Iteration loop with a user diagnostic (cg.hh:112-116): one iteration at a
@@ -1419,7 +1441,7 @@ static void run_cg_loop_diag(fsx_ctx * ctx, const cg_bufs & B, cg_state * st,
 	const int maxit = pinned->maxiter;
 	const unsigned g3 = (unsigned)((B.n + 255) / 256);
 	*flag = *pinned;
-	for (int it = 0; it < maxit; ++it) {
+	for (int it = pinned->iter; it < maxit; ++it) {
 		enqueue_iteration<T, V, I, true>(ctx, B, st, hist, it);
 		ctx->launches += 5;
 		FSX_HIP(hipMemcpyAsync(flag, st, sizeof(cg_state), hipMemcpyDeviceToHost,
@@ -1446,16 +1468,16 @@ static void run_cg_loop_diag(fsx_ctx * ctx, const cg_bufs & B, cg_state * st,
 }
 
 // The iteration loop in resident launches: all iterations in one (or one at a
-// time, the host calling the diagnostic after each).  False when a launch gave
-// up waiting: its vectors are not updated (FP64: r, z and p are overwritten).
+// time, the host calling the diagnostic after each).  When a launch gives up,
+// *pinned and the vectors are where the launch before left them.
 template<class T, bool SR>
-static bool run_cg_loop_resident(fsx_ctx * ctx, const cg_bufs & B, cg_state * st,
+static void run_cg_loop_resident(fsx_ctx * ctx, const cg_bufs & B, cg_state * st,
                                  cg_state * pinned, double * hist, fsx_vec * xv,
                                  fsx_diag_fn fn, void * user) {
 	const int maxit = pinned->maxiter;
 	while (!pinned->done && pinned->iter < maxit) {
-		enqueue_resident<T, SR>(ctx, B, st, hist, fn ? 1 : kResItersPerLaunch);
-		if (!read_resident(ctx, st, pinned)) return false;
+		enqueue_resident<T, SR>(ctx, B, st, hist, fn ? 1 : ctx->res_iters);
+		if (!read_resident(ctx, st, pinned)) return;
 		if (!fn) continue;
 		const int d = fn(user, xv, pinned->res);
 		if (d < 0) throw error(FSX_ERR_STATE, "cg: the user diagnostic reported an error");
@@ -1465,14 +1487,12 @@ static bool run_cg_loop_resident(fsx_ctx * ctx, const cg_bufs & B, cg_state * st
 			pinned->done = 1;
 		}
 	}
-	return true;
 }
 
 // Runs the iteration loop on the device.  `st_host` holds the initial state
-// and receives the final one; *x2_out receives |x|^2 of the final x.  False
-// when a resident launch gave up and the solve has to be set up again.
+// and receives the final one; *x2_out receives |x|^2 of the final x.
 template<class T, class V, class I>
-static bool run_cg_loop(fsx_ctx * ctx, const cg_bufs & B, const cg_work & wk,
+static void run_cg_loop(fsx_ctx * ctx, const cg_bufs & B, const cg_work & wk,
                         cg_state & st_host, fsx_vec * xv, double * x2_out,
                         fsx_diag_fn diag, void * user) {
 	cg_state * st = wk.st;
@@ -1481,24 +1501,16 @@ static bool run_cg_loop(fsx_ctx * ctx, const cg_bufs & B, const cg_work & wk,
 	std::memcpy(pinned, &st_host, sizeof(cg_state));
 	FSX_HIP(hipMemcpyAsync(st, pinned, sizeof(cg_state), hipMemcpyHostToDevice,
 	                       ctx->stream));
-	bool ran = false;
 	if constexpr (std::is_same_v<T, V>) {
 		constexpr bool SR = std::is_same_v<T, float>;
 		std::unique_lock<std::mutex> mine;
-		if (wk.resident && use_resident() && SR == (B.part2 != nullptr) &&
-		    fits_resident(B.A, B.n) && ctx->device < kResMaxDevices)
+		if (ctx->res_on && SR == (B.part2 != nullptr) && fits_resident(B.A, B.n) &&
+		    ctx->device < kResMaxDevices)
 			mine = std::unique_lock<std::mutex>(g_resident_mu[ctx->device], std::try_to_lock);
-		if (mine.owns_lock()) {
-			ran = run_cg_loop_resident<T, SR>(ctx, B, st, pinned, wk.hist, xv, diag, user);
-			if (!ran) {
-				if (!SR) return false;
-				std::memcpy(pinned, &st_host, sizeof(cg_state));
-				FSX_HIP(hipMemcpyAsync(st, pinned, sizeof(cg_state), hipMemcpyHostToDevice,
-				                       ctx->stream));
-			}
-		}
+		if (mine.owns_lock())
+			run_cg_loop_resident<T, SR>(ctx, B, st, pinned, wk.hist, xv, diag, user);
 	}
-	if (ran) {
+	if (pinned->done || pinned->iter >= pinned->maxiter) { // resident to the end
 		st_host = *pinned;
 		if (x2_out) *x2_out = 0.0;
 		if (xv && B.n > 0 && x2_out) {
@@ -1509,7 +1521,13 @@ static bool run_cg_loop(fsx_ctx * ctx, const cg_bufs & B, const cg_work & wk,
 			FSX_HIP(hipStreamSynchronize(ctx->stream));
 			*x2_out = ctx->host_scalars[kCgHostSlot + 4];
 		}
-		return true;
+		return;
+	}
+	if (pinned->iter > st_host.iter) { // the launched loop goes on where a launch gave up
+		pinned->base = pinned->iter;
+		st_host = *pinned;
+		FSX_HIP(hipMemcpyAsync(st, pinned, sizeof(cg_state), hipMemcpyHostToDevice,
+		                       ctx->stream));
 	}
 	if (diag) run_cg_loop_diag<T, V, I>(ctx, B, st, pinned, wk.hist, xv, diag, user);
 	else if (wk.graphs && B.part2)
@@ -1539,7 +1557,6 @@ static bool run_cg_loop(fsx_ctx * ctx, const cg_bufs & B, const cg_work & wk,
 	FSX_HIP(hipStreamSynchronize(ctx->stream));
 	std::memcpy(&st_host, pinned, sizeof(cg_state));
 	if (x2_out) *x2_out = (xv && B.n > 0) ? ctx->host_scalars[kCgHostSlot + 4] : 0.0;
-	return true;
 }
 
 // r = b - A x (op::core::residual, operators/core.hh:129-142: apply, then
@@ -1664,20 +1681,13 @@ static void cg_solve_impl(fsx_ctx * ctx, const fsx_csr * A, const fsx_vec * dinv
 	double xf2 = 0;
 	if (s.maxiter > 0) {
 		const bool sr = wk.single_reduction && !dinv && !diag;
-		cg_bufs B{A, x->ptr(), r, zz, wk.p, wk.w, dinv ? dinv->ptr() : nullptr, wk.part,
+		cg_bufs B{A, x->ptr(), r, zz, wk.zpub, wk.p, wk.w, dinv ? dinv->ptr() : nullptr, wk.part,
 		          sr ? wk.part + spmv_partials_size(A, 2) : nullptr, n};
-		bool ran = true;
 		by_matrix_type(A, [&](auto * vtag, auto * itag) {
 			using V = std::remove_pointer_t<decltype(vtag)>;
 			using I = std::remove_pointer_t<decltype(itag)>;
-			ran = run_cg_loop<T, V, I>(ctx, B, wk, st, x, &xf2, diag, user);
+			run_cg_loop<T, V, I>(ctx, B, wk, st, x, &xf2, diag, user);
 		});
-		if (!ran) { // from the guess again, in launches
-			cg_work again = wk;
-			again.resident = false;
-			cg_solve_impl<T>(ctx, A, dinv, b, x, s, info, again, hist_count, diag, user);
-			return;
-		}
 		current_res = st.res;
 		info->iters = st.iters;
 		if (st.iters) info->status = st.status;
@@ -2691,6 +2701,7 @@ int fsx_cg_solve_noalloc(fsx_ctx * ctx, const fsx_csr * A, const fsx_vec * dinv,
 		wk.part = (double *)(base + kNoallocPartOff);
 		wk.r = vec;
 		wk.z = dinv ? vec + kNoallocVecBytes : nullptr;
+		wk.zpub = vec + kNoallocVecBytes;
 		wk.p = vec + 2 * kNoallocVecBytes;
 		wk.w = vec + 3 * kNoallocVecBytes;
 		wk.hist = nullptr;
@@ -2933,7 +2944,7 @@ int fsx_ir_cg_rr_solve(fsx_ctx * ctx, const fsx_csr * A64, const fsx_csr * A32,
 		else {
 			const double c = rnorm;
 			double rho = replace(true, c);
-			cg_bufs B{A32, y->ptr(), iwk.r, iwk.r, iwk.p, iwk.w, nullptr, iwk.part,
+			cg_bufs B{A32, y->ptr(), iwk.r, iwk.r, nullptr, iwk.p, iwk.w, nullptr, iwk.part,
 			          iwk.part + spmv_partials_size(A32, 2), n};
 			for (;;) {
 				if (seg >= max_segments) {

@@ -461,6 +461,10 @@ int fsx_ctx_create(int device, fsx_ctx ** out) {
 		hipDeviceProp_t prop;
 		FSX_HIP(hipGetDeviceProperties(&prop, device));
 		c->num_cus = prop.multiProcessorCount;
+		if (const char * e = getenv("FSX_CG_RESIDENT")) c->res_on = e[0] != '0';
+		if (const char * e = getenv("FSX_CG_RESIDENT_ITERS"))
+			c->res_iters = std::max(1, atoi(e));
+		if (const char * e = getenv("FSX_CG_RESIDENT_GIVE_UP")) c->res_give_up = atoi(e);
 		// default-priority, non-blocking stream
 		FSX_HIP(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
 		// the no-allocation CG's scratch address on this device

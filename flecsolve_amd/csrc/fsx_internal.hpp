@@ -100,7 +100,7 @@ struct dbuf {
 constexpr int kRedBlocks = 2048;   // maximum blocks of a reduction grid
 constexpr int kScalarSlots = 64;   // device scalar slots per context
 constexpr int kStencilMax = 8;     // offsets of the stencil layout
-// Exchange slots of the resident CG (three buffers and an abort flag).
+// Exchange slots of the resident CG (three buffers and its verdict).
 constexpr int kXchSlots = 4096;
 constexpr int kXchDoubles = 3 * kXchSlots + 8;
 
@@ -136,6 +136,12 @@ struct fsx_ctx {
 	uint64_t next_id = 1;
 	std::vector<double> last_cg_hist;
 	std::unique_ptr<cg_graph_cache, cg_cache_deleter> cg_cache;
+	// resident CG (environment switches, read when the context is created):
+	// whether small systems take it, iterations of a launch at most, and the
+	// launch (1, 2, ...) that gives up although it could finish (0: none)
+	bool res_on = true;
+	int res_iters = 4096, res_give_up = 0;
+	uint64_t res_launches = 0;
 	~fsx_ctx();
 };
 

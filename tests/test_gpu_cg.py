@@ -474,3 +474,61 @@ def test_solves_from_two_threads(ctx):
         for it, x in out:
             assert it == want[0][0]
             np.testing.assert_array_equal(x, want[0][1])
+
+
+def context_with(monkeypatch, **env):
+    """A context created under environment switches (read at creation)."""
+    for k, v in env.items():
+        monkeypatch.setenv(k, str(v))
+    c = fsx.Context(0)
+    for k in env:
+        monkeypatch.delenv(k)
+    return c
+
+
+@pytest.mark.parametrize("how", ["jacobi", "identity", "noalloc", "diag", "rr"])
+@pytest.mark.parametrize("give_up", [1, 2, 4])
+def test_resident_give_up_continues(ctx, monkeypatch, how, give_up):
+    """A resident launch that gives up, at a solve's first launch or after
+    launches that already advanced it: the launched loop goes on from where
+    the last good launch ended, so iterates, iteration counts, history and the
+    diagnostic's calls are those of a solve that never was resident, bit for
+    bit (one row per lane on both sides)."""
+    n = 24
+    rp, ci, v, _ = diffusion(n)
+    N = n ** 3
+    b, x0 = P.uniform(N, 91), P.uniform(N, 92)
+
+    def solve(c):
+        A = c.csr(rp, ci, v)
+        bd, x, seen = c.vec(b), c.vec(x0), []
+        s = fsx.Settings(maxiter=500, rtol=1e-9)
+        if how == "rr":
+            A32 = A.convert(fsx.F32)
+            A32.set_values_sym_scaled(A)
+            i = fsx.ir_cg_rr_solve(A, A32, bd, x, 1e-10, fsx.Settings(maxiter=500, rtol=1e-3))
+            return x.get(), (i.status, i.outer_iters, i.inner_iters_total), seen, []
+        d = A.diag_inv() if how != "identity" else None
+        if how == "diag":
+            def diag(xv, res):
+                seen.append((res, xv.get().tobytes()))
+                return False
+            i = fsx.cg_solve_diag(A, bd, x, s, diag, dinv=d)
+        else:
+            i = (fsx.cg_solve_noalloc if how == "noalloc" else fsx.cg_solve)(A, bd, x, s, dinv=d)
+        h = [] if how == "noalloc" else fsx.cg_history(c)
+        return x.get(), i.as_dict(), seen, list(h)
+
+    want = solve(context_with(monkeypatch, FSX_CG_RESIDENT=0))
+    got = solve(context_with(monkeypatch, FSX_CG_RESIDENT_ITERS=7,
+                             FSX_CG_RESIDENT_GIVE_UP=give_up))
+    np.testing.assert_array_equal(got[0], want[0])
+    assert got[1:] == want[1:]
+    # past the last iteration: the launch before the end gives up, or none
+    if how == "jacobi" and give_up == 1:
+        last = (want[1]["iters"] + 6) // 7
+        for k in (last, last + 1):
+            got = solve(context_with(monkeypatch, FSX_CG_RESIDENT_ITERS=7,
+                                     FSX_CG_RESIDENT_GIVE_UP=k))
+            np.testing.assert_array_equal(got[0], want[0])
+            assert got[1:] == want[1:]
