@@ -1469,7 +1469,10 @@ static void run_cg_loop_diag(fsx_ctx * ctx, const cg_bufs & B, cg_state * st,
 
 // The iteration loop in resident launches: all iterations in one (or one at a
 // time, the host calling the diagnostic after each).  When a launch gives up,
-// *pinned and the vectors are where the launch before left them.
+// *pinned and the vectors are where the launch before left them, and the context
+// takes the launched loop from then on: what kept the workgroups from running at
+// once (another process's kernels, a mask on the CUs) tends to last, and every
+// segment of a refinement would wait for it again.
 template<class T, bool SR>
 static void run_cg_loop_resident(fsx_ctx * ctx, const cg_bufs & B, cg_state * st,
                                  cg_state * pinned, double * hist, fsx_vec * xv,
@@ -1477,7 +1480,10 @@ static void run_cg_loop_resident(fsx_ctx * ctx, const cg_bufs & B, cg_state * st
 	const int maxit = pinned->maxiter;
 	while (!pinned->done && pinned->iter < maxit) {
 		enqueue_resident<T, SR>(ctx, B, st, hist, fn ? 1 : ctx->res_iters);
-		if (!read_resident(ctx, st, pinned)) return;
+		if (!read_resident(ctx, st, pinned)) {
+			ctx->res_on = false;
+			return;
+		}
 		if (!fn) continue;
 		const int d = fn(user, xv, pinned->res);
 		if (d < 0) throw error(FSX_ERR_STATE, "cg: the user diagnostic reported an error");

@@ -137,8 +137,9 @@ struct fsx_ctx {
 	std::vector<double> last_cg_hist;
 	std::unique_ptr<cg_graph_cache, cg_cache_deleter> cg_cache;
 	// resident CG (environment switches, read when the context is created):
-	// whether small systems take it, iterations of a launch at most, and the
-	// launch (1, 2, ...) that gives up although it could finish (0: none)
+	// whether small systems take it (until a launch gives up), iterations of a
+	// launch at most, and the launch (1, 2, ...) that gives up although it could
+	// finish (0: none)
 	bool res_on = true;
 	int res_iters = 4096, res_give_up = 0;
 	uint64_t res_launches = 0;

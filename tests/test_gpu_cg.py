@@ -532,3 +532,37 @@ def test_resident_give_up_continues(ctx, monkeypatch, how, give_up):
                                      FSX_CG_RESIDENT_GIVE_UP=k))
             np.testing.assert_array_equal(got[0], want[0])
             assert got[1:] == want[1:]
+
+
+def test_resident_give_up_is_remembered(ctx, monkeypatch):
+    """After a give-up a context's solves take the launched loop (five launches
+    an iteration) at once, segments of a refinement included."""
+    n = 20
+    rp, ci, v, _ = diffusion(n)
+    b = P.uniform(n ** 3, 93)
+
+    def launches(c, refine=False):
+        A = c.csr(rp, ci, v)
+        d, bd, x = A.diag_inv(), c.vec(b), c.zeros(n ** 3)
+        A32 = A.convert(fsx.F32)
+        A32.set_values_sym_scaled(A)
+        before = c.counters()[1]
+        if refine:
+            i = fsx.ir_cg_rr_solve(A, A32, bd, x, 1e-10, fsx.Settings(maxiter=500, rtol=1e-2))
+            its = i.inner_iters_total
+        else:
+            its = fsx.cg_solve(A, bd, x, fsx.Settings(maxiter=500, rtol=1e-9), dinv=d).iters
+        return c.counters()[1] - before, its
+
+    # resident: a reset and a launch beside the setup's few
+    k, its = launches(context_with(monkeypatch, FSX_CG_RESIDENT_GIVE_UP=0))
+    assert its > 40 and k < 20
+    c = context_with(monkeypatch, FSX_CG_RESIDENT_GIVE_UP=1)
+    never = context_with(monkeypatch, FSX_CG_RESIDENT=0)
+    extra = 2
+    for refine in (False, False, True):
+        k, its = launches(c, refine)
+        k0, its0 = launches(never, refine)
+        assert its == its0 and k0 >= (3 if refine else 5) * its0
+        assert k == k0 + extra  # the reset and launch that gave up
+        extra = 0
