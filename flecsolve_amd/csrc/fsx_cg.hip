@@ -1012,8 +1012,10 @@ static void run_cg_loop_pipelined(fsx_ctx * ctx, const cg_bufs & B, cg_state * s
 //
 // The products, partial sums, totals and updates are those of the launched
 // kernels, in their order (blocks of 256 rows for the product's dot, of 1024
-// for the update's): the same bits as the launched loop takes on systems that
-// use one row per lane.
+// for the update's): the same bits, so that they do not depend on which of the
+// two a solve takes.  Where the launched FP64 product has two rows per lane
+// (PAIRS: from kStencilWideF64 rows), a thread's dot is over rows 2 t and 2 t + 1
+// of each 512, brought to it through shared memory.
 //
 // Bound by the exchanges, about 4.5 us each (partials acknowledged, seen by the
 // others, polled and summed).  98 x 98, FP64: 5.51 -> 3.29 ms a solve (9.5 us an
@@ -1040,6 +1042,8 @@ constexpr uint64_t kResWaitTicks = 100000000;  // of the 100 MHz counter: 1 s
 constexpr uint64_t kResSentinel = 0xFFF8DEADBEEF5A5Aull;
 enum res_verdict { RES_RUNNING = 0, RES_GAVE_UP, RES_FINISHED };
 static_assert(kResMaxBlocks * kResRows * 2 <= kXchSlots, "exchange slots");
+static_assert((int64_t)kResMaxBlocks * kResRows * kResThreads <= kStencilWideF32,
+              "the resident FP32 products' rows per lane");
 
 struct res_args {
 	int64_t n;
@@ -1179,15 +1183,18 @@ __device__ __forceinline__ bool res_exchange(const double (&d)[GRP][NV], int cou
 
 // SR: the single-reduction form (FP32, no preconditioner), else the
 // reference's sequence (FP64).
-template<class T, bool SR, bool JAC, int W>
+template<class T, bool SR, bool JAC, bool PAIRS, int W>
 __global__ __launch_bounds__(kResThreads) __attribute__((amdgpu_waves_per_eu(1, 1))) void
 cg_resident_kernel(res_args a) {
+	static_assert(!(SR && PAIRS), "FP32 products of these sizes have one row per lane");
 	constexpr int RPT = kResRows, N = W;
+	constexpr int DOTS = PAIRS ? RPT / 2 : RPT; // blocks of the product's dot
 	constexpr int UPD = RPT / kUpdPerThread; // update blocks of 1024 rows
 	cg_state & st = *a.st;
 	if (st.done) return;
 	const int64_t base = (int64_t)blockIdx.x * kResThreads * RPT + threadIdx.x;
-	const int count1 = (int)((a.n + kResThreads - 1) / kResThreads);
+	constexpr int kDotRows = kResThreads * (PAIRS ? 2 : 1);
+	const int count1 = (int)((a.n + kDotRows - 1) / kDotRows);
 	const int count2 = (int)((a.n + kResThreads * kUpdPerThread - 1) / (kResThreads * kUpdPerThread));
 	const T * val = (const T *)a.val;
 	T * gq = (T *)a.q; // gathered p
@@ -1229,9 +1236,10 @@ cg_resident_kernel(res_args a) {
 		prev = 1;
 	}
 	while (ok && it < last) {
-		// w = A p, the dot products of each 256-row block
+		// w = A p, the dot products of each 256-row (PAIRS: 512-row) block
 		constexpr int NA = SR ? 2 : 1;
-		double da[RPT][NA];
+		double da[DOTS][NA];
+		__shared__ double rows[PAIRS ? RPT * kResThreads : 1];
 #pragma unroll
 		for (int j = 0; j < RPT; ++j) {
 			const int64_t row = base + j * kResThreads;
@@ -1257,16 +1265,29 @@ cg_resident_kernel(res_args a) {
 				sum = ((pr[j] >> k) & 1u) ? t : sum;
 			}
 			w[j] = sum;
-			da[j][0] = 0.0;
-			if constexpr (SR) da[j][1] = 0.0;
-			if (row < a.n) {
-				da[j][0] += (double)sum * (double)p[j];
-				if constexpr (SR) da[j][1] += (double)sum * (double)sum;
+			if constexpr (PAIRS)
+				rows[j * kResThreads + threadIdx.x] = row < a.n ? sum * p[j] : 0.0;
+			else {
+				da[j][0] = 0.0;
+				if constexpr (SR) da[j][1] = 0.0;
+				if (row < a.n) {
+					da[j][0] += (double)sum * (double)p[j];
+					if constexpr (SR) da[j][1] += (double)sum * (double)sum;
+				}
+			}
+		}
+		if constexpr (PAIRS) {
+			__syncthreads();
+#pragma unroll
+			for (int g = 0; g < DOTS; ++g) {
+				const double * q = rows + 2 * (g * kResThreads + (int)threadIdx.x);
+				da[g][0] = 0.0 + q[0];
+				da[g][0] += q[1];
 			}
 		}
 		double ta[NA];
-		ok = res_exchange<NA, RPT>(da, count1, a.xch, turn, prev, ta);
-		prev = RPT * NA;
+		ok = res_exchange<NA, DOTS>(da, count1, a.xch, turn, prev, ta);
+		prev = DOTS * NA;
 		if (!ok) break;
 		pw = ta[0];
 		if (pw <= 0.0) ++ncurv;
@@ -1370,15 +1391,15 @@ cg_resident_kernel(res_args a) {
 	}
 }
 
-template<class T, bool SR, bool JAC>
+template<class T, bool SR, bool JAC, bool PAIRS = false>
 static void launch_resident(fsx_ctx * ctx, res_args a) {
 	const int64_t per = (int64_t)kResThreads * kResRows;
 	const dim3 grid((unsigned)((a.n + per - 1) / per));
 	if (a.sd.w == 7)
-		hipLaunchKernelGGL((cg_resident_kernel<T, SR, JAC, 7>), grid, dim3(kResThreads), 0,
+		hipLaunchKernelGGL((cg_resident_kernel<T, SR, JAC, PAIRS, 7>), grid, dim3(kResThreads), 0,
 		                   ctx->stream, a);
 	else
-		hipLaunchKernelGGL((cg_resident_kernel<T, SR, JAC, 5>), grid, dim3(kResThreads), 0,
+		hipLaunchKernelGGL((cg_resident_kernel<T, SR, JAC, PAIRS, 5>), grid, dim3(kResThreads), 0,
 		                   ctx->stream, a);
 }
 
@@ -1406,6 +1427,10 @@ static void enqueue_resident(fsx_ctx * ctx, const cg_bufs & B, cg_state * st, do
 	hipLaunchKernelGGL(res_reset_kernel, dim3((kXchDoubles + 255) / 256), dim3(256), 0,
 	                   ctx->stream, ctx->ws.xch, (int)(give_up ? RES_GAVE_UP : RES_RUNNING));
 	if constexpr (SR) launch_resident<T, true, false>(ctx, a);
+	else if (stencil_run(FSX_F64, a.n) == 2) {
+		if (B.dinv) launch_resident<T, false, true, true>(ctx, a);
+		else launch_resident<T, false, false, true>(ctx, a);
+	}
 	else if (B.dinv) launch_resident<T, false, true>(ctx, a);
 	else launch_resident<T, false, false>(ctx, a);
 	FSX_HIP(hipGetLastError());

@@ -444,12 +444,12 @@ def test_resident_solves_iteration_matched(ctx, dims):
         assert rel(xd.get(), xo) <= 1e-12
 
 
-def test_solves_from_two_threads(ctx):
+@pytest.mark.parametrize("n", [48, 400])  # one and two rows per lane in the launched product
+def test_solves_from_two_threads(ctx, n):
     """Two threads, each on a context of its own, solve small systems at once:
     one resident solve runs at a time and the other thread's takes the
     launched loop, with the same bits."""
     import threading
-    n = 48
     rp, ci, v = P.poisson2d(n)
     b = P.uniform(n * n, 81)
     s = dict(maxiter=2000, rtol=1e-10, use_zero_guess=True)
@@ -566,3 +566,35 @@ def test_resident_give_up_is_remembered(ctx, monkeypatch):
         assert its == its0 and k0 >= (3 if refine else 5) * its0
         assert k == k0 + extra  # the reset and launch that gave up
         extra = 0
+
+
+@pytest.mark.parametrize("dims", [(130, 1007), (362, 363), (64, 64, 50), (7, 93, 397), (512, 512)])
+def test_resident_bits_do_not_depend_on_the_path(ctx, monkeypatch, dims):
+    """Whether a solve of small size is resident depends on other threads, so
+    its bits must not: the launched loop and the resident one at sizes below,
+    at and past the two rows per lane of the launched FP64 product, up to the
+    largest resident system, in one launch and in several."""
+    S = None
+    for m in dims:
+        L = sp.diags([2.0 * np.ones(m), -np.ones(m - 1), -np.ones(m - 1)], [0, 1, -1])
+        S = L if S is None else sp.kron(sp.eye(m), S) + sp.kron(L, sp.eye(S.shape[0]))
+    S = sp.csr_matrix(S + sp.diags(P.uniform(S.shape[0], 71, 0.0, 2.0)))
+    S.sort_indices()
+    n = S.shape[0]
+    b, x0 = P.uniform(n, 72), P.uniform(n, 73)
+
+    def solve(c, jac):
+        A = c.csr(S.indptr.astype(np.int32), S.indices.astype(np.int32), S.data)
+        x = c.vec(x0)
+        i = fsx.cg_solve(A, c.vec(b), x, fsx.Settings(maxiter=60, rtol=1e-15),
+                         dinv=A.diag_inv() if jac else None)
+        return x.get(), i.as_dict(), list(fsx.cg_history(c))
+
+    launched = context_with(monkeypatch, FSX_CG_RESIDENT=0)
+    parts = context_with(monkeypatch, FSX_CG_RESIDENT_ITERS=13)
+    for jac in (True, False):
+        want = solve(launched, jac)
+        for c in (ctx, parts):
+            got = solve(c, jac)
+            np.testing.assert_array_equal(got[0], want[0])
+            assert got[1:] == want[1:]
