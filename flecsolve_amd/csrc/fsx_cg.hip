@@ -1025,8 +1025,8 @@ static void run_cg_loop_pipelined(fsx_ctx * ctx, const cg_bufs & B, cg_state * s
 // instead of stored and exchanged once more.
 //
 // Every wait ends.  At most one workgroup per CU is launched, and one resident
-// solve at a time in a process and device (a second thread's takes the launched
-// loop), so all of them start once other streams' and processes' kernels leave
+// launch at a time in a process and device (a second thread's solve takes the
+// launched loop), so all of them start once other streams' and processes' kernels leave
 // the CUs; a poll that lasts kResWaitTicks all the same gives up.
 //
 // A launch ends as a whole: one word says whether it gave up or finished, and
@@ -1437,8 +1437,9 @@ static void enqueue_resident(fsx_ctx * ctx, const cg_bufs & B, cg_state * st, do
 	ctx->launches += 2;
 }
 
-// The resident solve of a device, held from its launch to the read of its
-// state; one that is not free is not waited for.
+// The resident launch of a device, held from its enqueueing to the read of its
+// state (not while a diagnostic runs, which may solve something itself); one
+// that is not free is not waited for.
 constexpr int kResMaxDevices = 64;
 static std::mutex g_resident_mu[kResMaxDevices];
 
@@ -1493,9 +1494,10 @@ static void run_cg_loop_diag(fsx_ctx * ctx, const cg_bufs & B, cg_state * st,
 }
 
 // The iteration loop in resident launches: all iterations in one (or one at a
-// time, the host calling the diagnostic after each).  When a launch gives up,
-// *pinned and the vectors are where the launch before left them, and the context
-// takes the launched loop from then on: what kept the workgroups from running at
+// time, the host calling the diagnostic after each).  Ends early, *pinned and
+// the vectors where the launch before left them, when another thread's launch
+// is running or a launch gives up; after the latter the context takes the
+// launched loop from then on: what kept the workgroups from running at
 // once (another process's kernels, a mask on the CUs) tends to last, and every
 // segment of a refinement would wait for it again.
 template<class T, bool SR>
@@ -1504,10 +1506,14 @@ static void run_cg_loop_resident(fsx_ctx * ctx, const cg_bufs & B, cg_state * st
                                  fsx_diag_fn fn, void * user) {
 	const int maxit = pinned->maxiter;
 	while (!pinned->done && pinned->iter < maxit) {
-		enqueue_resident<T, SR>(ctx, B, st, hist, fn ? 1 : ctx->res_iters);
-		if (!read_resident(ctx, st, pinned)) {
-			ctx->res_on = false;
-			return;
+		{
+			std::unique_lock<std::mutex> mine(g_resident_mu[ctx->device], std::try_to_lock);
+			if (!mine.owns_lock()) return;
+			enqueue_resident<T, SR>(ctx, B, st, hist, fn ? 1 : ctx->res_iters);
+			if (!read_resident(ctx, st, pinned)) {
+				ctx->res_on = false;
+				return;
+			}
 		}
 		if (!fn) continue;
 		const int d = fn(user, xv, pinned->res);
@@ -1534,11 +1540,8 @@ static void run_cg_loop(fsx_ctx * ctx, const cg_bufs & B, const cg_work & wk,
 	                       ctx->stream));
 	if constexpr (std::is_same_v<T, V>) {
 		constexpr bool SR = std::is_same_v<T, float>;
-		std::unique_lock<std::mutex> mine;
 		if (ctx->res_on && SR == (B.part2 != nullptr) && fits_resident(B.A, B.n) &&
 		    ctx->device < kResMaxDevices)
-			mine = std::unique_lock<std::mutex>(g_resident_mu[ctx->device], std::try_to_lock);
-		if (mine.owns_lock())
 			run_cg_loop_resident<T, SR>(ctx, B, st, pinned, wk.hist, xv, diag, user);
 	}
 	if (pinned->done || pinned->iter >= pinned->maxiter) { // resident to the end
@@ -1554,7 +1557,7 @@ static void run_cg_loop(fsx_ctx * ctx, const cg_bufs & B, const cg_work & wk,
 		}
 		return;
 	}
-	if (pinned->iter > st_host.iter) { // the launched loop goes on where a launch gave up
+	if (pinned->iter > st_host.iter) { // the launched loop goes on from there
 		pinned->base = pinned->iter;
 		st_host = *pinned;
 		FSX_HIP(hipMemcpyAsync(st, pinned, sizeof(cg_state), hipMemcpyHostToDevice,

@@ -598,3 +598,37 @@ def test_resident_bits_do_not_depend_on_the_path(ctx, monkeypatch, dims):
             got = solve(c, jac)
             np.testing.assert_array_equal(got[0], want[0])
             assert got[1:] == want[1:]
+
+
+def test_resident_solve_inside_a_diagnostic(ctx):
+    """A diagnostic may solve on another context: nothing of the resident solve
+    it was called from is held meanwhile, so the inner one is resident too."""
+    n = 16
+    rp, ci, v, _ = diffusion(n)
+    b = P.uniform(n ** 3, 94)
+    s = fsx.Settings(maxiter=500, rtol=1e-9, use_zero_guess=True)
+
+    def solve(c, diag=None):
+        A = c.csr(rp, ci, v)
+        d, bd, x = A.diag_inv(), c.vec(b), c.zeros(n ** 3)
+        before = c.counters()[1]
+        i = fsx.cg_solve_diag(A, bd, x, s, diag, dinv=d) if diag else \
+            fsx.cg_solve(A, bd, x, s, dinv=d)
+        return i.iters, c.counters()[1] - before, x.get()
+
+    want = solve(ctx)
+    inner, other = [], fsx.Context(0)
+
+    def diag(x, res):
+        if len(inner) < 3:
+            inner.append(solve(other))
+        return False
+
+    got = solve(ctx, diag)
+    assert want[1] < 20 < want[0]
+    for it, k, x in inner:
+        assert (it, k) == want[:2]
+        np.testing.assert_array_equal(x, want[2])
+    # two launches an iteration on the outer context: it stayed resident
+    assert got[0] == want[0] and got[1] <= 2 * got[0] + 20
+    np.testing.assert_array_equal(got[2], want[2])
