@@ -1516,7 +1516,10 @@ static void run_cg_loop_resident(fsx_ctx * ctx, const cg_bufs & B, cg_state * st
 			}
 		}
 		if (!fn) continue;
-		const int d = fn(user, xv, pinned->res);
+		// a diagnostic's own reductions go through the same pinned scalars
+		const cg_state now = *pinned;
+		const int d = fn(user, xv, now.res);
+		*pinned = now;
 		if (d < 0) throw error(FSX_ERR_STATE, "cg: the user diagnostic reported an error");
 		if (d > 0) {
 			pinned->iters = pinned->iter;

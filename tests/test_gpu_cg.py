@@ -8,6 +8,8 @@ trajectories drift apart at the level of rounding; the solution comparison
 uses a tolerance a factor below the solve tolerance where the problem's
 conditioning allows, and otherwise compares against the exact solution.
 """
+import ctypes as C
+
 import numpy as np
 import pytest
 import scipy.sparse as sp
@@ -510,8 +512,14 @@ def test_resident_give_up_continues(ctx, monkeypatch, how, give_up):
             return x.get(), (i.status, i.outer_iters, i.inner_iters_total), seen, []
         d = A.diag_inv() if how != "identity" else None
         if how == "diag":
+            u = [c.vec(P.uniform(N, 95 + k)) for k in range(4)]
+            rr, rz = C.c_double(), C.c_double()
+
             def diag(xv, res):
-                seen.append((res, xv.get().tobytes()))
+                # sums of the diagnostic's own, on the same context
+                seen.append((res, xv.get().tobytes(), fsx.nrm2(xv)))
+                fsx.check(fsx.lib().fsx_cg_update(c.h, 0.0, u[0].h, u[1].h, None, u[2].h, u[3].h,
+                                                  None, C.byref(rr), C.byref(rz)))
                 return False
             i = fsx.cg_solve_diag(A, bd, x, s, diag, dinv=d)
         else:
@@ -632,3 +640,53 @@ def test_resident_solve_inside_a_diagnostic(ctx):
     # two launches an iteration on the outer context: it stayed resident
     assert got[0] == want[0] and got[1] <= 2 * got[0] + 20
     np.testing.assert_array_equal(got[2], want[2])
+
+
+def test_resident_slot_taken_between_launches(ctx, monkeypatch):
+    """A diagnostic's solve (a resident launch an iteration) whose slot another
+    thread's long solve takes meanwhile: it goes on in the launched loop from
+    its own state, whatever the diagnostic summed on its context, same bits."""
+    import threading
+    import time
+    n = 20
+    rp, ci, v, _ = diffusion(n)
+    N = n ** 3
+    b = P.uniform(N, 97)
+    big = P.poisson2d(512)
+    s = fsx.Settings(maxiter=500, rtol=1e-9, use_zero_guess=True)
+    u = [ctx.vec(P.uniform(N, 98 + k)) for k in range(4)]
+    rr, rz = C.c_double(), C.c_double()
+
+    def solve(at_five):
+        A = ctx.csr(rp, ci, v)
+        d, bd, x, calls = A.diag_inv(), ctx.vec(b), ctx.zeros(N), []
+
+        def diag(xv, res):
+            calls.append(res)
+            fsx.check(fsx.lib().fsx_cg_update(ctx.h, 0.0, u[0].h, u[1].h, None, u[2].h, u[3].h,
+                                              None, C.byref(rr), C.byref(rz)))
+            if len(calls) == 5:
+                at_five()
+            return False
+
+        before = ctx.counters()[1]
+        i = fsx.cg_solve_diag(A, bd, x, s, diag, dinv=d)
+        return x.get(), i.as_dict(), calls, ctx.counters()[1] - before
+
+    other = context_with(monkeypatch, FSX_CG_RESIDENT_ITERS=20000)
+    B = other.csr(*big)
+    bb, xb = other.vec(P.uniform(512 * 512, 99)), other.zeros(512 * 512)
+    long = fsx.Settings(maxiter=20000, rtol=1e-300, use_zero_guess=True)
+    fsx.cg_solve(B, bb, xb, fsx.Settings(maxiter=2, rtol=1e-300, use_zero_guess=True))
+    th = threading.Thread(target=fsx.cg_solve, args=(B, bb, xb, long))
+
+    def start():
+        th.start()
+        time.sleep(0.03)  # the long solve's one launch takes about 190 ms
+
+    want = solve(lambda: None)
+    got = solve(start)
+    th.join()
+    np.testing.assert_array_equal(got[0], want[0])
+    assert got[1:3] == want[1:3]
+    assert got[3] > want[3] + want[1]["iters"]  # it did go on in the launched loop
