@@ -645,8 +645,9 @@ def bench_batched(a, fsx, P):
     tune_ms = B.tune(bd, x, dinv, sample=64, iters=20)
     cfg = B.config()
     mapping_names = {0: "sliced", 1: "lanes", 2: "slice-offsets"}
+    lock_cg, lock_rr = B.lockstep()
     log(f"autotuned: workgroup {cfg[0]}, mapping {mapping_names[cfg[1]]}, "
-        f"lanes {cfg[2]} ({tune_ms:.2f} ms per sample run)")
+        f"lanes {cfg[2]}, lockstep: fp64 {lock_cg}, rr {lock_rr} ({tune_ms:.2f} ms)")
     L = fsx.lib()
     s64 = fsx.Settings(maxiter=a.maxiter, rtol=1e-10, use_zero_guess=True)
     inner = fsx.Settings(maxiter=a.maxiter, rtol=a.inner_rtol)
@@ -738,7 +739,7 @@ def bench_batched(a, fsx, P):
             "workload": f"batched_diffusion_{a.nsys}x_edges{a.emin}-{a.emax}_rtol1e-10",
             "systems": a.nsys, "rows": N, "nnz": nnz,
             "autotuned": {"workgroup": cfg[0], "mapping": mapping_names[cfg[1]],
-                          "lanes": cfg[2]},
+                          "lanes": cfg[2], "lockstep": {"fp64": lock_cg, "rr": lock_rr}},
             "fp64_cg": {"seconds": round(t64, 4), "iters_min": int(it64.min()),
                         "iters_max": int(it64.max()), "iters_sum": int(it64.sum()),
                         "max_true_rel_residual": float(rel64.max())},

@@ -53,6 +53,8 @@ struct fsx_batch {
 	// a configuration set by the caller names the kernel of one workgroup per
 	// system
 	bool fixed = false;
+	// FP64 solves in lockstep: as the tuner measured (0, 1) or by size (-1)
+	int lock = -1;
 	// lockstep solves: the blocks of rows (built by the first one), the
 	// systems' states, the partials, the count of running systems
 	std::unique_ptr<fsx::dbuf> ls_blocks, ls_st, ls_part, ls_active;
@@ -1177,9 +1179,14 @@ void copy_out(fsx_ctx * ctx, const batch_outputs & o, int64_t nsys, int * iters,
 //   256 of 16^3                   3.4 /  3.8 against  1.8 /  2.3
 //  2048 of 16^3                  13.8 / 22.2 against 12.0 / 16.3
 //  2048 of 8^3 .. 48^3            259 /  527 against  337 /  546
-bool use_lockstep(const fsx_batch * B, const fsx_csr * A32) {
-	if (B->fixed || B->mapping != 2 || (A32 && !A32->dg_vals)) return false;
-	if (B->min_rows <= 0 || B->max_rows <= 4096) return false;
+bool can_lockstep(const fsx_batch * B) {
+	return !B->fixed && has_sdia(B->A) && B->min_rows > 0 && B->max_rows > 4096;
+}
+
+bool use_lockstep(const fsx_batch * B, bool rr, const fsx_csr * A32 = nullptr) {
+	if (!can_lockstep(B) || (A32 && !A32->dg_vals)) return false;
+	if (!rr && B->lock >= 0) return B->lock == 1;
+	if (B->mapping != 2 && !B->tuned) return false;
 	const bool idle = B->max_rows * B->ctx->num_cus > 2 * B->A->nrows;
 	return idle || B->max_rows >= 32768;
 }
@@ -1396,6 +1403,15 @@ int fsx_batch_set_config(fsx_batch * B, int wg, int mapping, int lanes) {
 		B->mapping = mapping;
 		B->lanes = mapping == 1 ? lanes : 1;
 		B->fixed = true;
+		B->lock = -1;
+	});
+}
+
+int fsx_batch_lockstep(const fsx_batch * B, int * cg, int * rr) {
+	return guard([&] {
+		check_batch(B);
+		if (cg) *cg = use_lockstep(B, false);
+		if (rr) *rr = use_lockstep(B, true);
 	});
 }
 
@@ -1420,7 +1436,7 @@ static void batched_cg_run(fsx_ctx * ctx, fsx_batch * B, batch_work & W,
 		a.status = (int *)o.status->p;
 		a.res = (double *)o.res->p;
 		a.inner_iters = nullptr;
-		if (use_lockstep(B, nullptr)) {
+		if (use_lockstep(B, false)) {
 			if (dinv) ls_solve<false, true>(ctx, B, a);
 			else ls_solve<false, false>(ctx, B, a);
 		}
@@ -1576,7 +1592,7 @@ int fsx_batched_rr_cg(fsx_ctx * ctx, fsx_batch * B, const fsx_csr * A32,
 		a.status = (int *)o.status->p;
 		a.res = (double *)o.res->p;
 		a.inner_iters = (int *)o.inner->p;
-		if (use_lockstep(B, A32)) ls_solve<true, false>(ctx, B, a);
+		if (use_lockstep(B, true, A32)) ls_solve<true, false>(ctx, B, a);
 		else if (B->nsys > 0) launch<false, true>(ctx, B, a);
 		copy_out(ctx, o, B->nsys, segments, status, res, inner_iters);
 	});
@@ -1585,8 +1601,11 @@ int fsx_batched_rr_cg(fsx_ctx * ctx, fsx_batch * B, const fsx_csr * A32,
 // Autotuner: times each candidate configuration (workgroup size x row
 // mapping) on a sample of the batch's systems for a fixed amount of work
 // (`iters` CG iterations each, tolerance 0 so none stops early) and keeps the
-// fastest.  Results are cached per sparsity profile (mean nonzeros per row,
-// log2 of the median system size).
+// fastest.  Where the systems may go in lockstep, that is then timed against
+// the fastest on all of them (a sample leaves other CUs idle than the batch
+// does) by what 64 more iterations take.  Results are cached per profile: mean
+// nonzeros per row, log2 of the median and the largest system and of their
+// number, the layouts at hand.
 int fsx_batch_tune(fsx_ctx * ctx, fsx_batch * B, const fsx_vec * dinv,
                    const fsx_vec * b, fsx_vec * x, int sample, int iters,
                    double * best_ms) {
@@ -1602,18 +1621,22 @@ int fsx_batch_tune(fsx_ctx * ctx, fsx_batch * B, const fsx_vec * dinv,
 		FSX_REQUIRE(b->ptr() != x->ptr(), "b and x must differ");
 		if (dinv) check_same(dinv, b);
 		if (B->nsys == 0) return;
-		static std::map<std::pair<int, int>, std::tuple<int, int, int, double>> cache;
+		using profile = std::tuple<int, int, int, int, bool, bool, bool>;
+		static std::map<profile, std::tuple<int, int, int, int, double>> cache;
 		std::vector<int64_t> sizes(B->nsys);
 		for (int64_t s = 0; s < B->nsys; ++s) sizes[s] = B->h_rows[s + 1] - B->h_rows[s];
 		std::vector<int64_t> sorted = sizes;
 		std::nth_element(sorted.begin(), sorted.begin() + sorted.size() / 2, sorted.end());
 		const int64_t med = std::max<int64_t>(1, sorted[sorted.size() / 2]);
 		const int nnz_row = B->A->nrows ? (int)std::lround((double)B->A->nnz / B->A->nrows) : 0;
-		const std::pair<int, int> key{nnz_row, (int)std::floor(std::log2((double)med))};
+		auto lg = [](int64_t v) { return (int)std::floor(std::log2((double)std::max<int64_t>(1, v))); };
+		const profile key{nnz_row, lg(med), lg(B->max_rows), lg(B->nsys), B->min_rows > 0,
+		                  has_sdia(B->A), has_sliced(B->A)};
 		auto hit = cache.find(key);
 		if (hit != cache.end()) {
-			std::tie(B->wg, B->mapping, B->lanes, B->tuned_ms) = hit->second;
+			std::tie(B->wg, B->mapping, B->lanes, B->lock, B->tuned_ms) = hit->second;
 			B->tuned = true;
+			B->fixed = false;
 			if (best_ms) *best_ms = B->tuned_ms;
 			return;
 		}
@@ -1671,14 +1694,44 @@ int fsx_batch_tune(fsx_ctx * ctx, fsx_batch * B, const fsx_vec * dinv,
 				bc = c;
 			}
 		}
-		(void)hipEventDestroy(e0);
-		(void)hipEventDestroy(e1);
 		B->wg = bc.wg;
 		B->mapping = bc.mapping;
 		B->lanes = bc.lanes;
 		B->tuned = true;
+		B->fixed = false;
+		B->lock = -1;
+		if (can_lockstep(B)) {
+			fsx_vec * xs = nullptr; // x keeps its other systems
+			int rc = fsx_vec_create(ctx, b->n, FSX_F64, &xs);
+			if (rc) throw error(rc, get_error());
+			float ms[2][2];
+			try {
+				for (int lock = 0; lock < 2; ++lock) {
+					B->lock = lock;
+					for (int k = -1; k < 2; ++k) {
+						st.maxiter = iters + 64 * std::max(0, k);
+						FSX_HIP(hipEventRecord(e0, ctx->stream));
+						batched_cg_run(ctx, B, work_for(B, false), dinv, b, xs, &st, nullptr,
+						               nullptr, nullptr);
+						FSX_HIP(hipEventRecord(e1, ctx->stream));
+						FSX_HIP(hipEventSynchronize(e1));
+						FSX_HIP(hipEventElapsedTime(&ms[lock][std::max(0, k)], e0, e1));
+					}
+				}
+			}
+			catch (...) {
+				B->lock = -1;
+				(void)fsx_vec_release(xs);
+				throw;
+			}
+			fsx_vec_release(xs);
+			B->lock = ms[1][1] - ms[1][0] < ms[0][1] - ms[0][0] ? 1 : 0;
+			if (B->lock) best = ms[1][0];
+		}
+		(void)hipEventDestroy(e0);
+		(void)hipEventDestroy(e1);
 		B->tuned_ms = best;
-		cache[key] = std::make_tuple(bc.wg, bc.mapping, bc.lanes, best);
+		cache[key] = std::make_tuple(bc.wg, bc.mapping, bc.lanes, B->lock, best);
 		if (best_ms) *best_ms = best;
 	});
 }

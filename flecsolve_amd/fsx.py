@@ -188,6 +188,7 @@ _SIGS = {
     "fsx_batch_config": (C.c_int, [_P, C.POINTER(C.c_int), C.POINTER(C.c_int),
                                    C.POINTER(C.c_int)]),
     "fsx_batch_set_config": (C.c_int, [_P, C.c_int, C.c_int, C.c_int]),
+    "fsx_batch_lockstep": (C.c_int, [_P, C.POINTER(C.c_int), C.POINTER(C.c_int)]),
     "fsx_batch_tune": (C.c_int, [_P, _P, _P, _P, _P, C.c_int, C.c_int,
                                  C.POINTER(C.c_double)]),
     "fsx_batched_cg": (C.c_int, [_P, _P, _P, _P, _P, C.POINTER(Settings), _P, _P, _P]),
@@ -983,6 +984,13 @@ class Batch:
 
     def set_config(self, wg, mapping, lanes=1):
         check(lib().fsx_batch_set_config(self.h, wg, mapping, lanes), "set_config")
+
+    def lockstep(self) -> tuple[bool, bool]:
+        """Whether cg and rr_cg advance all systems in lockstep (instead of one
+        workgroup per system as configured)."""
+        a, b = C.c_int(), C.c_int()
+        check(lib().fsx_batch_lockstep(self.h, C.byref(a), C.byref(b)))
+        return bool(a.value), bool(b.value)
 
     def tune(self, b: Vector, x: Vector, dinv: Vector | None = None, sample=32,
              iters=20) -> float:

@@ -599,9 +599,16 @@ int fsx_batch_destroy(fsx_batch * B);
  * 1 `lanes` lanes per CSR row, 2 slice offsets). */
 int fsx_batch_config(const fsx_batch * B, int * wg, int * mapping, int * lanes);
 int fsx_batch_set_config(fsx_batch * B, int wg, int mapping, int lanes);
+/* Whether solves advance all systems in lockstep (1; three launches an
+ * iteration) instead of one workgroup per system as configured (0): fsx_batched_cg's
+ * as tuned, else by the systems' sizes; fsx_batched_rr_cg's by their sizes.
+ * Never after fsx_batch_set_config. */
+int fsx_batch_lockstep(const fsx_batch * B, int * cg, int * rr);
 /* Autotuner: times the candidate configurations on `sample` systems for
- * `iters` CG iterations each and keeps the fastest (cached per sparsity
- * profile).  Overwrites x on the sampled systems. */
+ * `iters` CG iterations each and keeps the fastest, then, where the sizes
+ * allow it, lockstep against it on all systems (cached per profile).  *best_ms:
+ * the time of the sample, or with lockstep of all systems.  Overwrites x on
+ * the sampled systems. */
 int fsx_batch_tune(fsx_ctx * ctx, fsx_batch * B, const fsx_vec * dinv,
                    const fsx_vec * b, fsx_vec * x, int sample, int iters,
                    double * best_ms);

@@ -310,3 +310,42 @@ def test_lockstep_matches_one_workgroup_per_system(ctx, edges):
     lock.cg(bd, x1, s, dinv=d)
     lock.cg(bd, x2, s, dinv=d)
     np.testing.assert_array_equal(x1.get(), x2.get())
+
+
+def test_tuner_chooses_between_lockstep_and_one_workgroup(ctx):
+    """The tuner times lockstep on the batch itself, says what it chose, and the
+    solves run that: few systems with one far larger go in lockstep (three
+    launches an iteration), systems of at most 4096 rows do not, a set
+    configuration never does.  x keeps the systems that were not sampled."""
+    def batch(edges):
+        probs = [P.diffusion3d(e, P.lognormal_field(e, 1.0, 4.0, 950 + e)) for e in edges]
+        S = sp.block_diag([sp.csr_matrix((v, ci, rp)) for rp, ci, v in probs], format="csr")
+        S.sort_indices()
+        A = ctx.csr(S.indptr.astype(np.int32), S.indices.astype(np.int32), S.data)
+        rows = np.concatenate([[0], np.cumsum([e ** 3 for e in edges])]).astype(np.int64)
+        return A, fsx.Batch(A, rows), int(rows[-1]), rows
+
+    s = fsx.Settings(maxiter=400, rtol=1e-9, use_zero_guess=True)
+    for edges, lock in (((40, 9, 8, 11), True), ((16, 9, 8, 11), False)):
+        A, B, n, rows = batch(edges)
+        d, bd = A.diag_inv(), ctx.vec(P.uniform(n, 33))
+        x0 = P.uniform(n, 34)
+        x = ctx.vec(x0)
+        assert B.lockstep() == (lock, lock)  # by size
+        for again in range(2):  # measured, then from the cache
+            assert B.tune(bd, x, d, sample=1, iters=10) > 0
+            assert B.lockstep() == (lock, lock)
+        np.testing.assert_array_equal(x.get()[rows[1]:], x0[rows[1]:])  # the largest is sampled
+        before = ctx.counters()[1]
+        it, st, _ = B.cg(bd, x, s, dinv=d)
+        launches = ctx.counters()[1] - before
+        assert (st == 1).all()
+        assert launches >= 3 * it.max() if lock else launches < 10
+        x1 = x.get()
+        B.set_config(512, 2, 1)
+        assert B.lockstep() == (False, False)
+        before = ctx.counters()[1]
+        it1, st1, _ = B.cg(bd, x, s, dinv=d)
+        assert ctx.counters()[1] - before < 10
+        assert (st1 == 1).all() and np.abs(it1 - it).max() <= 2
+        assert rel(x.get(), x1) <= 1e-8
