@@ -1173,12 +1173,26 @@ void copy_out(fsx_ctx * ctx, const batch_outputs & o, int64_t nsys, int * iters,
 // where a system outgrows the caches.  Measured to 1e-10 (ms, residual
 // replacement / FP64 CG, lockstep against the best workgroup size):
 //   160 systems of 8^3 .. 40^3   12.0        against 128 (256 threads)
-//    16 of 24^3                   3.0 /  2.7 against  5.3 /  8.1
+//   256 of 8^3 .. 48^3           30.0 / 54.1 against 107.9 / 170.5
+//  2048 of 8^3 .. 48^3            259 /  507 against  337 /  546
+//  1024 of 8^3 .. 32^3           25.7 / 45.7 against 29.2 / 47.6
 //    16 of 16^3                   1.8 /  1.6 against  1.3 /  1.9
-//   256 of 24^3                  10.3 / 14.2 against  7.7 / 15.0
 //   256 of 16^3                   3.4 /  3.8 against  1.8 /  2.3
-//  2048 of 16^3                  13.8 / 22.2 against 12.0 / 16.3
-//  2048 of 8^3 .. 48^3            259 /  527 against  337 /  546
+//    16 of 18^3                  1.60 / 1.42 against 1.73 / 2.61
+//    32 of 18^3                  1.74 / 1.65 against 1.74 / 2.62
+//    64 of 18^3                  2.14 / 2.26 against 1.79 / 2.80
+//   128 of 18^3                  2.71 / 3.23 against 2.23 / 2.86
+//    64 of 24^3                  3.97 / 4.95 against 6.12 / 8.19
+//   128 of 24^3                  6.14 / 8.16 against 6.55 / 8.30
+//   192 of 24^3                  7.70 / 11.1 against 6.81 / 12.7
+//   512 of 24^3                  16.1 / 27.6 against 14.2 / 28.9
+//   256 of 32^3                  23.1 / 43.1 against 31.7 / 46.8
+//   512 of 32^3                  44.9 / 87.7 against 62.0 / 93.8
+//   256 of 40^3                  53.3 /  109 against 75.7 /  121
+//   256 of 48^3                   114 /  236 against  162 /  253
+// Residual replacement reads half the bytes, so that its one workgroup keeps
+// up with a small system on more of the CUs: it leaves lockstep four times
+// earlier there.
 bool can_lockstep(const fsx_batch * B) {
 	return !B->fixed && has_sdia(B->A) && B->min_rows > 0 && B->max_rows > 4096;
 }
@@ -1187,7 +1201,8 @@ bool use_lockstep(const fsx_batch * B, bool rr, const fsx_csr * A32 = nullptr) {
 	if (!can_lockstep(B) || (A32 && !A32->dg_vals)) return false;
 	if (!rr && B->lock >= 0) return B->lock == 1;
 	if (B->mapping != 2 && !B->tuned) return false;
-	const bool idle = B->max_rows * B->ctx->num_cus > 2 * B->A->nrows;
+	const int64_t share = rr && B->max_rows < 8192 ? 8 : 2;
+	const bool idle = B->max_rows * B->ctx->num_cus > share * B->A->nrows;
 	return idle || B->max_rows >= 32768;
 }
 

@@ -349,3 +349,19 @@ def test_tuner_chooses_between_lockstep_and_one_workgroup(ctx):
         assert ctx.counters()[1] - before < 10
         assert (st1 == 1).all() and np.abs(it1 - it).max() <= 2
         assert rel(x.get(), x1) <= 1e-8
+
+
+def test_lockstep_by_size(ctx):
+    """The size rule on both sides of its lines: at most 4096 rows; small
+    systems enough to keep the CUs busy, for residual replacement earlier."""
+    for edge, count, want in ((16, 8, (False, False)), (17, 8, (True, True)),
+                              (18, 24, (True, True)), (18, 64, (True, False)),
+                              (18, 140, (False, False)), (24, 64, (True, True))):
+        rp, ci, v = P.diffusion3d(edge, P.lognormal_field(edge, 1.0, 4.0, 960))
+        n = edge ** 3
+        S = sp.csr_matrix((v, ci, rp))
+        S = sp.block_diag([S] * count, format="csr")
+        S.sort_indices()
+        A = ctx.csr(S.indptr.astype(np.int32), S.indices.astype(np.int32), S.data)
+        B = fsx.Batch(A, np.arange(count + 1, dtype=np.int64) * n)
+        assert B.lockstep() == want, (edge, count)
