@@ -858,7 +858,7 @@ __global__ __launch_bounds__(kLsThreads) void ls_b_kernel(ls_args g) {
 		st.alpha = alpha;
 		st.rho_b = rho;
 		st.tol_b = tol;
-		st.brk = RR && !(rho > 0.0);
+		st.brk = RR && phase == LS_START && !(rho > 0.0); // as a segment starts
 	}
 	ls_rows<RPT>(k, [&](int64_t r, int j) {
 		if constexpr (RR) {

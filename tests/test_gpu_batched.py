@@ -365,3 +365,66 @@ def test_lockstep_by_size(ctx):
         A = ctx.csr(S.indptr.astype(np.int32), S.indices.astype(np.int32), S.data)
         B = fsx.Batch(A, np.arange(count + 1, dtype=np.int64) * n)
         assert B.lockstep() == want, (edge, count)
+
+
+def same_or_close(a, b, tol):
+    """Equal infinities and NaN in the same places, the rest to a tolerance."""
+    np.testing.assert_array_equal(np.isnan(a), np.isnan(b))
+    np.testing.assert_array_equal(a[np.isinf(a)], b[np.isinf(a)])
+    ok = np.isfinite(b)
+    assert np.isfinite(a[ok]).all()
+    assert np.linalg.norm(a[ok] - b[ok]) <= tol * max(np.linalg.norm(b[ok]), 1e-300)
+
+
+@pytest.mark.parametrize("case", ["rhs", "matrix"])
+def test_lockstep_not_finite_as_one_workgroup(ctx, case):
+    """Systems whose numbers run out, beside sound ones: a NaN and an infinity
+    in the right-hand side, and a singular matrix whose first p.Ap is zero
+    (alpha infinite).  Counts, reasons and the places of NaN and infinity are
+    those of one workgroup per system."""
+    if case == "rhs":
+        edges = (20, 9, 17, 12)
+        S = sp.block_diag([sp.csr_matrix((v, ci, rp)) for rp, ci, v in
+                           (P.diffusion3d(e, P.lognormal_field(e, 1.0, 4.0, 970 + e))
+                            for e in edges)], format="csr")
+        rows = np.concatenate([[0], np.cumsum([e ** 3 for e in edges])]).astype(np.int64)
+        b = P.uniform(int(rows[-1]), 35)
+        b[rows[1] + 3], b[rows[3] - 70] = np.nan, np.inf
+    else:
+        m = 5000
+        one = sp.kron(sp.eye(m // 2), np.ones((2, 2)))
+        sound = sp.diags([np.full(m, 4.0), np.full(m - 1, -1.0), np.full(m - 1, -1.0)], [0, 1, -1])
+        S = sp.block_diag([sound, one, sound], format="csr")
+        rows = np.array([0, m, 2 * m, 3 * m], np.int64)
+        b = P.uniform(3 * m, 36)
+        b[m:2 * m] = np.tile([1.0, -1.0], m // 2)
+    S = sp.csr_matrix(S)
+    S.sort_indices()
+    A = ctx.csr(S.indptr.astype(np.int32), S.indices.astype(np.int32), S.data)
+    A.set_plan(3)
+    A32 = A.convert(fsx.F32)
+    A32.set_values_sym_scaled(A)
+    lock, one = fsx.Batch(A, rows), fsx.Batch(A, rows)
+    one.set_config(256, 2, 1)
+    assert lock.lockstep() == (True, True)
+    bd, d = ctx.vec(b), A.diag_inv()
+    for guess in (True, False):
+        for dinv in (d, None):
+            s = fsx.Settings(maxiter=25, rtol=1e-6, use_zero_guess=guess)
+            xl, xo = ctx.zeros(b.size), ctx.zeros(b.size)
+            l, o = lock.cg(bd, xl, s, dinv=dinv), one.cg(bd, xo, s, dinv=dinv)
+            np.testing.assert_array_equal(l[1], o[1])
+            np.testing.assert_array_equal(l[0], o[0])
+            same_or_close(l[2], o[2], 1e-6)
+            same_or_close(xl.get(), xo.get(), 1e-8)
+    xl, xo = ctx.zeros(b.size), ctx.zeros(b.size)
+    s = fsx.Settings(maxiter=60, rtol=3e-2)
+    l = lock.rr_cg(A32, bd, xl, 1e-9, s, max_segments=20)
+    o = one.rr_cg(A32, bd, xo, 1e-9, s, max_segments=20)
+    np.testing.assert_array_equal(l[2], o[2])
+    np.testing.assert_array_equal(l[0], o[0])
+    bad = o[2] != 1
+    assert bad.any()
+    np.testing.assert_array_equal(l[1][bad], o[1][bad])
+    assert np.abs(l[1] - o[1]).max() <= 2
+    same_or_close(xl.get(), xo.get(), 1e-8)
