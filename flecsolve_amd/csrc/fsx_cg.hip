@@ -593,7 +593,7 @@ static void append_layout(std::vector<const void *> & key, const fsx_csr * A) {
 	                       (const void *)(intptr_t)A->nnz,
 	                       (const void *)(intptr_t)A->plan_kind,
 	                       (const void *)(intptr_t)A->plan_lanes,
-	                       (const void *)(intptr_t)(A->st_full + 2 * A->st_serves)});
+	                       (const void *)(intptr_t)A->st_full});
 }
 } // namespace fsx
 

@@ -208,16 +208,14 @@ struct fsx_csr {
 	std::unique_ptr<fsx::dbuf> sl_vals; // values in the sliced-row layout
 	std::unique_ptr<fsx::dbuf> dg_vals; // values in the slice-offset layout
 	// values in the stencil layout; st_full: in its full form (else the CSR
-	// values are bitwise symmetric); st_serves: the products of plan 3 run on
-	// it (matrices planned by the library; a plan set by the caller names the
-	// kernel it asks for)
+	// values are bitwise symmetric)
 	std::unique_ptr<fsx::dbuf> st_vals;
-	bool st_full = false, st_serves = false;
+	bool st_full = false;
 	// dg_vals lag the CSR values (a rewrite served by the stencil layout
 	// skipped them); rebuilt by ensure_dg_fresh before any use
 	bool dg_stale = false;
 	// SpMV row mapping: 0 LDS-staged row blocks, 1 vector per row, 2 sliced
-	// rows, 3 slice offsets (or the stencil layout: st_serves), 4 symmetric
+	// rows, 3 slice offsets (or the stencil layout: on_stencil), 4 symmetric
 	// stencil
 	int plan_kind = 0;
 	int plan_lanes = 0;

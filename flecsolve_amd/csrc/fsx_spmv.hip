@@ -628,11 +628,8 @@ void refresh_sliced_values(fsx_ctx * ctx, fsx_csr * A) {
 	if (A->st_vals && A->idx->st_state > 0 && !stencil_fill(ctx, A)) {
 		// no longer symmetric: the full form serves the products of plan 3
 		A->st_vals.reset();
-		if (A->plan_kind == 4) {
-			A->plan_kind = 3;
-			A->st_serves = true;
-		}
-		if (A->st_serves) stencil_build(ctx, A, true);
+		if (A->plan_kind == 4) A->plan_kind = 3;
+		if (A->plan_kind == 3 && A->plan_lanes == 0) stencil_build(ctx, A, true);
 	}
 	if (A->idx->dg_ptr && A->dg_vals) {
 		// rebuilt when next read where the products run on the stencil layout
@@ -686,8 +683,10 @@ void choose_plan(fsx_ctx * ctx, fsx_csr * A, const void * host_rowptr,
 			// reported as plan 4 for symmetric FP64 matrices and as plan 3
 			// otherwise; the slice-offset layout is kept for the batched
 			// solves and for values that change
-			A->st_serves = ensure_stencil_any(ctx, A, host_rowptr, host_colind);
-			A->plan_kind = A->st_serves && A->vt == FSX_F64 && !A->st_full ? 4 : 3;
+			A->plan_kind = ensure_stencil_any(ctx, A, host_rowptr, host_colind) &&
+			                       A->vt == FSX_F64 && !A->st_full
+			                   ? 4
+			                   : 3;
 			A->plan_lanes = 0;
 			return;
 		}
@@ -1091,14 +1090,17 @@ int fsx_csr_convert(fsx_ctx * ctx, const fsx_csr * A, fsx_dtype vt,
 		if (A->dg_vals) B->dg_vals = cast_copy(*A->dg_vals, A->dg_vals->bytes / avsz);
 		else if (B->plan_kind == 3)
 			B->plan_kind = 0;
-		// a cast of symmetric values is symmetric; FP32 copies report plan 3
+		// a cast of symmetric values is symmetric; FP32 copies report plan 3,
+		// FP64 copies of what runs there on the symmetric stencil plan 4
 		if (A->st_vals) {
 			B->st_vals = cast_copy(*A->st_vals, A->st_vals->bytes / avsz);
 			B->st_full = A->st_full;
-			B->st_serves = A->st_serves || (A->plan_kind == 4 && vt == FSX_F32);
 		}
 		if (B->plan_kind == 4 && (vt == FSX_F32 || !B->st_vals))
 			B->plan_kind = B->dg_vals ? 3 : 0;
+		else if (A->vt == FSX_F32 && vt == FSX_F64 && A->plan_kind == 3 && on_stencil(A) &&
+		         !A->st_full)
+			B->plan_kind = 4;
 		FSX_HIP(hipStreamSynchronize(ctx->stream));
 		ctx_retain(ctx);
 		*out = B.release();
@@ -1164,6 +1166,9 @@ int fsx_csr_set_plan(fsx_csr * A, int kind, int lanes) {
 			FSX_REQUIRE(ensure_sdia(ctx, A, hrp.data(), hci.data(), false),
 			            "matrix structure does not fit the slice-offset layout");
 		}
+		// the layout the library's own plan 3 runs on, where the structure has it
+		if (kind == 3 && lanes == 0 && A->idx->st_state > 0)
+			ensure_stencil_any(A->ctx, A, nullptr, nullptr);
 		if (kind == 4) {
 			FSX_REQUIRE(A->nrows > 0, "the stencil layout needs a non-empty matrix");
 			FSX_REQUIRE(ensure_stencil(A->ctx, A, nullptr, nullptr),
@@ -1172,8 +1177,7 @@ int fsx_csr_set_plan(fsx_csr * A, int kind, int lanes) {
 			                : "matrix values are not symmetric (stencil layout)");
 		}
 		A->plan_kind = kind;
-		A->plan_lanes = kind == 1 ? lanes : 0;
-		A->st_serves = false;
+		A->plan_lanes = kind == 1 ? lanes : kind == 3 && lanes != 0 ? 1 : 0;
 	});
 }
 
@@ -1376,9 +1380,9 @@ int fsx_csr_shift_scale(fsx_ctx * ctx, const fsx_csr * F, double alpha, double b
 		// slice-offset values behind, rebuilt when next needed.
 		++A->vals_version;
 		const bool st_same = A->st_vals && F->st_vals && A->st_full == F->st_full;
-		const bool st_serves = on_stencil(A) && st_same;
+		const bool serves = on_stencil(A) && st_same;
 		if (ix.dg_ptr && A->dg_vals) {
-			if (st_serves)
+			if (serves)
 				A->dg_stale = true;
 			else if (F->dg_vals && ix.dg_nnz > 0) {
 				ensure_dg_fresh(ctx, F);
@@ -1409,11 +1413,8 @@ int fsx_csr_shift_scale(fsx_ctx * ctx, const fsx_csr * F, double alpha, double b
 		}
 		else if (A->st_vals && !stencil_fill(ctx, A)) {
 			A->st_vals.reset();
-			if (A->plan_kind == 4) {
-				A->plan_kind = 3;
-				A->st_serves = true;
-			}
-			if (A->st_serves) stencil_build(ctx, A, true);
+			if (A->plan_kind == 4) A->plan_kind = 3;
+			if (A->plan_kind == 3 && A->plan_lanes == 0) stencil_build(ctx, A, true);
 			ensure_dg_fresh(ctx, A);
 		}
 		if (ix.sl_ptr && A->sl_vals) {

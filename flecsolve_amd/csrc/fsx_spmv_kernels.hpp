@@ -664,10 +664,13 @@ inline unsigned stencil_blocks(fsx_dtype vt, int64_t nrows, bool reduces) {
 	return (unsigned)(reduces && vt == FSX_F32 ? std::min<int64_t>(g, kStencilMaxBlocksF32) : g);
 }
 
-// Products on the stencil layout: plan 4 (symmetric, FP64 by default), and
-// the matrices planned on slice offsets that have it too.
+// Products on the stencil layout: plan 4 (symmetric, FP64 by default), and plan
+// 3 without lanes on the FP32 and nonsymmetric matrices that have it (plan 3 of
+// a symmetric FP64 one, and with lanes, is slice offsets).  A function of the
+// plan alone, so that setting a matrix's reported plan gives its kernel back.
 inline bool on_stencil(const fsx_csr * A) {
-	return A->st_vals && (A->plan_kind == 4 || (A->plan_kind == 3 && A->st_serves));
+	return A->st_vals && (A->plan_kind == 4 || (A->plan_kind == 3 && A->plan_lanes == 0 &&
+	                                            (A->vt == FSX_F32 || A->st_full)));
 }
 
 template<class Epi, class ACC, class V, class G>

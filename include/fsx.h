@@ -191,8 +191,9 @@ int fsx_csr_info(const fsx_csr * A, int64_t * nrows, int64_t * ncols,
  * serves only structurally and bitwise symmetric values; chosen for such FP64
  * matrices, with slice offsets kept beside it).  FP32 and nonsymmetric matrices
  * with such an offset list report 3 and run on the stencil layout as well
- * (all offsets stored where not symmetric); set to 3 by the caller they run
- * on slice offsets.  A change of values that breaks the
+ * (all offsets stored where not symmetric); setting 3 with lanes = 0 gives them
+ * that, with another `lanes` slice offsets (reported as 3, 1).  A symmetric
+ * FP64 matrix set to 3 runs on slice offsets either way.  A change of values that breaks the
  * symmetry moves a plan-4 matrix to plan 3; fsx_csr_set_plan(A, 4, 0)
  * fails for a structure or values that do not fit.  Every mapping sums each
  * row serially in CSR order except 1. */

@@ -120,7 +120,7 @@ def test_every_plan_on_stencil(ctx, n):
         A.set_plan(plan)
         A32 = A.convert(fsx.F32)
         assert A32.plan() == (3, 0)
-        A32.set_plan(plan)
+        A32.set_plan(plan, 1 if plan == 3 else 0)  # 3, 1: slice offsets
         y32 = ctx.zeros(n ** 3, fsx.F32)
         A32.spmv(x32, y32)
         assert rel(y32.get().astype(np.float64), ref32) <= 1e-6
@@ -502,7 +502,7 @@ def test_stencil_runs_bit_exact(ctx, symmetric, dims, extra):
     outs = []
     for plan in (None, 3, 0):
         if plan is not None and A.plan()[0] >= 3:
-            A32.set_plan(plan)
+            A32.set_plan(plan, 1 if plan == 3 else 0)  # 3, 1: slice offsets
         y32, y64 = ctx.zeros(n, fsx.F32), ctx.zeros(n)
         A32.spmv(ctx.vec(x.astype(np.float32)), y32)
         A32.spmv(xd, y64)
@@ -536,3 +536,49 @@ def test_lanes_per_row_several_rows_a_group(ctx, lanes, n):
     assert (np.abs(y.get() - ref) <= 1e-13 * mag).all()
     pw = fsx.spmv_dot(A, ctx.vec(x), y)
     assert abs(pw - ref @ x) <= 1e-12 * (mag * np.abs(x)).sum()
+
+
+@pytest.mark.parametrize("kind", ["f64", "nonsym", "f32", "f32_nonsym"])
+def test_reported_plan_gives_its_kernel_back(ctx, kind):
+    """Setting a matrix's reported plan back, at once or after another one,
+    returns the layout it was on (told apart by the bytes its product moves),
+    for library-planned stencil matrices of every kind, their copies, and
+    plan 3 with lanes (slice offsets); the bits stay the same throughout."""
+    rp, ci, v = box_stencil((61, 53, 41), 11, "nonsym" not in kind)
+    n = rp.size - 1
+    A = ctx.csr(rp, ci, v)
+    if kind.startswith("f32"):
+        A = A.convert(fsx.F32)
+    dt, ft = (np.float32, fsx.F32) if kind.startswith("f32") else (np.float64, fsx.F64)
+    x, y = ctx.vec(np.random.default_rng(3).standard_normal(n).astype(dt)), ctx.zeros(n, ft)
+
+    def state(M):
+        M.spmv(x, y)
+        return M.plan(), M.layout_bytes(8), y.get().tobytes()
+
+    own = state(A)
+    assert own[0] == ((4, 0) if kind == "f64" else (3, 0))
+    A.set_plan(3, 1)
+    slices = state(A)
+    assert slices[0] == (3, 1) and slices[1] > own[1] and slices[2] == own[2]
+    for other in ((3, 1), (3, 0), (0, 0), (2, 0)):
+        A.set_plan(*own[0])
+        assert state(A) == own
+        A.set_plan(*other)
+        there = state(A)
+        assert there[2] == own[2]
+        A.set_plan(*there[0])
+        assert state(A) == there
+        B = A.convert(ft)
+        copy = state(B)
+        assert copy == there
+        B.set_plan(*copy[0])
+        assert state(B) == copy
+    A.set_plan(3, 1)
+    A.set_plan(*own[0])
+    # an FP64 copy of an FP32 matrix, and the other way, report what they run on
+    for M in (A.convert(fsx.F64), A.convert(fsx.F32)):
+        p, b = M.plan(), M.layout_bytes(8)
+        assert p == ((4, 0) if kind in ("f64", "f32") and M.vtype == fsx.F64 else (3, 0))
+        M.set_plan(*p)
+        assert (M.plan(), M.layout_bytes(8)) == (p, b)
