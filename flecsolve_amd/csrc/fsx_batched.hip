@@ -1084,7 +1084,6 @@ void check_batch(const fsx_batch * B) {
 }
 
 bool has_sliced(const fsx_csr * A) { return A->idx->sl_ptr && A->sl_vals; }
-bool has_sdia(const fsx_csr * A) { return A->idx->dg_ptr && A->dg_vals; }
 
 struct batch_outputs {
 	std::unique_ptr<dbuf> iters, status, res, inner;
@@ -1096,10 +1095,17 @@ struct batch_outputs {
 	}
 };
 
+// Whether the systems may go in lockstep (use_lockstep: whether they do).
+bool can_lockstep(const fsx_batch * B) {
+	return !B->fixed && has_sdia(B->A) && B->min_rows > 0 && B->max_rows > 4096;
+}
+
 batch_args base_args(fsx_batch * B, const fsx_csr * A32) {
 	const fsx_csr * A = B->A;
-	ensure_dg_fresh(B->ctx, A);
-	if (A32) ensure_dg_fresh(B->ctx, A32);
+	if (B->mapping == 2 || can_lockstep(B)) { // they read the slice-offset layout
+		ensure_dg_fresh(B->ctx, A);
+		if (A32) ensure_dg_fresh(B->ctx, A32);
+	}
 	batch_args a{};
 	a.nsys = B->nsys;
 	a.rows = (const int64_t *)B->rows->p;
@@ -1193,12 +1199,8 @@ void copy_out(fsx_ctx * ctx, const batch_outputs & o, int64_t nsys, int * iters,
 // Residual replacement reads half the bytes, so that its one workgroup keeps
 // up with a small system on more of the CUs: it leaves lockstep four times
 // earlier there.
-bool can_lockstep(const fsx_batch * B) {
-	return !B->fixed && has_sdia(B->A) && B->min_rows > 0 && B->max_rows > 4096;
-}
-
 bool use_lockstep(const fsx_batch * B, bool rr, const fsx_csr * A32 = nullptr) {
-	if (!can_lockstep(B) || (A32 && !A32->dg_vals)) return false;
+	if (!can_lockstep(B) || (A32 && !has_sdia(A32))) return false;
 	if (!rr && B->lock >= 0) return B->lock == 1;
 	if (B->mapping != 2 && !B->tuned) return false;
 	const int64_t share = rr && B->max_rows < 8192 ? 8 : 2;
@@ -1374,6 +1376,7 @@ int fsx_batch_create(fsx_ctx * ctx, const fsx_csr * A, int64_t nsys,
 		B->mapping = has_sdia(A) ? 2 : has_sliced(A) ? 0 : 1;
 		B->lanes = B->mapping == 1 ? 4 : 1;
 		B->wg = default_workgroup(B.get());
+		if (B->mapping == 2) ensure_dg_fresh(ctx, A); // not in the first solve
 		ctx_retain(ctx);
 		*out = B.release();
 	});
@@ -1496,7 +1499,7 @@ int fsx_batched_ir_cg(fsx_ctx * ctx, fsx_batch * B, const fsx_csr * A32,
 		FSX_REQUIRE(A32->vt == FSX_F32 && A32->idx == B->A->idx,
 		            "A32 must be fsx_csr_convert(A, FSX_F32) of the batch matrix");
 		FSX_REQUIRE(B->mapping != 0 || A32->sl_vals, "A32 lacks the sliced layout");
-		FSX_REQUIRE(B->mapping != 2 || A32->dg_vals, "A32 lacks the slice-offset layout");
+		FSX_REQUIRE(B->mapping != 2 || has_sdia(A32), "A32 lacks the slice-offset layout");
 		FSX_REQUIRE(jacobi >= 0 && jacobi <= 2, "jacobi must be 0, 1 or 2");
 		auto & W = work_for(B, true);
 		if (jacobi == 2) {
@@ -1568,7 +1571,7 @@ int fsx_batched_rr_cg(fsx_ctx * ctx, fsx_batch * B, const fsx_csr * A32,
 		            "A32 must be fsx_csr_convert(A, FSX_F32) of the batch matrix holding "
 		            "fsx_csr_set_values_f32_sym_scaled values");
 		FSX_REQUIRE(B->mapping != 0 || A32->sl_vals, "A32 lacks the sliced layout");
-		FSX_REQUIRE(B->mapping != 2 || A32->dg_vals, "A32 lacks the slice-offset layout");
+		FSX_REQUIRE(B->mapping != 2 || has_sdia(A32), "A32 lacks the slice-offset layout");
 		FSX_REQUIRE(inner->rtol > 0.0 && inner->rtol < 1.0,
 		            "the segment reduction inner->rtol must lie in (0, 1)");
 		FSX_REQUIRE(inner->maxiter >= 1, "inner->maxiter must be at least 1");

@@ -212,7 +212,8 @@ struct fsx_csr {
 	std::unique_ptr<fsx::dbuf> st_vals;
 	bool st_full = false;
 	// dg_vals lag the CSR values (a rewrite served by the stencil layout
-	// skipped them); rebuilt by ensure_dg_fresh before any use
+	// skipped them) or are not there yet (the products run on the stencil
+	// layout); built by ensure_dg_fresh before any use
 	bool dg_stale = false;
 	// SpMV row mapping: 0 LDS-staged row blocks, 1 vector per row, 2 sliced
 	// rows, 3 slice offsets (or the stencil layout: on_stencil), 4 symmetric
@@ -237,6 +238,10 @@ void ctx_release(fsx_ctx * c);
 // Rebuild A's slice-offset values from its CSR values if they lag
 // (stream-ordered; A's layouts are caches of its CSR values).
 void ensure_dg_fresh(fsx_ctx * ctx, const fsx_csr * A);
+// Whether A has the slice-offset layout, its values possibly still to be built.
+inline bool has_sdia(const fsx_csr * A) {
+	return A->idx->dg_ptr && (A->dg_vals || A->dg_stale);
+}
 
 inline fsx_ctx * ctx_of(const fsx_vec * v) { return v->ctx; }
 void check_vec(const fsx_vec * v, const char * name);

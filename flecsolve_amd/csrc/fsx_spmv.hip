@@ -344,8 +344,9 @@ static void sdia_fill(fsx_ctx * ctx, fsx_csr * A) {
 	}
 }
 
-bool ensure_sdia(fsx_ctx * ctx, fsx_csr * A, const void * host_rowptr,
-                 const void * host_colind, bool check_budget) {
+// The slice-offset index of A's structure, if it qualifies.
+static bool sdia_index(fsx_ctx * ctx, fsx_csr * A, const void * host_rowptr,
+                       const void * host_colind, bool check_budget) {
 	auto & X = *A->idx;
 	if (!X.dg_ptr) {
 		if (A->nrows == 0) return false;
@@ -378,11 +379,22 @@ bool ensure_sdia(fsx_ctx * ctx, fsx_csr * A, const void * host_rowptr,
 		}
 		FSX_HIP(hipStreamSynchronize(ctx->stream)); // host vectors go out of scope
 	}
+	return true;
+}
+
+static void sdia_alloc(fsx_csr * A) {
+	const size_t vsz = A->vt == FSX_F64 ? 8 : 4;
+	A->dg_vals = std::make_unique<dbuf>(std::max<int64_t>(1, A->idx->dg_nnz) * vsz);
+}
+
+bool ensure_sdia(fsx_ctx * ctx, fsx_csr * A, const void * host_rowptr,
+                 const void * host_colind, bool check_budget) {
+	if (!sdia_index(ctx, A, host_rowptr, host_colind, check_budget)) return false;
 	if (!A->dg_vals) {
-		const size_t vsz = A->vt == FSX_F64 ? 8 : 4;
-		A->dg_vals = std::make_unique<dbuf>(std::max<int64_t>(1, X.dg_nnz) * vsz);
+		sdia_alloc(A);
 		sdia_fill(ctx, A);
 		FSX_HIP(hipStreamSynchronize(ctx->stream));
+		A->dg_stale = false;
 	}
 	return true;
 }
@@ -619,7 +631,10 @@ static bool ensure_stencil_any(fsx_ctx * ctx, fsx_csr * A, const void * host_row
 void ensure_dg_fresh(fsx_ctx * ctx, const fsx_csr * A) {
 	if (!A->dg_stale) return;
 	fsx_csr * M = const_cast<fsx_csr *>(A);
-	if (M->idx->dg_ptr && M->dg_vals) sdia_fill(ctx, M);
+	if (M->idx->dg_ptr) {
+		if (!M->dg_vals) sdia_alloc(M);
+		sdia_fill(ctx, M);
+	}
 	M->dg_stale = false;
 }
 
@@ -678,16 +693,16 @@ void choose_plan(fsx_ctx * ctx, fsx_csr * A, const void * host_rowptr,
 	A->avg_row = A->nrows ? (double)A->nnz / (double)A->nrows : 0.0;
 	const double per_row_budget = (double)kStreamCap / kStreamRows;
 	if (A->avg_row <= per_row_budget) {
-		if (host_colind && ensure_sdia(ctx, A, host_rowptr, host_colind, true)) {
+		if (host_colind && sdia_index(ctx, A, host_rowptr, host_colind, true)) {
 			// one short offset list: the products run on the stencil layout,
 			// reported as plan 4 for symmetric FP64 matrices and as plan 3
-			// otherwise; the slice-offset layout is kept for the batched
-			// solves and for values that change
-			A->plan_kind = ensure_stencil_any(ctx, A, host_rowptr, host_colind) &&
-			                       A->vt == FSX_F64 && !A->st_full
-			                   ? 4
-			                   : 3;
+			// otherwise; the slice-offset values are built when something
+			// reads them (batched solves, a plan set to slice offsets)
+			const bool st = ensure_stencil_any(ctx, A, host_rowptr, host_colind);
+			A->plan_kind = st && A->vt == FSX_F64 && !A->st_full ? 4 : 3;
 			A->plan_lanes = 0;
+			if (st) A->dg_stale = true;
+			else ensure_sdia(ctx, A, host_rowptr, host_colind, true);
 			return;
 		}
 		const int64_t padded =
@@ -1049,7 +1064,6 @@ int fsx_csr_convert(fsx_ctx * ctx, const fsx_csr * A, fsx_dtype vt,
                     fsx_csr ** out) {
 	return guard([&] {
 		FSX_REQUIRE(ctx && A && out, "null argument");
-		ensure_dg_fresh(ctx, A); // B copies A's layouts
 		auto B = std::make_unique<fsx_csr>();
 		B->ctx = ctx;
 		B->nrows = A->nrows;
@@ -1087,7 +1101,7 @@ int fsx_csr_convert(fsx_ctx * ctx, const fsx_csr * A, fsx_dtype vt,
 		if (A->sl_vals) B->sl_vals = cast_copy(*A->sl_vals, A->sl_vals->bytes / avsz);
 		else if (B->plan_kind == 2)
 			B->plan_kind = 0;
-		if (A->dg_vals) B->dg_vals = cast_copy(*A->dg_vals, A->dg_vals->bytes / avsz);
+		if (has_sdia(A)) B->dg_stale = true; // filled below where B reads them
 		else if (B->plan_kind == 3)
 			B->plan_kind = 0;
 		// a cast of symmetric values is symmetric; FP32 copies report plan 3,
@@ -1097,10 +1111,11 @@ int fsx_csr_convert(fsx_ctx * ctx, const fsx_csr * A, fsx_dtype vt,
 			B->st_full = A->st_full;
 		}
 		if (B->plan_kind == 4 && (vt == FSX_F32 || !B->st_vals))
-			B->plan_kind = B->dg_vals ? 3 : 0;
+			B->plan_kind = has_sdia(B.get()) ? 3 : 0;
 		else if (A->vt == FSX_F32 && vt == FSX_F64 && A->plan_kind == 3 && on_stencil(A) &&
 		         !A->st_full)
 			B->plan_kind = 4;
+		if (!on_stencil(B.get())) ensure_dg_fresh(ctx, B.get());
 		FSX_HIP(hipStreamSynchronize(ctx->stream));
 		ctx_retain(ctx);
 		*out = B.release();
@@ -1151,8 +1166,7 @@ int fsx_csr_set_plan(fsx_csr * A, int kind, int lanes) {
 			FSX_REQUIRE(A->nrows > 0, "sliced rows need a non-empty matrix");
 			ensure_sliced(A->ctx, A, nullptr);
 		}
-		if (kind == 3) ensure_dg_fresh(A->ctx, A);
-		if (kind == 3 && !(A->idx->dg_ptr && A->dg_vals)) {
+		if (kind == 3 && !has_sdia(A)) {
 			FSX_REQUIRE(A->nrows > 0, "slice offsets need a non-empty matrix");
 			fsx_ctx * ctx = A->ctx;
 			const size_t isz = A->it == FSX_I32 ? 4 : 8;
@@ -1178,6 +1192,7 @@ int fsx_csr_set_plan(fsx_csr * A, int kind, int lanes) {
 		}
 		A->plan_kind = kind;
 		A->plan_lanes = kind == 1 ? lanes : kind == 3 && lanes != 0 ? 1 : 0;
+		if (kind == 3 && !on_stencil(A)) ensure_dg_fresh(A->ctx, A);
 	});
 }
 

@@ -189,7 +189,7 @@ int fsx_csr_info(const fsx_csr * A, int64_t * nrows, int64_t * ncols,
  * per row for the offsets it has, values stored only for the offsets >= 0; the
  * entries below the diagonal are read from their mirrors above it, so it
  * serves only structurally and bitwise symmetric values; chosen for such FP64
- * matrices, with slice offsets kept beside it).  FP32 and nonsymmetric matrices
+ * matrices; their slice-offset values are built when something reads them).  FP32 and nonsymmetric matrices
  * with such an offset list report 3 and run on the stencil layout as well
  * (all offsets stored where not symmetric); setting 3 with lanes = 0 gives them
  * that, with another `lanes` slice offsets (reported as 3, 1).  A symmetric

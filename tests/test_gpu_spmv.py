@@ -582,3 +582,38 @@ def test_reported_plan_gives_its_kernel_back(ctx, kind):
         assert p == ((4, 0) if kind in ("f64", "f32") and M.vtype == fsx.F64 else (3, 0))
         M.set_plan(*p)
         assert (M.plan(), M.layout_bytes(8)) == (p, b)
+
+
+@pytest.mark.parametrize("kind", ["f64", "nonsym", "f32"])
+def test_stencil_matrix_holds_one_product_layout(ctx, kind):
+    """Device memory of a matrix whose products run on the stencil layout: CSR,
+    that layout and the slice-offset index; slice-offset values appear only when
+    something reads them (a plan set to them, a batch), then up to date."""
+    rp, ci, v = box_stencil((61, 53, 41), 13, kind != "nonsym")
+    n, nnz = rp.size - 1, ci.size
+    src = ctx.csr(rp, ci, v)
+    before = fsx.alloc_stats()[1]
+    A = src.convert(fsx.F32) if kind == "f32" else ctx.csr(rp, ci, v)
+    held = fsx.alloc_stats()[1] - before
+    vb = 4 if kind == "f32" else 8
+    stored = 4 if kind != "nonsym" else 7
+    need = nnz * vb + (n + 64) * stored * vb
+    if kind != "f32":  # the copy shares the index arrays
+        need += nnz * 4 + n * 4 + n * 5 + n // 64 * 16 * 12
+    assert held <= 1.02 * need + 65536
+    dt, ft = (np.float32, fsx.F32) if kind == "f32" else (np.float64, fsx.F64)
+    x = np.random.default_rng(3).standard_normal(n).astype(dt)
+    xd, y, z = ctx.vec(x), ctx.zeros(n, ft), ctx.zeros(n, ft)
+    v2 = v * 1.25
+    if kind == "f32":
+        src.set_values(v2)
+        A.set_values_from(src)
+    else:
+        A.set_values(v2)
+    A.spmv(xd, y)
+    A.set_plan(3, 1)
+    A.spmv(xd, z)
+    np.testing.assert_array_equal(y.get(), z.get())
+    if kind != "f32":
+        B = fsx.Batch(ctx.csr(rp, ci, v), np.array([0, n], np.int64))
+        assert B.config()[1] == 2
