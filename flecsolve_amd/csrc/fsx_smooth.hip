@@ -387,6 +387,14 @@ __global__ __launch_bounds__(kLdsThreads) void gs_lds_kernel(int n, gs_dir_view 
 // Largest matrix gs_lds_kernel takes: x, a zero and the count in the 160 KB
 // of a CU.
 constexpr int64_t kGsLdsRows = 160 * 1024 / (int64_t)sizeof(double) - 2;
+// Its widest levels, in rows on average: a launch per level works on them with
+// every CU, one workgroup with one.  A symmetric sweep in one workgroup / in a
+// launch per level or run of levels (us): 9-point, 10000 rows in levels of 34
+// rows 186 / 892, of 156 61 / 204, of 625 55 / 94, of 2500 53 / 33; 19600 rows
+// of 306 119 / 331, of 1225 113 / 97; red-black 5-point, 1024 rows of 512
+// 12 / 21, 4096 of 2048 26 / 21, 19600 of 9800 113 / 22; random structure, 20000
+// rows of 323 625 / 959, of 556 335 / 410, of 690 267 / 305, of 1429 204 / 97.
+constexpr int64_t kGsLdsLevelRows = 768;
 
 // Refresh the copy's values from the matrix (entry index per slot, -1 for
 // padding / a missing diagonal).
@@ -684,9 +692,9 @@ void build_tiles(fsx_ctx * ctx, fsx_gs & G) {
 }
 
 // gs_lds_kernel's copy of one sweep direction of a one-colour matrix, if it
-// takes the matrix: x fits LDS, no row is longer than kLdsMaxWidth, and no
-// entry couples rows of one level or a later row of a lower level (earlier
-// rows lie in lower levels by construction).
+// takes the matrix: x fits LDS, the levels are narrow enough, no row is longer
+// than kLdsMaxWidth, and no entry couples rows of one level or a later row of a
+// lower level (earlier rows lie in lower levels by construction).
 template<class I>
 void build_lds_records(fsx_ctx * ctx, const std::vector<int64_t> & rp,
                        const std::vector<int32_t> & lev, bool fwd,
@@ -695,6 +703,7 @@ void build_lds_records(fsx_ctx * ctx, const std::vector<int64_t> & rp,
                        fsx_gs::dir & D) {
 	const int64_t n = (int64_t)order.size();
 	if (n == 0 || n > kGsLdsRows) return;
+	if (n > kGsLdsLevelRows * ((int64_t)D.lev.size() - 1)) return;
 	const int maxlen = *std::max_element(slen.begin(), slen.end());
 	if (maxlen > kLdsMaxWidth) return;
 	const int w = std::max(8, (maxlen + 7) / 8 * 8);

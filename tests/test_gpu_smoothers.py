@@ -238,3 +238,42 @@ def test_relaxation_in_shared_memory_bit_exact(ctx, itype, n, per_row, long_rows
         got, ref, _ = run_both(ctx, rp.astype(itype), ci.astype(itype), v, sweep, nrelax, 1,
                                seed=9 + sweep)
         np.testing.assert_array_equal(got, ref)
+
+
+def wide_level_csr(m, parts):
+    """9-point matrix on m x m, numbered part by part of parts x parts rows of
+    independent points: `parts`^2 levels of m^2 / parts^2 rows."""
+    T = sp.diags([np.ones(m), np.ones(m - 1), np.ones(m - 1)], [0, 1, -1])
+    S = sp.csr_matrix(sp.kron(T, T))
+    rng = np.random.default_rng(m)
+    S.data = rng.uniform(-1.0, 1.0, S.nnz)
+    S = sp.csr_matrix(S + sp.diags(np.full(m * m, 12.0)))
+    i = np.arange(m * m)
+    order = np.argsort((i % m) % parts + parts * ((i // m) % parts), kind="stable")
+    S = S[order][:, order].tocsr()
+    S.sort_indices()
+    return S.indptr.astype(np.int32), S.indices.astype(np.int32), S.data
+
+
+@pytest.mark.parametrize("m,parts,shared", [(130, 4, False), (140, 2, False)])
+def test_wide_levels_keep_their_launches(ctx, m, parts, shared):
+    """Matrices whose x fits one CU's shared memory, with levels of 1056
+    and 4900 rows: every CU works on a level, not one workgroup on all of
+    them.  The oracle's bits, and one copy of the matrix on the device."""
+    rp, ci, v = wide_level_csr(m, parts)
+    n, off = m * m, ci.size - m * m
+    A = ctx.csr(rp, ci, v)
+    before = fsx.alloc_stats()[1]
+    G = fsx.HybridGS(A)
+    held = fsx.alloc_stats()[1] - before
+    levels = G.levels()[0]
+    assert (n / levels <= 768) == shared
+    per_row = n * (4 + 4 + 8 + 8)          # ids, lengths, diagonals and their entries
+    record = n * (8 * 18 + 4)              # eight columns, values and entries
+    slots = 2 * (off + n) * 20 + 8 * n     # columns, values and entries; x kept aside
+    want = 2 * per_row + (2 * record if shared else slots)
+    assert held <= want * 1.05 + 65536, (held, want)
+    del G
+    for sweep, nrelax in ((0, 1), (1, 1), (2, 2)):
+        got, ref, _ = run_both(ctx, rp, ci, v, sweep, nrelax, 1, seed=19 + sweep)
+        np.testing.assert_array_equal(got, ref)
