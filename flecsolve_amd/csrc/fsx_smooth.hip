@@ -1013,11 +1013,25 @@ int fsx_gs_create(fsx_ctx * ctx, const fsx_csr * A, int ncolours, fsx_gs ** out)
 		if (G->tiles) build_tiles(ctx, *G);
 		// an explicit FSX_GS_RUN_ROWS asks for the launches it shapes
 		G->lds = !re && G->fw.rwidth && G->bw.rwidth;
+		// the copy that is not read: the level-ordered one (ids, lengths and
+		// diagonals serve both), or one direction's records
+		for (fsx_gs::dir * D : {&G->fw, &G->bw}) {
+			if (G->lds) {
+				for (auto * d : {&D->srow, &D->scol, &D->sval, &D->vfrom, &D->dlev, &D->dbase,
+				                 &D->dwidth})
+					d->reset();
+				D->nslots = 0;
+			}
+			else {
+				for (auto * d : {&D->steps, &D->lrow, &D->rcol, &D->rval, &D->rfrom}) d->reset();
+				D->rwidth = 0;
+			}
+		}
 		if (G->lds)
 			FSX_HIP(hipFuncSetAttribute((const void *)&gs_lds_kernel,
 			                            hipFuncAttributeMaxDynamicSharedMemorySize,
 			                            (int)((kGsLdsRows + 2) * sizeof(double))));
-		G->xold = std::make_unique<dbuf>(std::max<int64_t>(1, n) * sizeof(double));
+		else G->xold = std::make_unique<dbuf>(std::max<int64_t>(1, n) * sizeof(double));
 		refresh_values(*G);
 		G->version = A->vals_version;
 		ctx_retain(ctx);

@@ -255,11 +255,11 @@ def wide_level_csr(m, parts):
     return S.indptr.astype(np.int32), S.indices.astype(np.int32), S.data
 
 
-@pytest.mark.parametrize("m,parts,shared", [(130, 4, False), (140, 2, False)])
+@pytest.mark.parametrize("m,parts,shared", [(140, 8, True), (130, 4, False), (140, 2, False)])
 def test_wide_levels_keep_their_launches(ctx, m, parts, shared):
-    """Matrices whose x fits one CU's shared memory, with levels of 1056
-    and 4900 rows: every CU works on a level, not one workgroup on all of
-    them.  The oracle's bits, and one copy of the matrix on the device."""
+    """Matrices whose x fits one CU's shared memory, with levels of 306, 1056
+    and 4900 rows: one workgroup takes the first, every CU works on a level of
+    the others.  The oracle's bits, and one copy of the matrix on the device."""
     rp, ci, v = wide_level_csr(m, parts)
     n, off = m * m, ci.size - m * m
     A = ctx.csr(rp, ci, v)
