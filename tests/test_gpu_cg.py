@@ -418,8 +418,9 @@ def test_cg_user_diagnostic(ctx):
 def test_resident_solves_iteration_matched(ctx, dims):
     """Small stencil systems run all iterations in one launch, a thread per
     four rows: row counts below, at and past a workgroup's 1024, and at and
-    past the largest system (262144 rows); 25 iterations with Jacobi and
-    without, from a nonzero guess, against the oracle's trajectory."""
+    past the largest system (262144 rows), told by the launches made; 25
+    iterations with Jacobi and without, from a nonzero guess, against the
+    oracle's trajectory."""
     S = None
     for m in dims:
         L = sp.diags([2.0 * np.ones(m), -np.ones(m - 1), -np.ones(m - 1)], [0, 1, -1])
@@ -439,8 +440,10 @@ def test_resident_solves_iteration_matched(ctx, dims):
         xo, io, ho = O.cg(Ao, b, x0, O.Settings(**s), P=O.prec(1, Ao.dinv()) if jac else None,
                           hist_cap=25)
         xd = ctx.vec(x0)
-        info = fsx.cg_solve(A, ctx.vec(b), xd, fsx.Settings(**s),
-                            dinv=A.diag_inv() if jac else None)
+        d, bd, before = A.diag_inv() if jac else None, ctx.vec(b), ctx.counters()[1]
+        info = fsx.cg_solve(A, bd, xd, fsx.Settings(**s), dinv=d)
+        launches = ctx.counters()[1] - before
+        assert (launches < 25) == (n <= 262144 and A.plan() == (4, 0)), launches
         assert info.reason == io.reason
         np.testing.assert_allclose(fsx.cg_history(ctx), ho, rtol=1e-9)
         assert rel(xd.get(), xo) <= 1e-12
@@ -690,3 +693,34 @@ def test_resident_slot_taken_between_launches(ctx, monkeypatch):
     np.testing.assert_array_equal(got[0], want[0])
     assert got[1:3] == want[1:3]
     assert got[3] > want[3] + want[1]["iters"]  # it did go on in the launched loop
+
+
+@pytest.mark.parametrize("where", ["rhs", "guess", "matrix"])
+def test_resident_not_finite_as_launched(ctx, monkeypatch, where):
+    """A NaN or an infinity in the right-hand side, the guess or the matrix: the
+    resident solve runs into it as the launched one does -- the same counts,
+    history and places of NaN -- and ends."""
+    n = 40
+    rp, ci, v = P.poisson2d(n)
+    rows = np.repeat(np.arange(n * n), np.diff(rp))
+    never = context_with(monkeypatch, FSX_CG_RESIDENT=0)
+    for bad in (np.nan, np.inf):
+        b, x0, w = P.uniform(n * n, 61), P.uniform(n * n, 62), v.copy()
+        if where == "rhs":
+            b[777] = bad
+        elif where == "guess":
+            x0[5] = bad
+        else:
+            w[(rows == 801) & (ci == 801)] = bad
+        for jac in (True, False):
+            out = []
+            for c in (ctx, never):
+                A = c.csr(rp, ci, w)
+                assert A.plan() == (4, 0)
+                x = c.vec(x0)
+                i = fsx.cg_solve(A, c.vec(b), x, fsx.Settings(maxiter=30, rtol=1e-8),
+                                 dinv=A.diag_inv() if jac else None)
+                out.append((x.get(), i.reason, i.iters, fsx.cg_history(c)))
+            np.testing.assert_array_equal(out[0][0], out[1][0])
+            assert out[0][1:3] == out[1][1:3]
+            np.testing.assert_array_equal(out[0][3], out[1][3])

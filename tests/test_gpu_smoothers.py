@@ -277,3 +277,22 @@ def test_wide_levels_keep_their_launches(ctx, m, parts, shared):
     for sweep, nrelax in ((0, 1), (1, 1), (2, 2)):
         got, ref, _ = run_both(ctx, rp, ci, v, sweep, nrelax, 1, seed=19 + sweep)
         np.testing.assert_array_equal(got, ref)
+
+
+@pytest.mark.parametrize("bad", [np.nan, np.inf, -np.inf])
+def test_shared_memory_relaxation_not_finite(ctx, bad):
+    """A NaN or an infinity in b or x reaches exactly the rows it reaches in the
+    sequential sweep (rows of more and fewer than 24 entries, padded ones)."""
+    n = 3000
+    rp, ci, v = mirrored_csr(n, 9, 3, 5)
+    A = ctx.csr(rp.astype(np.int32), ci.astype(np.int32), v)
+    Ao = O.Csr(rp.astype(np.int32), ci.astype(np.int32), v)
+    G = fsx.HybridGS(A)
+    for in_b, at in ((True, n - 3), (False, 1500), (False, 0)):
+        b, x = P.uniform(n, 41), P.uniform(n, 42)
+        (b if in_b else x)[at] = bad
+        for sweep in (0, 1, 2):
+            xd = ctx.vec(x)
+            G.apply(ctx.vec(b), xd, sweep, 1)
+            ref = Ao.hybrid_gs(b, x, sweep=sweep, nrelax=1)
+            np.testing.assert_array_equal(xd.get(), ref)
