@@ -754,7 +754,9 @@ def bench_batched(a, fsx, P):
             "rr": rr,
             "value_is": "rr" if (rr and a.ir_method == "rr") else "ir",
         },
-        "roofline": {"bound": "hbm", "kernel": "batched_cg_kernel<jacobi, fp64>",
+        "roofline": {"bound": "hbm",
+                     "kernel": "ls_a/b/c_kernel<fp64, jacobi> (lockstep)" if lock_cg
+                     else "batched_cg_kernel<jacobi, fp64>",
                      "achieved": round(gbs, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(gbs / HBM_PEAK_GBS, 4), "traffic": None,
                      "algorithmic_bytes": bytes64,

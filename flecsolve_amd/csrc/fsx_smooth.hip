@@ -223,11 +223,11 @@ __global__ __launch_bounds__(kRunThreads) void gs_run_kernel(
 //
 // Measured (MI355X) on the seven Gauss-Seidel levels of a 48 x 44 x 40
 // aggregation hierarchy, 15671 rows and fewer, ~900 levels per direction:
-// the AMG-CG solve 371 ms -> 120 ms, of which a level costs ~0.5 us against
-// 1.7 us in gs_run_kernel.  Also measured: a barrier per step for the whole
-// workgroup 290 ms (each step then waits for its group's next loads to be
-// issued); 1024 threads, which leave no registers to gather a row's x at
-// once, 184 ms.
+// the AMG-CG solve 442 ms -> 134 ms, a level ~0.5 us against 1.7 us in
+// gs_run_kernel.  Also measured, on a solve of fewer iterations (120 ms so):
+// a barrier per step for the whole workgroup 290 ms (each step then waits for
+// its group's next loads to be issued); 1024 threads, which leave no registers
+// to gather a row's x at once, 184 ms.
 constexpr int kLdsThreads = 512; // 2 waves per SIMD: a row's entries and x stay in registers
 constexpr int kLdsWaves = kLdsThreads / 64;
 constexpr int kLdsRow = 24;      // entries of a row kept in registers

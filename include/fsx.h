@@ -590,8 +590,9 @@ int fsx_be_adjoint_rr(fsx_ctx * ctx, const fsx_csr * A, const fsx_csr * A32,
  * A is the block-diagonal concatenation (int32 indices, FP64 values, global
  * column ids) of nsys systems; system s owns rows [sys_rows[s],
  * sys_rows[s+1]).  Each system is solved with op::cg::apply's iteration
- * (flecsolve/solvers/cg.hh:43-139) by one workgroup; per-system results are
- * written to the host arrays (any may be NULL). */
+ * (flecsolve/solvers/cg.hh:43-139) by one workgroup, or all systems advance in
+ * lockstep (fsx_batch_lockstep); per-system results are written to the host
+ * arrays (any may be NULL). */
 typedef struct fsx_batch fsx_batch;
 int fsx_batch_create(fsx_ctx * ctx, const fsx_csr * A, int64_t nsys,
                      const int64_t * sys_rows, fsx_batch ** out);
