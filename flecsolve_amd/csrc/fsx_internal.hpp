@@ -196,6 +196,8 @@ struct csr_index {
 	// bit per entry, set at each diag_pos entry
 	int diag_full = -1;
 	std::unique_ptr<fsx::dbuf> diag_pos, diag_bits;
+	// median |column - row| of the entries (of a sample of rows); -1: unknown
+	double col_dist = -1;
 };
 
 struct fsx_csr {

@@ -665,15 +665,38 @@ void refresh_sliced_values(fsx_ctx * ctx, fsx_csr * A) {
 	}
 }
 
+// Median |column - row| over at most 4096 rows, evenly spread, and 64 entries of
+// each (the median: a few couplings to anywhere do not move what the others hit).
+template<class I>
+static double column_distance(int64_t nrows, const I * rp, const I * ci) {
+	const int64_t rows = std::min<int64_t>(nrows, 4096);
+	std::vector<int64_t> d;
+	for (int64_t k = 0; k < rows; ++k) {
+		const int64_t r = k * (nrows / rows) + k * (nrows % rows) / rows;
+		const int64_t lo = rp[r], len = (int64_t)rp[r + 1] - lo, m = std::min<int64_t>(len, 64);
+		for (int64_t e = 0; e < m; ++e) d.push_back(std::abs((int64_t)ci[lo + e * len / m] - r));
+	}
+	if (d.empty()) return 0;
+	std::nth_element(d.begin(), d.begin() + d.size() / 2, d.end());
+	return (double)d[d.size() / 2];
+}
+
 // Short rows whose slices share few column offsets (stencils) -> slice
 // offsets, or the stencil layout when all rows draw on one short offset list;
 // other short rows of similar length -> sliced rows (padding <= 10%,
 // addressable with the index type); other short-row matrices -> LDS-staged
-// row blocks; long rows -> LANES lanes per row with LANES the largest power of
+// row blocks; long rows -> LANES lanes per row.  LANES is the largest power of
 // two within the mean row length (2..64): fewer idle lanes than the next one
-// costs trips (us at lanes 8 / 16 / 32 / 64: mean 9.4 entries 70 / 77 / 105 /
-// 202, 13.4 33 / 34 / 44 / 84, 19.3 147 / 121 / 140 / 210, 34.1 127 / 98 /
-// 89 / 112).
+// costs trips (us at lanes 8 / 16 / 32 / 64, columns near the diagonal, two rows
+// a group: mean 9.4 entries 70 / 77 / 105 / 202, 13.4 33 / 34 / 44 / 84, 19.3
+// 147 / 121 / 140 / 210, 34.1 127 / 98 / 89 / 112).  Where the trips are not
+// hidden it is the next power: few rows, so that the lanes do not fill the chip
+// (5000 rows of mean 45, 32 / 64 lanes: 3.6 / 3.1; 12000 of 9.4, 8 / 16: 3.0 / 2.7;
+// 25000 of 26, 16 / 32: 6.4 / 6.2 and CG's product 7.1 / 7.9), or x past a chiplet's
+// L2 with columns all over it (1 M rows of mean 20, 16 / 32: 233 / 211; of 28 335 /
+// 297; 400 k rows, whose x fits, 64 / 61 and CG's product 66 / 76).
+constexpr double kVectorFar = 3 << 19; // bytes of x from the diagonal
+
 void choose_plan(fsx_ctx * ctx, fsx_csr * A, const void * host_rowptr,
                  const void * host_colind) {
 	int64_t maxr = 0;
@@ -689,6 +712,13 @@ void choose_plan(fsx_ctx * ctx, fsx_csr * A, const void * host_rowptr,
 		}
 		maxr = std::max(maxr, b - a);
 	}
+	if (host_colind)
+		A->idx->col_dist =
+			A->it == FSX_I32
+				? column_distance<int32_t>(A->nrows, (const int32_t *)host_rowptr,
+				                           (const int32_t *)host_colind)
+				: column_distance<int64_t>(A->nrows, (const int64_t *)host_rowptr,
+				                           (const int64_t *)host_colind);
 	A->max_row = maxr;
 	A->avg_row = A->nrows ? (double)A->nnz / (double)A->nrows : 0.0;
 	const double per_row_budget = (double)kStreamCap / kStreamRows;
@@ -721,9 +751,11 @@ void choose_plan(fsx_ctx * ctx, fsx_csr * A, const void * host_rowptr,
 	}
 	else {
 		A->plan_kind = 1;
-		int l = 2;
+		int next = 2, l = 2;
+		while (next < 64 && next < A->avg_row) next <<= 1;
 		while (l < 64 && 2 * l <= A->avg_row) l <<= 1;
-		A->plan_lanes = l;
+		const bool far = A->idx->col_dist * (A->vt == FSX_F64 ? 8 : 4) > kVectorFar;
+		A->plan_lanes = far || A->nrows * next <= kVectorFull ? next : l;
 	}
 }
 

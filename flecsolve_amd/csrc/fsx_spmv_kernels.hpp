@@ -280,14 +280,33 @@ __global__ __launch_bounds__(kSpmvThreads) void spmv_stream_kernel(
 
 // Rows per group of lanes.  What bounds this mapping on ragged rows is the
 // rate of the gathers (3.8 cycles each and CU at 19 entries a row), then the
-// memory trips of a row: two rows at once, and lanes no more than the mean
-// row has entries (plan rule), 160 -> 120 us at 1 M rows of 3 .. 60 entries
-// (mean 19.3).  Four rows 127 us, eight 177 (registers); larger workgroups
-// walking contiguous rows, so that a CU's gathers stay in one window of x,
-// 126 us at best.
-constexpr int kVectorRows = 2;
+// memory trips of a row: two rows at once overlap those, but widen the part of
+// x that a CU's rows gather from, and leave half the waves.  So two rows where
+// the columns lie near the diagonal (median distance times element size within
+// 4 KB; a CU's L1 holds 32) and the rows fill the chip, else one.  One / two rows
+// (us; 400 k rows, y = A x FP64, CG's product FP64, y = A x FP32), columns within
+// +-w of the row:
+//   mean 20, 16 lanes: w 300 44.2 51.3 34.9 / 41.5 47.7 28.9; 1000 48.2 54.2
+//   36.6 / 48.6 52.5 31.3; 2000 53.6 58.4 38.2 / 57.9 59.4 36.7; 20000 62.8 66.1
+//   45.9 / 67.6 70.2 52.9
+//   mean 51, 32 lanes: w 300 88.7 103 74.4 / 82.4 95.0 60.4; 2000 108 117 80.4 /
+//   124 121 74.1; 20000 142 144 112 / 158 160 131
+// 1 M rows of mean 19.3, 16 lanes, normal of deviation 300 and 2% anywhere: 128 /
+// 121 (one row on 32 lanes 160).  5000 rows of mean 253, 64 lanes: 8.4 9.0 7.7 /
+// 12.3 12.9 8.6; 12000 of 9.4, 8 lanes: 3.0 3.7 2.8 / 3.9 4.6 3.4.  Four rows are slower
+// than two (registers), as are larger workgroups walking contiguous rows.
+constexpr double kVectorNear = 4096;           // bytes of x from the diagonal
+constexpr int64_t kVectorFull = 3 << 17;       // lanes: three quarters of the chip's
 
-template<int LANES, class Epi, class ACC, class V, class I, class G>
+inline int vector_rows_of(const fsx_csr * A) {
+	const double d = A->idx->col_dist * (A->vt == FSX_F64 ? 8 : 4);
+	return A->plan_lanes >= 8 && d >= 0 && d <= kVectorNear &&
+	               A->nrows * A->plan_lanes > kVectorFull
+	           ? 2
+	           : 1;
+}
+
+template<int LANES, int NR, class Epi, class ACC, class V, class I, class G>
 __global__ __launch_bounds__(kSpmvThreads) void spmv_vector_kernel(
 	int64_t nrows, const I * __restrict__ rowptr, const I * __restrict__ colind,
 	const V * __restrict__ vals, G x, Epi epi) {
@@ -295,15 +314,15 @@ __global__ __launch_bounds__(kSpmvThreads) void spmv_vector_kernel(
 	x.init();
 	constexpr int RPB = kSpmvThreads / LANES;
 	const unsigned blk = blockIdx.x;
-	const int64_t row0 = (int64_t)blk * RPB * kVectorRows + threadIdx.x / LANES;
-	ACC sum[kVectorRows];
-	vector_rows<LANES, kVectorRows, ACC>(row0, RPB, nrows, rowptr, colind, vals, x, sum);
+	const int64_t row0 = (int64_t)blk * RPB * NR + threadIdx.x / LANES;
+	ACC sum[NR];
+	vector_rows<LANES, NR, ACC>(row0, RPB, nrows, rowptr, colind, vals, x, sum);
 	double d[Epi::NV];
 #pragma unroll
 	for (int i = 0; i < Epi::NV; ++i) d[i] = 0.0;
 	if ((threadIdx.x & (LANES - 1)) == 0) {
 #pragma unroll
-		for (int i = 0; i < kVectorRows; ++i) {
+		for (int i = 0; i < NR; ++i) {
 			const int64_t row = row0 + (int64_t)i * RPB;
 			if (row < nrows) epi.row(row, sum[i], d, [&] { return x(row); });
 		}
@@ -790,13 +809,23 @@ void spmv_launch_gather(hipStream_t st, const fsx_csr * A, const G & x,
 		                   dim3(kSpmvThreads), 0, st, A->nrows, rp, ci, vv, x, epi);
 	}
 	else {
-		auto go = [&](auto lanes_c) {
-			constexpr int L = decltype(lanes_c)::value;
-			constexpr int RPB = kSpmvThreads / L * kVectorRows;
+		auto launch = [&](auto lanes_c, auto nr_c) {
+			constexpr int L = decltype(lanes_c)::value, NR = decltype(nr_c)::value;
+			constexpr int RPB = kSpmvThreads / L * NR;
 			unsigned g = (unsigned)((A->nrows + RPB - 1) / RPB);
-			hipLaunchKernelGGL((spmv_vector_kernel<L, Epi, ACC, V, I, G>), dim3(g),
+			hipLaunchKernelGGL((spmv_vector_kernel<L, NR, Epi, ACC, V, I, G>), dim3(g),
 			                   dim3(kSpmvThreads), 0, st, A->nrows, rp, ci, vv, x,
 			                   epi);
+		};
+		const bool two = vector_rows_of(A) == 2;
+		auto go = [&](auto lanes_c) {
+			if constexpr (decltype(lanes_c)::value >= 8) {
+				if (two) {
+					launch(lanes_c, std::integral_constant<int, 2>{});
+					return;
+				}
+			}
+			launch(lanes_c, std::integral_constant<int, 1>{});
 		};
 		switch (A->plan_lanes) {
 		case 2: go(std::integral_constant<int, 2>{}); break;
@@ -827,7 +856,7 @@ inline unsigned spmv_blocks(const fsx_csr * A) {
 	if (A->plan_kind == 2) return sliced_blocks(A->nrows);
 	if (A->plan_kind == 0)
 		return (unsigned)((A->nrows + kStreamRows - 1) / kStreamRows);
-	const int rpb = kSpmvThreads / A->plan_lanes * kVectorRows;
+	const int rpb = kSpmvThreads / A->plan_lanes * vector_rows_of(A);
 	return (unsigned)((A->nrows + rpb - 1) / rpb);
 }
 

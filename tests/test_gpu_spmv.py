@@ -617,3 +617,44 @@ def test_stencil_matrix_holds_one_product_layout(ctx, kind):
     if kind != "f32":
         B = fsx.Batch(ctx.csr(rp, ci, v), np.array([0, n], np.int64))
         assert B.config()[1] == 2
+
+
+def banded_ragged(n, mean, width, seed):
+    """About `mean` entries a row (a tenth of the rows twice that, some none),
+    columns within `width` of the row (0: anywhere)."""
+    rng = np.random.default_rng(seed)
+    ln = rng.poisson(mean, n)
+    ln = np.where(rng.random(n) < 0.1, 2 * ln, ln)
+    ln[rng.random(n) < 0.01] = 0
+    r = np.repeat(np.arange(n), ln)
+    c = np.clip(r + rng.integers(-width, width + 1, r.size), 0, n - 1) if width else \
+        rng.integers(0, n, r.size)
+    S = sp.csr_matrix((rng.uniform(-1, 1, r.size), (r, c)), (n, n))
+    S.sum_duplicates()
+    S.sort_indices()
+    return S
+
+
+@pytest.mark.parametrize("n,mean,width,lanes", [
+    (5000, 45, 2000, 64),     # few rows: the next power of two
+    (12000, 12, 2000, 16),
+    (40000, 12, 300, 8),      # many: the one within the mean; two rows a group
+    (33001, 22, 200, 16),
+    (40000, 40, 3000, 32),    # columns too far for two rows
+    (900_000, 10, 0, 16),     # x past an L2, columns all over it
+])
+def test_lanes_rule(ctx, n, mean, width, lanes):
+    """The lanes-per-row rule on both sides of its lines, the products (FP64
+    and FP32, SpMV+dot) against scipy within rounding of a tree sum."""
+    S = banded_ragged(n, mean, width, 5)
+    A = ctx.csr(S.indptr.astype(np.int32), S.indices.astype(np.int32), S.data)
+    assert A.plan() == (1, lanes)
+    x = np.random.default_rng(6).standard_normal(n)
+    ref, mag = S @ x, abs(S) @ np.abs(x)
+    y = ctx.zeros(n)
+    pw = fsx.spmv_dot(A, ctx.vec(x), y)
+    assert (np.abs(y.get() - ref) <= 1e-13 * mag).all()
+    assert abs(pw - ref @ x) <= 1e-12 * (mag * np.abs(x)).sum()
+    A32, y32 = A.convert(fsx.F32), ctx.zeros(n, fsx.F32)
+    A32.spmv(ctx.vec(x.astype(np.float32)), y32)
+    assert (np.abs(y32.get() - ref) <= 2e-5 * mag).all()  # 100 sums in FP32
