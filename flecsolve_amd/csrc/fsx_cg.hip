@@ -2596,6 +2596,16 @@ static char * noalloc_base(int device) {
 using namespace fsx;
 
 namespace fsx {
+// The residual history of a solve, kept for fsx_cg_history.  On the context's
+// stream: a copy on the null stream would break into another thread's capture.
+static void keep_history(fsx_ctx * ctx, int cnt) {
+	ctx->last_cg_hist.assign(cnt, 0.0);
+	if (cnt == 0) return;
+	FSX_HIP(hipMemcpyAsync(ctx->last_cg_hist.data(), ctx->cg_cache->histbuf->p,
+	                       sizeof(double) * cnt, hipMemcpyDeviceToHost, ctx->stream));
+	FSX_HIP(hipStreamSynchronize(ctx->stream));
+}
+
 // Average duration of `reps` back-to-back launches of the fused CG's K1 on A
 // (NV = 1: partials of w.p; NV = 2: of w.p and w.w, the single-reduction
 // inner CG), on the context stream.
@@ -2673,10 +2683,7 @@ int fsx_cg_solve(fsx_ctx * ctx, const fsx_csr * A, const fsx_vec * dinv,
 		int cnt = 0;
 		if (b->dt == FSX_F64) cg_solve_impl<double>(ctx, A, dinv, b, x, *s, info, wk, &cnt);
 		else cg_solve_impl<float>(ctx, A, dinv, b, x, *s, info, wk, &cnt);
-		ctx->last_cg_hist.assign(cnt, 0.0);
-		if (cnt > 0)
-			FSX_HIP(hipMemcpy(ctx->last_cg_hist.data(), ctx->cg_cache->histbuf->p,
-			                  sizeof(double) * cnt, hipMemcpyDeviceToHost));
+		keep_history(ctx, cnt);
 	});
 }
 
@@ -2700,10 +2707,7 @@ int fsx_cg_solve_diag(fsx_ctx * ctx, const fsx_csr * A, const fsx_vec * dinv,
 		if (b->dt == FSX_F64)
 			cg_solve_impl<double>(ctx, A, dinv, b, x, *s, info, wk, &cnt, diag, user);
 		else cg_solve_impl<float>(ctx, A, dinv, b, x, *s, info, wk, &cnt, diag, user);
-		ctx->last_cg_hist.assign(cnt, 0.0);
-		if (cnt > 0)
-			FSX_HIP(hipMemcpy(ctx->last_cg_hist.data(), ctx->cg_cache->histbuf->p,
-			                  sizeof(double) * cnt, hipMemcpyDeviceToHost));
+		keep_history(ctx, cnt);
 	});
 }
 

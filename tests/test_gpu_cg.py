@@ -724,3 +724,40 @@ def test_resident_not_finite_as_launched(ctx, monkeypatch, where):
             np.testing.assert_array_equal(out[0][0], out[1][0])
             assert out[0][1:3] == out[1][1:3]
             np.testing.assert_array_equal(out[0][3], out[1][3])
+
+
+def test_solves_while_another_thread_captures(ctx, monkeypatch):
+    """One thread captures graphs over and over (a new matrix each solve, in the
+    launched loop) while another finishes small solves and reads their history:
+    nothing it does touches the other's capture."""
+    import threading
+    rp, ci, v = P.poisson2d(24)
+    b = P.uniform(24 * 24, 82)
+    s = fsx.Settings(maxiter=400, rtol=1e-8, use_zero_guess=True)
+    cap, sol = context_with(monkeypatch, FSX_CG_RESIDENT=0), fsx.Context(0)
+    done, err, out = threading.Event(), [], []
+
+    def capture():
+        try:
+            for _ in range(60):
+                A = cap.csr(rp, ci, v)
+                x = cap.zeros(b.size)
+                out.append((fsx.cg_solve(A, cap.vec(b), x, s).iters, x.get()))
+                A.destroy()
+        except Exception as e:
+            err.append(e)
+        done.set()
+
+    th = threading.Thread(target=capture)
+    A = sol.csr(rp, ci, v)
+    bd, x = sol.vec(b), sol.zeros(b.size)
+    th.start()
+    want = fsx.cg_solve(A, bd, x, s).iters, x.get()
+    while not done.is_set():
+        assert fsx.cg_solve(A, bd, x, s).iters == want[0]
+        assert len(fsx.cg_history(sol)) == want[0]
+    th.join()
+    assert not err, err
+    for it, xo in out:
+        assert it == want[0]
+        np.testing.assert_array_equal(xo, want[1])
