@@ -813,8 +813,7 @@ constexpr int kResMaxBlocks = 256;
 // stencil lists, at most kResRows rows for each thread of a workgroup per CU.
 static bool fits_resident(const fsx_csr * A, size_t n) {
 	const size_t blocks = (size_t)std::min(kResMaxBlocks, A->ctx->num_cus);
-	return n > 0 && on_stencil(A) && (A->idx->st_w == 5 || A->idx->st_w == 7) &&
-	       n <= blocks * kResThreads * kResRows;
+	return n > 0 && resident_candidate(A) && n <= blocks * kResThreads * kResRows;
 }
 
 // Work of an allocating CG solve: pooled context vectors in slots slot0 ..
@@ -1042,8 +1041,10 @@ constexpr uint64_t kResWaitTicks = 100000000;  // of the 100 MHz counter: 1 s
 constexpr uint64_t kResSentinel = 0xFFF8DEADBEEF5A5Aull;
 enum res_verdict { RES_RUNNING = 0, RES_GAVE_UP, RES_FINISHED };
 static_assert(kResMaxBlocks * kResRows * 2 <= kXchSlots, "exchange slots");
-static_assert((int64_t)kResMaxBlocks * kResRows * kResThreads <= kStencilWideF32,
-              "the resident FP32 products' rows per lane");
+static_assert((int64_t)kResMaxBlocks * kResRows * kResThreads == kResidentMaxRows, "");
+static_assert(kResidentMaxRows <= kStencilWideF32 && kResidentMaxRows <= kSdiaWideRows,
+              "the launched products the resident one follows: one FP32 row per lane, "
+              "256 rows a block on slice offsets");
 
 struct res_args {
 	int64_t n;
@@ -1427,7 +1428,7 @@ static void enqueue_resident(fsx_ctx * ctx, const cg_bufs & B, cg_state * st, do
 	hipLaunchKernelGGL(res_reset_kernel, dim3((kXchDoubles + 255) / 256), dim3(256), 0,
 	                   ctx->stream, ctx->ws.xch, (int)(give_up ? RES_GAVE_UP : RES_RUNNING));
 	if constexpr (SR) launch_resident<T, true, false>(ctx, a);
-	else if (stencil_run(FSX_F64, a.n) == 2) {
+	else if (on_stencil(A) && stencil_run(FSX_F64, a.n) == 2) {
 		if (B.dinv) launch_resident<T, false, true, true>(ctx, a);
 		else launch_resident<T, false, false, true>(ctx, a);
 	}

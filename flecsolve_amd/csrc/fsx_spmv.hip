@@ -638,6 +638,17 @@ void ensure_dg_fresh(fsx_ctx * ctx, const fsx_csr * A) {
 	M->dg_stale = false;
 }
 
+// After the plan, the form or the values of A (`changed`) may have changed: the
+// slice-offset values up to date where the products read them (or somebody does
+// who made them), stale elsewhere; no stencil values that nothing reads.
+static void settle_layouts(fsx_ctx * ctx, fsx_csr * A, bool changed) {
+	const bool have = has_sdia(A);
+	if (have && changed) A->dg_stale = true;
+	if (have && !on_stencil(A) && (A->plan_kind == 3 || A->dg_vals)) ensure_dg_fresh(ctx, A);
+	if (A->st_vals && stencil_planned(A) && !on_stencil(A) && !resident_candidate(A))
+		A->st_vals.reset();
+}
+
 void refresh_sliced_values(fsx_ctx * ctx, fsx_csr * A) {
 	++A->vals_version;
 	if (A->st_vals && A->idx->st_state > 0 && !stencil_fill(ctx, A)) {
@@ -646,14 +657,7 @@ void refresh_sliced_values(fsx_ctx * ctx, fsx_csr * A) {
 		if (A->plan_kind == 4) A->plan_kind = 3;
 		if (A->plan_kind == 3 && A->plan_lanes == 0) stencil_build(ctx, A, true);
 	}
-	if (A->idx->dg_ptr && A->dg_vals) {
-		// rebuilt when next read where the products run on the stencil layout
-		if (on_stencil(A)) A->dg_stale = true;
-		else {
-			sdia_fill(ctx, A);
-			A->dg_stale = false;
-		}
-	}
+	settle_layouts(ctx, A, true);
 	if (!(A->idx->sl_ptr && A->sl_vals)) return;
 	if (A->it == FSX_I32) {
 		if (A->vt == FSX_F64) refresh_sliced_t<int32_t, double>(ctx, A);
@@ -731,8 +735,8 @@ void choose_plan(fsx_ctx * ctx, fsx_csr * A, const void * host_rowptr,
 			const bool st = ensure_stencil_any(ctx, A, host_rowptr, host_colind);
 			A->plan_kind = st && A->vt == FSX_F64 && !A->st_full ? 4 : 3;
 			A->plan_lanes = 0;
-			if (st) A->dg_stale = true;
-			else ensure_sdia(ctx, A, host_rowptr, host_colind, true);
+			A->dg_stale = true;
+			settle_layouts(ctx, A, false);
 			return;
 		}
 		const int64_t padded =
@@ -1148,6 +1152,7 @@ int fsx_csr_convert(fsx_ctx * ctx, const fsx_csr * A, fsx_dtype vt,
 		         !A->st_full)
 			B->plan_kind = 4;
 		if (!on_stencil(B.get())) ensure_dg_fresh(ctx, B.get());
+		settle_layouts(ctx, B.get(), false);
 		FSX_HIP(hipStreamSynchronize(ctx->stream));
 		ctx_retain(ctx);
 		*out = B.release();
@@ -1224,7 +1229,7 @@ int fsx_csr_set_plan(fsx_csr * A, int kind, int lanes) {
 		}
 		A->plan_kind = kind;
 		A->plan_lanes = kind == 1 ? lanes : kind == 3 && lanes != 0 ? 1 : 0;
-		if (kind == 3 && !on_stencil(A)) ensure_dg_fresh(A->ctx, A);
+		settle_layouts(A->ctx, A, false);
 	});
 }
 
@@ -1462,7 +1467,7 @@ int fsx_csr_shift_scale(fsx_ctx * ctx, const fsx_csr * F, double alpha, double b
 			A->st_vals.reset();
 			if (A->plan_kind == 4) A->plan_kind = 3;
 			if (A->plan_kind == 3 && A->plan_lanes == 0) stencil_build(ctx, A, true);
-			ensure_dg_fresh(ctx, A);
+			settle_layouts(ctx, A, false);
 		}
 		if (ix.sl_ptr && A->sl_vals) {
 			if (A->it == FSX_I32) refresh_sliced_t<int32_t, double>(ctx, A);

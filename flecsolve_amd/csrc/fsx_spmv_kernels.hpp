@@ -683,13 +683,48 @@ inline unsigned stencil_blocks(fsx_dtype vt, int64_t nrows, bool reduces) {
 	return (unsigned)(reduces && vt == FSX_F32 ? std::min<int64_t>(g, kStencilMaxBlocksF32) : g);
 }
 
-// Products on the stencil layout: plan 4 (symmetric, FP64 by default), and plan
-// 3 without lanes on the FP32 and nonsymmetric matrices that have it (plan 3 of
-// a symmetric FP64 one, and with lanes, is slice offsets).  A function of the
-// plan alone, so that setting a matrix's reported plan gives its kernel back.
+// Matrices planned on the stencil layout: plan 4 (symmetric, FP64 by default),
+// and plan 3 without lanes on the FP32 and nonsymmetric ones that have it (plan 3
+// of a symmetric FP64 one, and with lanes, is slice offsets).
+inline bool stencil_planned(const fsx_csr * A) {
+	return A->plan_kind == 4 || (A->plan_kind == 3 && A->plan_lanes == 0 &&
+	                             (A->vt == FSX_F32 || A->st_full));
+}
+
+// Five or seven offsets, -1, 0, +1 in the middle: the kernel's own instances.
+inline bool stencil_near(const csr_index & X) {
+	const int c = X.st_w / 2;
+	return (X.st_w == 5 || X.st_w == 7) && X.st_off[c - 1] == -1 && X.st_off[c] == 0 &&
+	       X.st_off[c + 1] == 1;
+}
+
+// Whether products of a matrix planned on it run there.  Plan 4 and the lists
+// with instances of their own always do.  The general lists' kernel tests each
+// offset against the list's length between its loads; on plan 3 it loses to slice
+// offsets in the full form of six offsets and more, and below a million rows in
+// FP32.  Iterations on it / on slice offsets (us): BiCGSTAB, FP64 full form, seven
+// offsets without +-1, 100 k rows 33.5 / 32.7, 4 M 216 / 207; eight 33.9 / 32.8,
+// 228 / 213; four 4 M 182 / 193; three 167 / 191; FP32 CG with residual
+// replacement, five offsets, 700 k rows 22.8 / 22.2, 1.2 M 26.1 / 28.7, 8 M 91 / 95;
+// seven 700 k 23.2 / 22.4, 8 M 99 / 101; three 100 k 14.8 / 14.4, 1.2 M 20.9 / 27.2.
+inline bool stencil_wins(const fsx_csr * A) {
+	const csr_index & X = *A->idx;
+	if (A->plan_kind == 4 || stencil_near(X)) return true;
+	if (A->st_full && X.st_w >= 6) return false;
+	return A->vt == FSX_F64 || A->nrows >= kStencilWideF32;
+}
+
+// Products on the stencil layout.  A function of the plan, the type, the form and
+// the size, so that setting a matrix's reported plan gives its kernel back.
 inline bool on_stencil(const fsx_csr * A) {
-	return A->st_vals && (A->plan_kind == 4 || (A->plan_kind == 3 && A->plan_lanes == 0 &&
-	                                            (A->vt == FSX_F32 || A->st_full)));
+	return A->st_vals && stencil_planned(A) && stencil_wins(A);
+}
+
+// Whether CG on A may run in one resident launch, which reads the stencil values
+// (also where the products do not): five or seven offsets, few rows.
+inline bool resident_candidate(const fsx_csr * A) {
+	return A->st_vals && stencil_planned(A) && (A->idx->st_w == 5 || A->idx->st_w == 7) &&
+	       A->nrows <= kResidentMaxRows;
 }
 
 template<class Epi, class ACC, class V, class G>
@@ -699,9 +734,7 @@ void stencil_launch(hipStream_t st, const fsx_csr * A, const G & x, const Epi & 
 	// 32-bit offsets while a row's byte offset in a vector (at most 8-byte
 	// elements) fits
 	const bool o32 = (uint64_t)A->nrows * 8 < ((uint64_t)1 << 32);
-	const int c = sd.w / 2;
-	const bool tri = sd.w % 2 && sd.w >= 3 && sd.off[c - 1] == -1 && sd.off[c] == 0 &&
-	                 sd.off[c + 1] == 1;
+	const bool tri = stencil_near(X);
 	const unsigned g = stencil_blocks(A->vt, A->nrows, Epi::reduces);
 	auto launch = [&](auto r_c, auto w_c, auto sym_c, auto o32_c) {
 		constexpr int R = decltype(r_c)::value, W = decltype(w_c)::value;

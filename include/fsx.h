@@ -190,8 +190,8 @@ int fsx_csr_info(const fsx_csr * A, int64_t * nrows, int64_t * ncols,
  * entries below the diagonal are read from their mirrors above it, so it
  * serves only structurally and bitwise symmetric values; chosen for such FP64
  * matrices; their slice-offset values are built when something reads them).  FP32 and nonsymmetric matrices
- * with such an offset list report 3 and run on the stencil layout as well
- * (all offsets stored where not symmetric); setting 3 with lanes = 0 gives them
+ * with such an offset list report 3 and run on the stencil layout as well where
+ * it is the faster (all offsets stored where not symmetric); setting 3 with lanes = 0 gives them
  * that, with another `lanes` slice offsets (reported as 3, 1).  A symmetric
  * FP64 matrix set to 3 runs on slice offsets either way.  A change of values that breaks the
  * symmetry moves a plan-4 matrix to plan 3; fsx_csr_set_plan(A, 4, 0)

@@ -611,6 +611,44 @@ def test_resident_bits_do_not_depend_on_the_path(ctx, monkeypatch, dims):
             assert got[1:] == want[1:]
 
 
+@pytest.mark.parametrize("symmetric", [True, False])
+@pytest.mark.parametrize("n", [20_000, 150_001])
+def test_resident_bits_on_general_lists(ctx, monkeypatch, n, symmetric):
+    """Seven offsets without -1 and +1: the launched FP64 products run on the
+    stencil layout (two rows a lane from 131072) or, not symmetric, on slice
+    offsets, the FP32 ones on slice offsets; the resident solves keep their
+    bits."""
+    m = int(n ** 0.5)
+    rng = np.random.default_rng(n)
+    S = sp.diags([4.5 + rng.random(n)], [0])
+    for o in (2, 7, m):
+        u = -rng.uniform(0.2, 0.8, n - o)
+        S = S + sp.diags([u, u if symmetric else u * rng.uniform(0.9, 1.1, n - o)], [o, -o])
+    S = sp.csr_matrix(S)
+    S.sort_indices()
+    b, x0 = P.uniform(n, 72), P.uniform(n, 73)
+
+    def solve(c):
+        A = c.csr(S.indptr.astype(np.int32), S.indices.astype(np.int32), S.data)
+        assert A.plan() == ((4, 0) if symmetric else (3, 0))
+        x, before = c.vec(x0), c.counters()[1]
+        i = fsx.cg_solve(A, c.vec(b), x, fsx.Settings(maxiter=40, rtol=1e-15), dinv=A.diag_inv())
+        out = [x.get(), i.as_dict(), list(fsx.cg_history(c)), c.counters()[1] - before]
+        A32 = A.convert(fsx.F32)
+        A32.set_values_sym_scaled(A)
+        x = c.vec(x0)
+        r = fsx.ir_cg_rr_solve(A, A32, c.vec(b), x, 1e-10, fsx.Settings(maxiter=20, rtol=1e-2),
+                               max_segments=3)
+        return out + [x.get(), r.inner_iters_total]
+
+    want, got = solve(context_with(monkeypatch, FSX_CG_RESIDENT=0)), solve(ctx)
+    assert got[3] < 30 < want[3]
+    np.testing.assert_array_equal(got[0], want[0])
+    assert got[1:3] == want[1:3]
+    np.testing.assert_array_equal(got[4], want[4])
+    assert got[5] == want[5]
+
+
 def test_resident_solve_inside_a_diagnostic(ctx):
     """A diagnostic may solve on another context: nothing of the resident solve
     it was called from is held meanwhile, so the inner one is resident too."""

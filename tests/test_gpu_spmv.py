@@ -658,3 +658,60 @@ def test_lanes_rule(ctx, n, mean, width, lanes):
     A32, y32 = A.convert(fsx.F32), ctx.zeros(n, fsx.F32)
     A32.spmv(ctx.vec(x.astype(np.float32)), y32)
     assert (np.abs(y32.get() - ref) <= 2e-5 * mag).all()  # 100 sums in FP32
+
+
+@pytest.mark.parametrize("n,offs,symmetric,kinds", [
+    (60_000, (-1, 0, 1), True, "ts"),             # a general list of three: FP32 on slices
+    (60_000, (-1, 0, 1), False, "ts"),
+    (300_000, (-540, -5, 0, 5, 540), True, "ts"),
+    (300_000, (-540, -7, -2, 0, 2, 7, 540), False, "ss"),
+    (300_000, (-540, -2, 0, 3), False, "ts"),
+    (1_100_000, (-1000, -5, 0, 5, 1000), True, "tt"),
+    (1_100_000, (-1000, -7, -2, 0, 2, 7, 1000), False, "ss"),
+    (70_000, (-260, -1, 0, 1, 260), False, "tt"),  # the kernel's own instance
+])
+def test_general_lists_run_where_faster(ctx, n, offs, symmetric, kinds):
+    """Which layout serves (t: stencil, s: slice offsets; FP64, FP32), told by
+    the bytes of the slice-offset plan, with the serial loop's bits before and
+    after a change of values and across plans."""
+    rng = np.random.default_rng(n)
+    up = {o: rng.uniform(-1, 1, n - o) for o in offs if o > 0}
+    diags = []
+    for o in offs:
+        k = n - abs(o)
+        diags.append(rng.uniform(4, 5, n) if o == 0 else
+                     up[-o] if symmetric and o < 0 else up.get(o, rng.uniform(-1, 1, k)))
+    S = sp.csr_matrix(sp.diags(diags, offs))
+    S.sort_indices()
+    rp, ci = S.indptr.astype(np.int32), S.indices.astype(np.int32)
+    x = rng.standard_normal(n)
+    A = ctx.csr(rp, ci, S.data)
+    xd, y = ctx.vec(x), ctx.zeros(n)
+    x32, y32 = ctx.vec(x.astype(np.float32)), ctx.zeros(n, fsx.F32)
+    A32 = A.convert(fsx.F32)
+    S32 = A.convert(fsx.F32)
+    S32.set_plan(3, 1)
+    T = A.convert(fsx.F64)
+    T.set_plan(3, 1)
+    for M, sl, k in ((A, T, kinds[0]), (A32, S32, kinds[1])):
+        assert (M.layout_bytes(8) == sl.layout_bytes(8)) == (k == "s")
+    for v in (S.data, S.data * 1.5, np.where(ci > np.repeat(np.arange(n), np.diff(rp)),
+                                             S.data * 0.75, S.data)):
+        A.set_values(v)
+        A32.set_values_from(A)
+        S32.set_values_from(A)
+        ref = O.Csr(rp, ci, v).spmv(x)
+        A.spmv(xd, y)
+        np.testing.assert_array_equal(y.get(), ref)
+        A32.spmv(x32, y32)
+        got = y32.get()
+        S32.spmv(x32, y32)
+        np.testing.assert_array_equal(y32.get(), got)
+    p = A.plan()
+    for other in ((0, 0), (3, 1), (3, 0)):
+        A.set_plan(*other)
+        A.spmv(xd, y)
+        np.testing.assert_array_equal(y.get(), ref)
+        A.set_plan(*p)
+        A.spmv(xd, y)
+        np.testing.assert_array_equal(y.get(), ref)
