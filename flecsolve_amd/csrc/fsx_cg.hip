@@ -561,6 +561,8 @@ struct cg_graph_cache {
 	fsx::dbuf * statebuf = nullptr;
 	fsx::dbuf * histbuf = nullptr;
 	size_t hist_cap = 0;
+	double * hist_pin = nullptr; // pinned, kHistPinned entries
+	static constexpr int kHistPinned = 4096;
 	void clear_graphs() {
 		for (auto & kv : mv) {
 			if (kv.second.ge) (void)hipGraphExecDestroy(kv.second.ge);
@@ -573,6 +575,7 @@ struct cg_graph_cache {
 		for (auto & kv : pool) fsx_vec_release(kv.second);
 		delete statebuf;
 		delete histbuf;
+		if (hist_pin) (void)hipHostFree(hist_pin);
 	}
 };
 
@@ -786,6 +789,8 @@ static double * history_buffer(fsx_ctx * ctx, int maxiter) {
 		c.histbuf = nullptr;
 		size_t cap = std::max<size_t>(need, 4096);
 		c.histbuf = new dbuf(cap * sizeof(double));
+		if (!c.hist_pin)
+			FSX_HIP(hipHostMalloc((void **)&c.hist_pin, c.kHistPinned * sizeof(double)));
 		c.hist_cap = cap;
 	}
 	return (double *)c.histbuf->p;
@@ -2602,9 +2607,12 @@ namespace fsx {
 static void keep_history(fsx_ctx * ctx, int cnt) {
 	ctx->last_cg_hist.assign(cnt, 0.0);
 	if (cnt == 0) return;
-	FSX_HIP(hipMemcpyAsync(ctx->last_cg_hist.data(), ctx->cg_cache->histbuf->p,
-	                       sizeof(double) * cnt, hipMemcpyDeviceToHost, ctx->stream));
+	auto & c = *ctx->cg_cache;
+	double * to = cnt <= c.kHistPinned ? c.hist_pin : ctx->last_cg_hist.data();
+	FSX_HIP(hipMemcpyAsync(to, c.histbuf->p, sizeof(double) * cnt, hipMemcpyDeviceToHost,
+	                       ctx->stream));
 	FSX_HIP(hipStreamSynchronize(ctx->stream));
+	if (to == c.hist_pin) std::memcpy(ctx->last_cg_hist.data(), to, sizeof(double) * cnt);
 }
 
 // Average duration of `reps` back-to-back launches of the fused CG's K1 on A

@@ -669,15 +669,16 @@ void refresh_sliced_values(fsx_ctx * ctx, fsx_csr * A) {
 	}
 }
 
-// Median |column - row| over at most 4096 rows, evenly spread, and 64 entries of
+// Median |column - row| over at most 256 rows, evenly spread, and 16 entries of
 // each (the median: a few couplings to anywhere do not move what the others hit).
 template<class I>
 static double column_distance(int64_t nrows, const I * rp, const I * ci) {
-	const int64_t rows = std::min<int64_t>(nrows, 4096);
+	const int64_t rows = std::min<int64_t>(nrows, 256);
 	std::vector<int64_t> d;
+	d.reserve((size_t)rows * 16);
 	for (int64_t k = 0; k < rows; ++k) {
 		const int64_t r = k * (nrows / rows) + k * (nrows % rows) / rows;
-		const int64_t lo = rp[r], len = (int64_t)rp[r + 1] - lo, m = std::min<int64_t>(len, 64);
+		const int64_t lo = rp[r], len = (int64_t)rp[r + 1] - lo, m = std::min<int64_t>(len, 16);
 		for (int64_t e = 0; e < m; ++e) d.push_back(std::abs((int64_t)ci[lo + e * len / m] - r));
 	}
 	if (d.empty()) return 0;
