@@ -1044,7 +1044,7 @@ static void run_cg_loop_pipelined(fsx_ctx * ctx, const cg_bufs & B, cg_state * s
 // there.
 constexpr uint64_t kResWaitTicks = 100000000;  // of the 100 MHz counter: 1 s
 constexpr uint64_t kResSentinel = 0xFFF8DEADBEEF5A5Aull;
-enum res_verdict { RES_RUNNING = 0, RES_GAVE_UP, RES_FINISHED };
+enum res_outcome { RES_RUNNING = 0, RES_GAVE_UP, RES_FINISHED };
 static_assert(kResMaxBlocks * kResRows * 2 <= kXchSlots, "exchange slots");
 static_assert((int64_t)kResMaxBlocks * kResRows * kResThreads == kResidentMaxRows, "");
 static_assert(kResidentMaxRows <= kStencilWideF32 && kResidentMaxRows <= kSdiaWideRows,
@@ -1075,15 +1075,15 @@ __device__ __forceinline__ void dev_store(T * p, T v) {
 	__hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// All slots the sentinel; the verdict open (or already that it gave up).
-__global__ void res_reset_kernel(double * xch, int verdict) {
+// All slots the sentinel; the outcome open (or already that it gave up).
+__global__ void res_reset_kernel(double * xch, int outcome) {
 	const int i = blockIdx.x * blockDim.x + threadIdx.x;
 	if (i < 3 * kXchSlots) ((uint64_t *)xch)[i] = kResSentinel;
 	else if (i < kXchDoubles) ((uint64_t *)xch)[i] = 0;
-	if (i == 3 * kXchSlots) *(int *)(xch + i) = verdict;
+	if (i == 3 * kXchSlots) *(int *)(xch + i) = outcome;
 }
 
-// The launch's verdict, `mine` if none was reached before.
+// The launch's outcome, `mine` if none was reached before.
 __device__ __forceinline__ int res_claim(double * xch, int mine) {
 	int * word = (int *)(xch + 3 * kXchSlots);
 	int was = RES_RUNNING;
@@ -1152,10 +1152,10 @@ __device__ __forceinline__ bool res_exchange(const double (&d)[GRP][NV], int cou
 		if ((spin & 255) == 255) {
 			const uint64_t now = wall_clock64();
 			if (!t0) t0 = now;
-			int verdict = dev_load((const int *)(xch + 3 * kXchSlots));
-			if (verdict == RES_RUNNING && now - t0 > kResWaitTicks)
-				verdict = res_claim(xch, RES_GAVE_UP);
-			if (__any(verdict == RES_GAVE_UP)) {
+			int outcome = dev_load((const int *)(xch + 3 * kXchSlots));
+			if (outcome == RES_RUNNING && now - t0 > kResWaitTicks)
+				outcome = res_claim(xch, RES_GAVE_UP);
+			if (__any(outcome == RES_GAVE_UP)) {
 				live = false;
 				break;
 			}
@@ -1369,10 +1369,10 @@ cg_resident_kernel(res_args a) {
 		first = false;
 	}
 	if (!ok) return;
-	__shared__ int verdict;
-	if (threadIdx.x == 0) verdict = res_claim(a.xch, RES_FINISHED);
+	__shared__ int outcome;
+	if (threadIdx.x == 0) outcome = res_claim(a.xch, RES_FINISHED);
 	__syncthreads();
-	if (verdict != RES_FINISHED) return;
+	if (outcome != RES_FINISHED) return;
 #pragma unroll
 	for (int j = 0; j < RPT; ++j) {
 		const int64_t row = base + j * kResThreads;
@@ -1451,13 +1451,13 @@ static std::mutex g_resident_mu[kResMaxDevices];
 
 // Reads the state after a resident launch; false when the launch gave up.
 static bool read_resident(fsx_ctx * ctx, const cg_state * st, cg_state * pinned) {
-	int * verdict = (int *)(ctx->host_scalars + kScalarSlots - 1);
+	int * outcome = (int *)(ctx->host_scalars + kScalarSlots - 1);
 	FSX_HIP(hipMemcpyAsync(pinned, st, sizeof(cg_state), hipMemcpyDeviceToHost, ctx->stream));
-	FSX_HIP(hipMemcpyAsync(verdict, ctx->ws.xch + 3 * kXchSlots, sizeof(int),
+	FSX_HIP(hipMemcpyAsync(outcome, ctx->ws.xch + 3 * kXchSlots, sizeof(int),
 	                       hipMemcpyDeviceToHost, ctx->stream));
 	FSX_HIP(hipStreamSynchronize(ctx->stream));
 	ctx->host_syncs++;
-	return *verdict != RES_GAVE_UP;
+	return *outcome != RES_GAVE_UP;
 }
 
 // Iteration loop with a user diagnostic (cg.hh:112-116): one iteration at a

@@ -100,7 +100,7 @@ struct dbuf {
 constexpr int kRedBlocks = 2048;   // maximum blocks of a reduction grid
 constexpr int kScalarSlots = 64;   // device scalar slots per context
 constexpr int kStencilMax = 8;     // offsets of the stencil layout
-// Exchange slots of the resident CG (three buffers and its verdict).
+// Exchange slots of the resident CG (three buffers and the outcome).
 constexpr int kXchSlots = 4096;
 // Most rows a resident CG holds: four for each of 256 threads on 256 CUs.
 constexpr int64_t kResidentMaxRows = 256 * 256 * 4;
