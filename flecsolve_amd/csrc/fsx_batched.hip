@@ -1212,9 +1212,15 @@ bool use_lockstep(const fsx_batch * B, bool rr, const fsx_csr * A32 = nullptr) {
 // sets or tunes one: few systems leave a CU to each, so all its waves serve
 // it (256 systems of 16^3: 1.8 ms at 1024 threads, 4.0 at 256); with many, a
 // CU holds several and small groups synchronise for less (2048 of 8^3: 1.0
-// ms at 256, 2.3 at 1024).
+// ms at 256, 2.3 at 1024).  The line in rows, residual replacement / FP64 CG /
+// refinement at 1024 against 256: 64 of 12^3 0.72 0.82 0.91 against 0.97 0.93
+// 1.22; 300 of 12^3, more than CUs, 1.36 1.68 1.72 against 1.35 1.52 1.61; 300 of
+// 14^3 2.06 2.74 2.63 against 2.67 2.74 3.42; 512 of 1600 rows with lanes per row
+// 3.1 against 3.6.
 int default_workgroup(const fsx_batch * B) {
-	if (B->max_rows >= 1536 && B->nsys <= 2 * (int64_t)B->ctx->num_cus) return 1024;
+	const int64_t cus = B->ctx->num_cus;
+	const int64_t from = B->mapping == 2 && B->nsys > cus ? 2048 : 1536;
+	if (B->max_rows >= from && B->nsys <= 2 * cus) return 1024;
 	return B->max_rows >= 4096 ? 512 : 256;
 }
 

@@ -437,3 +437,16 @@ def test_lockstep_not_finite_as_one_workgroup(ctx, case):
     np.testing.assert_array_equal(l[1][bad], o[1][bad])
     assert np.abs(l[1] - o[1]).max() <= 2
     same_or_close(xl.get(), xo.get(), 1e-8)
+
+
+@pytest.mark.parametrize("count,edge,wg", [(200, 12, 1024), (300, 12, 256), (300, 13, 1024),
+                                           (64, 11, 256), (520, 12, 256)])
+def test_default_workgroup(ctx, count, edge, wg):
+    """The size a batch starts with, on both sides of its lines (rows, more
+    systems than CUs, than twice that)."""
+    rp, ci, v = P.diffusion3d(edge, P.lognormal_field(edge, 1.0, 4.0, 980))
+    S = sp.block_diag([sp.csr_matrix((v, ci, rp))] * count, format="csr")
+    S.sort_indices()
+    A = ctx.csr(S.indptr.astype(np.int32), S.indices.astype(np.int32), S.data)
+    B = fsx.Batch(A, np.arange(count + 1, dtype=np.int64) * edge ** 3)
+    assert B.config() == (wg, 2, 1)
